@@ -1624,8 +1624,8 @@ int g4acc_sp_enable(g4acc_handle* h, int n_sp_freq, const int* r_sub, int accumu
   G4_TRY(h->alloc(&h->d_sp_perm, W2 * NM, "sp perm"));
   G4_TRY(h->alloc(&h->d_sp_off, W2 * (n_orb + 1), "sp off"));
   G4_TRY(h->alloc(&h->d_rsub, static_cast<size_t>(nc) * nc, "r_sub"));
-  G4_TRY(h->alloc(&h->d_sp_T, W2 * NM * n_w, "sp phases"));
-  G4_TRY(h->alloc(&h->d_sp_C, W2 * n_orb * n_orb * n_w, "sp orbital sums"));
+  G4_TRY(h->alloc(&h->d_sp_T, W2 * NM * n_w / 2, "sp phases"));
+  G4_TRY(h->alloc(&h->d_sp_C, W2 * n_orb * n_orb * n_w / 2, "sp orbital sums"));
   G4_TRY(h->alloc(&h->d_sp_acc, 2 * entries, "sp M_r_w"));
   if (accumulate_m_sqr)
     G4_TRY(h->alloc(&h->d_sp_acc_sqr, 2 * entries, "sp M_r_w_sqr"));

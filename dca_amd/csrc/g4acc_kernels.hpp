@@ -153,8 +153,8 @@ struct SpArgs {
   int n_slots, n_max, n_w;     // n_w = 2 * single-particle frequencies
   const int* perm;             // sort of the slots' vertices by caller orbital b + nb r
   const int* off;
-  double2* T;                  // [n_slots][n_max][n_w] phases
-  double2* C;                  // [n_slots][n_orb][n_orb][n_w] orbital-pair sums
+  double2* T;                  // [n_slots][n_max][n_w / 2] phases (upper half of the frequencies)
+  double2* C;                  // [n_slots][n_orb][n_orb][n_w / 2] orbital-pair sums
   const int* rsub;             // [Nc][Nc], rsub[a + Nc b] = index(r_b - r_a)
   double2* acc;
   double2* acc_sqr;

@@ -112,3 +112,29 @@ def test_gpu_sp_accumulator(nb, L, n_sp, precision):
     assert err < 1e-7
     a.resetAccumulation()
     assert np.all(a.get_sign_times_M_r_w() == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nb,L,n_sp,n_range", [(1, 2, 1, (1, 3)), (1, 2, 65, (60, 90)), (2, 2, 128, (30, 45)),
+                                               (1, 4, 63, (17, 80))])
+def test_gpu_sp_orbital_pair_edges(nb, L, n_sp, n_range):
+    """One wave per orbital pair: orbitals of no, one and more than sixteen vertices, frequency
+    counts around multiples of 64, batches that leave a wave of the reduction without a slot, and
+    exp(V) hand-over. FP64 sums of at most 90^2 terms: 1e-12, as the accumulator's other tests."""
+    from dca_amd import g4acc
+    wl = _wl(nb, L, n_range=n_range, seed=504)
+    g = wl.geometry
+    ms = wl.draw(5)
+    ms[1].n[0], ms[1].M[0] = 0, np.zeros((0, 0))
+    ms[1].tau[0], ms[1].site[0], ms[1].band[0] = np.zeros(0), np.zeros(0, np.int32), np.zeros(0, np.int32)
+    exact = so.m_r_w_exact(nb, g.nc, g.beta, n_sp, g.cluster.rsub, ms)
+    acc = g4acc.TpAccumulator(g, precision="fp64", max_walkers=5, max_vertices=wl.n_max)
+    acc.enable_sp(n_sp)
+    acc.resetAccumulation()
+    acc.accumulate_batch(ms)
+    assert bf.difference(exact, acc.get_sign_times_M_r_w())["l_inf"] < 1e-12
+    rs = synth.Stream(505)
+    pairs = [synth.walker_n_pair(m, rs) for m in ms]
+    acc.resetAccumulation()
+    acc.accumulate_batch_n([p[0] for p in pairs], [p[1] for p in pairs])
+    assert bf.difference(exact, acc.get_sign_times_M_r_w())["l_inf"] < 1e-12
