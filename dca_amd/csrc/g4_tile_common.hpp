@@ -40,8 +40,23 @@ template <typename Real>
 __device__ __forceinline__ bool tile_coords(const TiledArgs<Real>& a, int& w1, int& w2, int& z) {
   const int nw = a.g.nw;
   const int nz = a.g.nv * a.nqg;
-  if (a.sym) {
-    // Transpose symmetry: the nw (nw + 1) / 2 tiles w1 <= w2 in triangular order, w2 slowest.
+  if (a.sym >= SYM_CONJ) {
+    // The computed tiles in table order, exchange frequency and momentum group innermost and each
+    // XCD taking a contiguous range (batches), or outermost (one walker).
+    const unsigned total = static_cast<unsigned>(a.n_sym_tiles) * nz;
+    unsigned L = blockIdx.x;
+    if (a.n_xcd > 1)
+      L = (blockIdx.x % a.n_xcd) * (gridDim.x / a.n_xcd) + blockIdx.x / a.n_xcd;
+    if (L >= total)
+      return false;
+    const int packed = a.sym_tiles[a.n_xcd > 1 ? L / nz : L % a.n_sym_tiles];
+    z = a.n_xcd > 1 ? L % nz : L / a.n_sym_tiles;
+    w1 = packed & 0xffff;
+    w2 = packed >> 16;
+    return sym_tile_computed(nw, a.w_ex[z / a.nqg], w1, w2, a.need_y, a.need_z, a.sym);
+  }
+  if (a.sym == SYM_TRANSPOSE) {
+    // The nw (nw + 1) / 2 tiles w1 <= w2 in triangular order, w2 slowest.
     const unsigned L = blockIdx.x / nz;
     z = blockIdx.x % nz;
     int r = static_cast<int>((sqrt(8.0 * L + 1.0) - 1.0) * 0.5);
@@ -87,11 +102,37 @@ __device__ __forceinline__ bool tile_coords(const TiledArgs<Real>& a, int& w1, i
   return w1 < nw && w2 < nw;
 }
 
+// G[(ka, wa), (kb, wb)] of one slot (extended frequencies), read from the half of the frequency
+// pairs with wa + wb >= nwE - 1 where G is conjugate symmetric.
+template <typename Real>
+__device__ __forceinline__ Cplx<Real> g_upper(const TiledArgs<Real>& a, const Cplx<Real>* H, int ka, int wa, int kb,
+                                             int wb) {
+  const Geo& g = a.g;
+  const bool mir = a.half_g && wa + wb < g.nwE - 1;
+  if (mir) {
+    ka = a.k_neg[ka];
+    kb = a.k_neg[kb];
+    wa = g.nwE - 1 - wa;
+    wb = g.nwE - 1 - wb;
+  }
+  Cplx<Real> v = H[ka + static_cast<size_t>(g.nc) * wa + static_cast<size_t>(g.D) * (kb + static_cast<size_t>(g.nc) * wb)];
+  if (mir)
+    v.y = -v.y;
+  return v;
+}
+
 // Grid size of a tile launch; fills in the schedule fields of a.
 template <typename Real>
 inline unsigned tile_schedule(TiledArgs<Real>& a) {
   const Geo& g = a.g;
-  if (a.sym) {
+  if (a.sym >= SYM_CONJ) {
+    const unsigned tiles = static_cast<unsigned>(a.n_sym_tiles) * g.nv * a.nqg;
+    a.tile_perm = nullptr;
+    a.super_tile = a.n_super = 1;
+    a.n_xcd = a.tile_order == 0 ? 0 : 8;
+    return a.n_xcd ? (tiles + 7) / 8 * 8 : tiles;
+  }
+  if (a.sym == SYM_TRANSPOSE) {
     a.tile_perm = nullptr;
     a.super_tile = a.n_super = 1;
     a.n_xcd = 0;

@@ -61,10 +61,9 @@ __global__ void __launch_bounds__(256) uv_kernel(TiledArgs<Real> a) {
   const size_t D = g.D;
   const C* G0 = a.G + (2 * static_cast<size_t>(m)) * D * D;
   const C* G1 = G0 + D * D;
-  const size_t ru = k + static_cast<size_t>(g.nc) * (w + g.ext);
-  const size_t cu = kq + static_cast<size_t>(g.nc) * (w + nu + g.ext);
-  const C u0 = G0[ru + D * cu], u1 = G1[ru + D * cu];
-  const C v0 = G0[cu + D * ru], v1 = G1[cu + D * ru];
+  const int we = w + g.ext, wq = w + nu + g.ext;
+  const C u0 = g_upper(a, G0, k, we, kq, wq), u1 = g_upper(a, G1, k, we, kq, wq);
+  const C v0 = g_upper(a, G0, kq, wq, k, we), v1 = g_upper(a, G1, kq, wq, k, we);
   const Real alpha = static_cast<Real>(0.5 * a.desc[2 * m].sign);
   C* out = a.UV + (static_cast<size_t>(m) * 4 * nqv + qv) * P + p;
   const size_t plane = static_cast<size_t>(nqv) * P;
@@ -100,10 +99,21 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
   P2* Yl = reinterpret_cast<P2*>(lds);  // [b][a] (a fastest): {spin 0, spin 1}
   P2* Zl = Yl + (needY ? bs : 0);
   P2* Ul = Zl + (needZ ? bs : 0);       // [side][qi][k]: side 0 {a(u0-u1), a(u0+u1)}, 1 {v0-v1, v0+v1}
-  const size_t xoff = nc * static_cast<size_t>(w1 + e) + D * (nc * static_cast<size_t>(w2 + e));
-  const size_t yoff = nc * static_cast<size_t>(w2 + nu + e) + D * (nc * static_cast<size_t>(w1 + nu + e));
-  const size_t zoff = nc * static_cast<size_t>(nu + nw - 1 - w1 + e) +
-                      D * (nc * static_cast<size_t>(nu + nw - 1 - w2 + e));
+  // Blocks (wa, wb) of G (extended frequencies). Of a conjugate symmetric G only the half
+  // wa + wb >= nwE - 1 is read: another block is the conjugate of (-wa, -wb) at (-ka, -kb); its sign
+  // is applied where the block is staged (Y, Z) or scaled by alpha (X).
+  auto mirrored = [&](int wa, int wb) { return a.half_g && wa + wb < g.nwE - 1; };
+  auto block = [&](int wa, int wb) {
+    const bool m = mirrored(wa, wb);
+    return nc * static_cast<size_t>(m ? g.nwE - 1 - wa : wa) + D * (nc * static_cast<size_t>(m ? g.nwE - 1 - wb : wb));
+  };
+  const int wy = nu + e, wz = nu + nw - 1 + e;
+  const bool xm = mirrored(w1 + e, w2 + e), ym = mirrored(w2 + wy, w1 + wy), zm = mirrored(wz - w1, wz - w2);
+  const size_t xoff = block(w1 + e, w2 + e), yoff = block(w2 + wy, w1 + wy), zoff = block(wz - w1, wz - w2);
+  const Real xs_im = xm ? -1 : 1, ys_im = ym ? -1 : 1, zs_im = zm ? -1 : 1;
+  auto element = [&](int ka, int kb, bool m) {
+    return (m ? a.k_neg[ka] : ka) + D * (m ? a.k_neg[kb] : kb);
+  };
   const int nqv = g.nq * g.nv;
 
   int k1[PPT], k2[PPT];
@@ -198,6 +208,7 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
     const int ncc = nc * nc, n_items = NBK * ncc, n_walk = a.n_walkers;
     int psrc[PS], pdst[PS];
     bool puse[PS];
+    Real pim[PS];  // sign of the imaginary part
 #pragma unroll
     for (int j = 0; j < PS; ++j) {
       const int f = threadIdx.x + TT * j;
@@ -206,7 +217,8 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
       // Blocks in LDS order: Y (if staged), Z (if staged), X.
       const bool isx = blk == NBK - 1, isy = !isx && needY && blk == 0;
       const size_t boff = isx ? xoff : (isy ? yoff : zoff);
-      psrc[j] = puse[j] ? static_cast<int>(boff + (idx % nc) + D * (idx / nc)) : 0;
+      psrc[j] = puse[j] ? static_cast<int>(boff + element(idx % nc, idx / nc, isx ? xm : (isy ? ym : zm))) : 0;
+      pim[j] = isx ? xs_im : (isy ? ys_im : zs_im);
       pdst[j] = blk * bs + (idx / nc) * ld + idx % nc;
     }
     C pre[2][PS][2];
@@ -223,7 +235,7 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
 #pragma unroll
       for (int j = 0; j < PS; ++j)
         if (puse[j])
-          store_pair(Yl[pdst[j]], cur[j][0], cur[j][1]);
+          store_pair(Yl[pdst[j]], C{cur[j][0].x, cur[j][0].y * pim[j]}, C{cur[j][1].x, cur[j][1].y * pim[j]});
       __syncthreads();
     };
     auto consume = [&](int m) {
@@ -278,6 +290,15 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
   // staged blocks (each thread stages at most PPT elements per block, nc^2 <= 256 PPT), the
   // rank-one factors and (for few pairs per thread) the thread's own X entries.
   C pre[4][PPT], pre_uv, pre_x[2][kPrefetchX ? PPT : 1];
+  size_t ysrc[PPT], zsrc[PPT], xsrc[PPT];  // this thread's elements of the three blocks
+#pragma unroll
+  for (int j = 0; j < PPT; ++j) {
+    const int idx = threadIdx.x + TT * j;
+    const int idc = idx < nc * nc ? idx : 0;
+    ysrc[j] = yoff + element(idc % nc, idc / nc, ym);
+    zsrc[j] = zoff + element(idc % nc, idc / nc, zm);
+    xsrc[j] = xoff + element(k1[j], k2[j], xm);  // pair 0 for idle pairs
+  }
   auto prefetch = [&](int m) {
     if constexpr (kXFirst) {
       const int mc = m < a.n_walkers ? m : a.n_walkers - 1;
@@ -285,16 +306,13 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
       const C* H1 = H0 + DD;
 #pragma unroll
       for (int j = 0; j < PPT; ++j) {
-        const int idx = threadIdx.x + TT * j;
-        const int idc = idx < nc * nc ? idx : 0;
-        const size_t go = (idc % nc) + D * (idc / nc);
         if (needY) {
-          pre[0][j] = H0[yoff + go];
-          pre[1][j] = H1[yoff + go];
+          pre[0][j] = H0[ysrc[j]];
+          pre[1][j] = H1[ysrc[j]];
         }
         if (needZ) {
-          pre[2][j] = H0[zoff + go];
-          pre[3][j] = H1[zoff + go];
+          pre[2][j] = H0[zsrc[j]];
+          pre[3][j] = H1[zsrc[j]];
         }
       }
       pre_uv = a.UV[static_cast<size_t>(mc) * 4 * plane + (u_valid ? u_src : 0)];
@@ -306,21 +324,19 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
     for (int j = 0; j < PPT; ++j) {
       const int idx = threadIdx.x + TT * j;
       if (idx < nc * nc) {
-        const size_t go = (idx % nc) + D * (idx / nc);
         if (needY) {
-          pre[0][j] = H0[yoff + go];
-          pre[1][j] = H1[yoff + go];
+          pre[0][j] = H0[ysrc[j]];
+          pre[1][j] = H1[ysrc[j]];
         }
         if (needZ) {
-          pre[2][j] = H0[zoff + go];
-          pre[3][j] = H1[zoff + go];
+          pre[2][j] = H0[zsrc[j]];
+          pre[3][j] = H1[zsrc[j]];
         }
       }
       if constexpr (kPrefetchX) {
         if (ok[j]) {
-          const size_t xo = xoff + k1[j] + D * k2[j];
-          pre_x[0][j] = H0[xo];
-          pre_x[1][j] = H1[xo];
+          pre_x[0][j] = H0[xsrc[j]];
+          pre_x[1][j] = H1[xsrc[j]];
         }
       }
     }
@@ -337,9 +353,9 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
       if (idx < nc * nc) {
         const int li = (idx / nc) * ld + (idx % nc);
         if (needY)
-          store_pair(Yl[li], pre[0][j], pre[1][j]);
+          store_pair(Yl[li], C{pre[0][j].x, pre[0][j].y * ys_im}, C{pre[1][j].x, pre[1][j].y * ys_im});
         if (needZ)
-          store_pair(Zl[li], pre[2][j], pre[3][j]);
+          store_pair(Zl[li], C{pre[2][j].x, pre[2][j].y * zs_im}, C{pre[3][j].x, pre[3][j].y * zs_im});
       }
     }
     if (u_valid)
@@ -359,9 +375,8 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
     if constexpr (kXFirst) {
 #pragma unroll
       for (int j = 0; j < PPT; ++j) {
-        const size_t xo = xoff + k1[j] + D * k2[j];  // pair 0 for idle pairs
-        xr[j][0] = G0m[xo];
-        xr[j][1] = G0m[DD + xo];
+        xr[j][0] = G0m[xsrc[j]];
+        xr[j][1] = G0m[DD + xsrc[j]];
       }
       prefetch(m + 1);
     }
@@ -382,14 +397,13 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
         x1 = xw[1][j];
       }
       else {
-        const size_t xo = xoff + k1[j] + D * k2[j];
-        x0 = G0m[xo];
-        x1 = G0m[DD + xo];
+        x0 = G0m[xsrc[j]];
+        x1 = G0m[DD + xsrc[j]];
       }
       x0.x *= alpha;
-      x0.y *= alpha;
+      x0.y *= alpha * xs_im;
       x1.x *= alpha;
-      x1.y *= alpha;
+      x1.y *= alpha * xs_im;
 #pragma unroll
       for (int qi = 0; qi < QG; ++qi) {
         if (!qok[qi])
@@ -515,26 +529,62 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
         store(c, idx, tot[j][qi][c]);
     }
   }
-  if (a.sym && w1 != w2) {
-    // Mirror tile (w2, w1): G4(k2, w2, k1, w1) = G4(k1, w1, k2, w2), transposed through LDS (the
-    // staging area is free now) so that the stores run along k1 of the mirror tile.
-    double2* tl = reinterpret_cast<double2*>(lds);
+  if (a.sym == SYM_NONE)
+    return;
+  // Images of the tile (G4Sym) that no workgroup computes. P keeps the order of k1 up to a
+  // permutation of its Nc entries and is stored directly; T, C and both together (v = 0) go through
+  // LDS (the staging area is free now), so that the stores run along k1 of the image. Thread
+  // (k1, k2) of an image takes the tile's pair (src1, src2) below.
+  const bool ht = a.need_y, hp = a.need_z;
+  auto left_out = [&](int wa, int wb) {
+    return wa >= 0 && wa < nw && wb >= 0 && wb < nw && !sym_tile_computed(nw, nu, wa, wb, ht, hp, a.sym);
+  };
+  const int c1 = nw - 1 - nu - w2, c2 = nw - 1 - nu - w1;  // C
+  const int p1 = nw - 1 + nu - w1, p2 = nw - 1 + nu - w2;  // P
+  const bool img_t = (a.sym & 1) && w1 != w2;
+  const bool img_c = a.sym == SYM_CONJ ? left_out(c1, c2) : a.sym == SYM_CONJ_TRANSPOSE && w1 + w2 != nw - 1;
+  const bool img_p = a.sym == SYM_CONJ && left_out(p1, p2);
+  double2* tl = reinterpret_cast<double2*>(lds);
 #pragma unroll
-    for (int qi = 0; qi < QG; ++qi) {
-      if (!qok[qi])
+  for (int qi = 0; qi < QG; ++qi) {
+    if (!qok[qi])
+      continue;
+    const int q = a.k_ex[q0 + qi];
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if (a.ch[c] == PP_UP_DOWN) {
+        if (img_p)
+#pragma unroll
+          for (int j = 0; j < PPT; ++j)
+            if (ok[j])
+              store(c, g4_index(a.k_sub[k1[j] + nc * q], p1, a.k_sub[k2[j] + nc * q], p2, qv[qi]), tot[j][qi][c]);
         continue;
+      }
+      if (!img_t && !img_c)
+        continue;
+      __syncthreads();
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) {
-        __syncthreads();
+      for (int j = 0; j < PPT; ++j)
+        if (ok[j])
+          tl[k1[j] + ld * k2[j]] = tot[j][qi][c];
+      __syncthreads();
 #pragma unroll
-        for (int j = 0; j < PPT; ++j)
-          if (ok[j])
-            tl[k2[j] + nc * k1[j]] = tot[j][qi][c];
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < PPT; ++j)
-          if (ok[j])
-            store(c, g4_index(k1[j], w2, k2[j], w1, qv[qi]), tl[k1[j] + nc * k2[j]]);
+      for (int j = 0; j < PPT; ++j) {
+        if (!ok[j])
+          continue;
+        if (img_t)
+          store(c, g4_index(k1[j], w2, k2[j], w1, qv[qi]),
+                tl[a.k_sub[q + nc * k2[j]] + ld * a.k_sub[q + nc * k1[j]]]);
+        if (img_c) {
+          double2 v = tl[a.k_neg[a.k_add[k2[j] + nc * q]] + ld * a.k_neg[a.k_add[k1[j] + nc * q]]];
+          v.y = -v.y;
+          store(c, g4_index(k1[j], c1, k2[j], c2, qv[qi]), v);
+        }
+        if (img_t && img_c) {
+          double2 v = tl[a.k_neg[k1[j]] + ld * a.k_neg[k2[j]]];
+          v.y = -v.y;
+          store(c, g4_index(k1[j], c2, k2[j], c1, qv[qi]), v);
+        }
       }
     }
   }
@@ -645,6 +695,35 @@ std::vector<int> diagonal_tile_order(int nw, int strip) {
   return out;
 }
 
+std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>& w_ex, bool has_ph, bool has_pp,
+                                      int sym) {
+  std::vector<int> out;
+  auto used = [&](int w1, int w2) {
+    for (int nu : w_ex)
+      if (sym_tile_computed(nw, nu, w1, w2, has_ph, has_pp, sym))
+        return true;
+    return false;
+  };
+  // A tile's X block lies on the diagonal w1 - w2 = d, its Y block on -d and the conjugate of its Z
+  // block on d again, each shifted along it by v: strips of both diagonals together.
+  if (strip <= 0) {
+    for (int w2 = 0; w2 < nw; ++w2)
+      for (int w1 = 0; w1 < nw; ++w1)
+        if (used(w1, w2))
+          out.push_back(w1 | (w2 << 16));
+    return out;
+  }
+  for (int d = 0; d < nw; ++d)
+    for (int p0 = 0; p0 < nw - d; p0 += strip)
+      for (int sgn = 0; sgn < (d == 0 ? 1 : 2); ++sgn)
+        for (int p = p0; p < std::min(p0 + strip, nw - d); ++p) {
+          const int w1 = sgn ? p : p + d, w2 = sgn ? p + d : p;
+          if (used(w1, w2))
+            out.push_back(w1 | (w2 << 16));
+        }
+  return out;
+}
+
 size_t tiled_lds_bytes(const Geo& g, bool need_y, bool need_z, size_t cplx_bytes, int qg) {
   const size_t bs = static_cast<size_t>(g.nc) * (g.nc + 1);
   return cplx_bytes * (bs * 2 * ((need_y ? 1 : 0) + (need_z ? 1 : 0)) + 4 * static_cast<size_t>(qg) * g.nc);
@@ -691,7 +770,8 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
   if constexpr (std::is_same<Real, float>::value) {
     if (a.mfma && ts.threads == 256 && ppt == 1) {
       TiledArgs<float> b = a;
-      b.sym = false;  // the matrix-core tile writes no mirror tiles
+      b.sym = SYM_NONE;  // the matrix-core tile computes every tile and reads all of G
+      b.half_g = false;
       if (launch_g4_mfma(b, qg, st))
         return true;
     }

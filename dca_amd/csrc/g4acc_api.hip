@@ -134,10 +134,15 @@ struct g4acc_handle {
   bool large_ok = false, large_e = false, right_fused_ok = false;
   int g4_qg = 0;                   // tuning: momenta per G4 workgroup (0: register limit)
   int g4_mfma = 0;                 // tuning: rank-one G4 terms on the matrix cores (FP32 G, Nc <= 16)
-  // tuning: transpose-symmetric G4 tiles (one q = 0, one v = 0, channels among magnetic, charge,
-  // transverse); sym_ok when the geometry allows it.
+  // tuning: g4_sym = 0 computes every G4 tile. sym_ok: the transpose symmetry alone applies (one
+  // q = 0, one v = 0, channels among magnetic, charge, transverse). conj_sym: G4Sym of handles
+  // whose G is conjugate symmetric (SYM_NONE otherwise), their inversion table and tile tables in
+  // natural and diagonal order.
   int g4_sym = 0;
   bool sym_ok = false;
+  int conj_sym = SYM_NONE;
+  int *d_kneg = nullptr, *d_stab[2] = {nullptr, nullptr};
+  int n_stab = 0;
   // tuning: rank-one MAGNETIC / CHARGE terms of a batch as one matrix-core GEMM (g4_rank1.hip),
   // stored in d_R (complex64, one G4-sized plane per channel) and added by the tile kernel.
   int g4_rank1 = 0;
@@ -306,6 +311,61 @@ int detect_grid(int nc, const double* dft, std::vector<int>& xy, std::vector<int
       return L;
     }
   return 0;
+}
+
+// Finds the inversion k -> -k of the caller's momenta and whether G(-p1, -p2) = conj G(p1, p2)
+// holds for real M: the tables are those of an abelian group, dft(-k, r) = conj dft(k, r) and
+// G0(-p) = conj G0(p) (and the band phases likewise). The last must hold to `tol` of |G0|: the
+// conjugate then stands for an entry that differs from it by less than G's own rounding. A G0
+// without the symmetry (or holding a NaN) fails the test, and every tile is computed.
+bool conjugate_symmetric(const Geo& g, const g4acc_geometry* gm, double tol, double dft_tol, std::vector<int>& neg) {
+  const int nc = g.nc;
+  auto add = [&](int a, int b) { return gm->k_add[a + static_cast<size_t>(nc) * b]; };
+  auto sub = [&](int a, int b) { return gm->k_sub[a + static_cast<size_t>(nc) * b]; };  // k_b - k_a
+  int zero = -1;
+  for (int z = 0; z < nc && zero < 0; ++z) {
+    bool unit = true;
+    for (int k = 0; k < nc && unit; ++k)
+      unit = add(z, k) == k && add(k, z) == k;
+    if (unit)
+      zero = z;
+  }
+  if (zero < 0)
+    return false;
+  neg.assign(nc, -1);
+  for (int k = 0; k < nc; ++k) {
+    for (int j = 0; j < nc; ++j)
+      if (add(k, j) == zero)
+        neg[k] = j;
+    if (neg[k] < 0)
+      return false;
+  }
+  for (int a = 0; a < nc; ++a)
+    for (int b = 0; b < nc; ++b)
+      if (add(a, b) != add(b, a) || neg[add(a, b)] != add(neg[a], neg[b]) || sub(a, b) != add(b, neg[a]) ||
+          sub(a, add(b, a)) != b || sub(sub(a, b), b) != a)
+        return false;
+  auto pair = [&](const double* x, const double* y, double bound) {  // y = conj x
+    return std::abs(y[0] - x[0]) <= bound && std::abs(y[1] + x[1]) <= bound;
+  };
+  for (int r = 0; r < nc; ++r)
+    for (int k = 0; k < nc; ++k)
+      if (!pair(gm->dft + 2 * (k + static_cast<size_t>(nc) * r), gm->dft + 2 * (neg[k] + static_cast<size_t>(nc) * r),
+                dft_tol))
+        return false;
+  if (gm->band_phase)
+    for (int k = 0; k < nc; ++k)
+      if (!pair(gm->band_phase + 2 * k, gm->band_phase + 2 * neg[k], tol))
+        return false;
+  for (int w = 0; w < g.nwE; ++w)
+    for (int k = 0; k < nc; ++k)
+      for (int s = 0; s < 2; ++s) {
+        const double* x = gm->g0 + 2 * (s + 2 * (k + static_cast<size_t>(nc) * w));
+        const double* y = gm->g0 + 2 * (s + 2 * (neg[k] + static_cast<size_t>(nc) * (g.nwE - 1 - w)));
+        if (!pair(x, y, tol * std::hypot(x[0], x[1])))
+          return false;
+      }
+  return true;
 }
 
 // One walker's inputs as the staging reads them. The real walker (g4acc_walker), the CT-AUX
@@ -507,8 +567,10 @@ void run_mtog(g4acc_handle* h, int n_slots, hipStream_t st) {
   launch_mtog<Real>(mtog_args<Real>(h, n_slots), st);
 }
 
+// own_g: G is the handle's own (from M), not the caller's (g4acc_accumulate_G), which may lack the
+// conjugate symmetry.
 template <typename Real>
-void run_g4(g4acc_handle* h, int n_walkers) {
+void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
   if (h->use_tiled) {
     TiledArgs<Real> a;
     a.g = h->g;
@@ -537,7 +599,14 @@ void run_g4(g4acc_handle* h, int n_walkers) {
     a.tile_perm = h->d_tperm;
     a.sum_mode = h->sum_mode;
     a.mfma = h->g4_mfma;
-    a.sym = h->g4_sym != 0;
+    // One walker's launch is the G4 read-modify-write, which half of the tiles with scattered
+    // images does no faster (4x4, 8 transfers, three channels, 32 frequencies: 13.6 against 13.1 ms
+    // for 64 measurements); from two walkers on the tiles' reads and products count.
+    a.half_g = h->g4_sym && own_g && h->conj_sym;
+    a.sym = a.half_g && n_walkers > 1 ? h->conj_sym : h->g4_sym && h->sym_ok ? SYM_TRANSPOSE : SYM_NONE;
+    a.k_neg = h->d_kneg;
+    a.sym_tiles = h->d_stab[a.tile_order == 0 ? 0 : 1];
+    a.n_sym_tiles = h->n_stab;
     const bool r1 = std::is_same<Real, float>::value && h->g4_rank1 && h->d_R;
     a.R = r1 ? h->d_R : nullptr;
     a.n_r1 = h->n_r1;
@@ -914,8 +983,36 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
       ok = ok && (c == G4ACC_PARTICLE_HOLE_MAGNETIC || c == G4ACC_PARTICLE_HOLE_CHARGE ||
                   c == G4ACC_PARTICLE_HOLE_TRANSVERSE);
     h->sym_ok = ok && getenv("G4ACC_NO_SYM") == nullptr;
-    h->g4_sym = h->sym_ok ? 1 : 0;
   }
+  // Conjugate symmetry of G (single band, real M). Tolerances: complex64 G rounds at 2^-24, so
+  // 2^-30 of G0 does not show; complex128 G allows 16 roundings of G0 itself. The DFT table enters
+  // M -> G only for clusters without the L x L transforms.
+  if (h->use_tiled && getenv("G4ACC_NO_SYM") == nullptr) {
+    const bool dp = h->precision == G4ACC_FP64;
+    const double eps = 2.220446049250313e-16;
+    std::vector<int> neg;
+    if (conjugate_symmetric(g, gm, dp ? 16 * eps : 0x1p-30, dp && !h->grid_L ? 64 * eps : 1e-9, neg)) {
+      bool has_ph = false, has_pp = false, self = g.nv == 1 && gm->w_ex[0] == 0;
+      for (int c : h->channels)
+        (c == G4ACC_PARTICLE_PARTICLE_UP_DOWN ? has_pp : has_ph) = true;
+      for (int q : h->k_ex)
+        self = self && neg[q] == q;
+      h->conj_sym = self && !has_pp ? SYM_CONJ_TRANSPOSE : SYM_CONJ;
+      // One buffer: the inversion, then the tiles w1 fastest and on diagonal strips of two.
+      std::vector<int> tab = neg;
+      for (int k = 0; k < 2; ++k) {
+        const std::vector<int> t = symmetric_tile_order(g.nw, 2 * k, h->w_ex, has_ph, has_pp, h->conj_sym);
+        h->n_stab = static_cast<int>(t.size());
+        tab.insert(tab.end(), t.begin(), t.end());
+      }
+      if ((rc = h->alloc(&h->d_kneg, tab.size(), "symmetric tiles")) ||
+          (rc = h->check(hipMemcpy(h->d_kneg, tab.data(), sizeof(int) * tab.size(), hipMemcpyHostToDevice), "copy")))
+        return bail(rc);
+      for (int k = 0; k < 2; ++k)
+        h->d_stab[k] = h->d_kneg + g.nc + static_cast<size_t>(k) * h->n_stab;
+    }
+  }
+  h->g4_sym = h->sym_ok || h->conj_sym ? 1 : 0;
   h->d_g4.assign(h->channels.size(), nullptr);
   for (auto& p : h->d_g4)
     if ((rc = h->alloc(reinterpret_cast<double2**>(&p), h->g4_entries, "G4")))
@@ -1522,11 +1619,11 @@ int g4acc_accumulate_G(g4acc_handle* h, const double* G_ref, double sign) {
   if (rc == G4ACC_OK) {
     if (h->precision == G4ACC_FP64) {
       launch_import_G<double>(tmp, static_cast<double2*>(h->d_G), h->g, h->stream);
-      run_g4<double>(h, 1);
+      run_g4<double>(h, 1, false);
     }
     else {
       launch_import_G<float>(tmp, static_cast<float2*>(h->d_G), h->g, h->stream);
-      run_g4<float>(h, 1);
+      run_g4<float>(h, 1, false);
     }
     rc = h->check(hipStreamSynchronize(h->stream), "accumulate_G");
   }

@@ -90,6 +90,29 @@ struct G4Args {
 template <typename Real>
 void launch_g4(const G4Args<Real>& a, hipStream_t st);
 
+// Symmetries of the single-band G4 over the pairs p = (k, w), with Q = (q, v) the transfer:
+//   transpose    T: (p1, p2) -> (p2 + Q, p1 + Q): for particle-hole channels X and Y, and the two
+//                   rank-one factors, swap. Needs 2 Q = 0 (v = 0, q its own inverse).
+//   conjugate    C: (p1, p2) -> (-p2 - Q, -p1 - Q), value conjugated: the same swap when
+//                   G(-p1, -p2) = conj G(p1, p2), i.e. for real M and G0(-p) = conj G0(p).
+//   pair swap    P: (p1, p2) -> (Q - p1, Q - p2): X and Z of the pp channel swap.
+// SYM_TRANSPOSE uses T alone (one q = 0, one v = 0, no pp channel); SYM_CONJ uses C for the
+// particle-hole channels and P for pp; SYM_CONJ_TRANSPOSE C and T (no pp channel).
+enum G4Sym { SYM_NONE = 0, SYM_TRANSPOSE = 1, SYM_CONJ = 2, SYM_CONJ_TRANSPOSE = 3 };
+
+// Whether tile (w1, w2) of exchange frequency index nu is computed, for sym >= SYM_CONJ: the
+// tiles on or above the anti-diagonals about which C and P reflect (w1 + w2 = nw - 1 - nu and
+// nw - 1 + nu; the lower of the two bounds both, so every tile left out has its image in), and
+// those whose image of a channel in use lies outside the compact frequencies.
+__host__ __device__ inline bool sym_tile_computed(int nw, int nu, int w1, int w2, bool has_ph, bool has_pp, int sym) {
+  const int an = nu < 0 ? -nu : nu;
+  if (w1 + w2 >= nw - 1 - an)
+    return sym != SYM_CONJ_TRANSPOSE || w1 <= w2;
+  const int hi = w1 > w2 ? w1 : w2, lo = w1 > w2 ? w2 : w1;
+  return (has_ph && (nw - 1 - nu - hi < 0 || nw - 1 - nu - lo >= nw)) ||
+         (has_pp && (nw - 1 + nu - hi < 0 || nw - 1 + nu - lo >= nw));
+}
+
 // Single-band, all channels in one launch (g4_tiled.hip). Returns false when the geometry is
 // outside what the tiled kernel handles (the caller then uses launch_g4 per channel).
 template <typename Real>
@@ -121,10 +144,13 @@ struct TiledArgs {
   const int* r1_planes;  // device, n_r1 entries
   int r1_slot[4];
   bool need_y, need_z, has_trans;
-  // Transpose symmetry (one exchange momentum q = 0, one exchange frequency v = 0, channels among
-  // magnetic, charge and transverse): G4 over ((k1, w1), (k2, w2)) is then symmetric, so only the
-  // tiles w1 <= w2 are computed and each also writes its mirror tile (w2, w1).
-  bool sym = false;
+  // Symmetries of G4 used to compute a part of the tiles and write their images (G4Sym).
+  int sym = 0;
+  // G is conjugate symmetric: only its half wa + wb >= nwE - 1 (extended frequencies) is read.
+  bool half_g = false;
+  const int* k_neg = nullptr;       // device [Nc], index(-k); half_g only
+  const int* sym_tiles = nullptr;   // computed tiles (w1 | w2 << 16) for sym >= SYM_CONJ, in dispatch order
+  int n_sym_tiles = 0;
 };
 
 template <typename Real>
@@ -142,6 +168,10 @@ bool launch_g4_band(TiledArgs<Real> a, hipStream_t st);
 int tiled_pairs_per_thread(int nc);
 // Tile schedule 2: (w1 | w2 << 16) for all nw^2 frequency pairs, in dispatch order.
 std::vector<int> diagonal_tile_order(int nw, int strip);
+// The tiles computed for any of the exchange frequencies under sym >= SYM_CONJ, on diagonal strips
+// (strip > 0) or w1 fastest (strip = 0).
+std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>& w_ex, bool has_ph, bool has_pp,
+                                      int sym);
 // LDS of one tile workgroup with momentum groups of qg (staged blocks and rank-one factors).
 size_t tiled_lds_bytes(const Geo& g, bool need_y, bool need_z, size_t cplx_bytes, int qg);
 

@@ -20,3 +20,7 @@ mv "$HERE/_build/host_logic_test.tmp" "$HERE/_build/host_logic_test"
 g++ -std=c++17 -O2 -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__ -I/opt/rocm/include \
     "$HERE/site_fft_test.cpp" -o "$HERE/_build/site_fft_test.tmp"
 mv "$HERE/_build/site_fft_test.tmp" "$HERE/_build/site_fft_test"
+# The tile sets of the symmetric G4 update, checked on the CPU.
+g++ -std=c++17 -O2 -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__ -I/opt/rocm/include \
+    "$HERE/sym_tiles_test.cpp" -o "$HERE/_build/sym_tiles_test.tmp"
+mv "$HERE/_build/sym_tiles_test.tmp" "$HERE/_build/sym_tiles_test"

@@ -110,6 +110,18 @@ def test_site_fft_host():
     assert out.returncode == 0 and out.stdout.strip() == "OK", out.stdout
 
 
+def test_symmetric_tiles_cover_g4_once():
+    """The computed tiles of the symmetric G4 update and their images (tests/cpp/sym_tiles_test.cpp)."""
+    exe = os.path.join(HERE, "cpp", "_build", "sym_tiles_test")
+    if not os.path.exists(exe):
+        os.makedirs(os.path.dirname(exe), exist_ok=True)
+        subprocess.run(["g++", "-std=c++17", "-O2", "-Wno-unknown-pragmas", "-D__HIP_PLATFORM_AMD__",
+                        "-I/opt/rocm/include", os.path.join(HERE, "cpp", "sym_tiles_test.cpp"), "-o", exe],
+                       check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.strip() == "OK", out.stdout
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("nb,L,precision,tol", [(1, 4, 0, 1e-12), (1, 4, 1, 1e-6), (3, 2, 0, 1e-12)])
 def test_cpp_mirror_matches_oracle(oracle_lib, tmp_path, nb, L, precision, tol):
