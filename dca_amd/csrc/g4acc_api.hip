@@ -192,6 +192,9 @@ struct g4acc_handle {
     *p = static_cast<T*>(q);
     return G4ACC_OK;
   }
+  // The G4 stage reads the half w1 + w2 >= nwE - 1 of G only (the matrix-core tile kernel of
+  // g4_mfma reads all of it), so M -> G forms that half.
+  bool half_g() const { return g4_sym && conj_sym && !(g4_mfma && precision == G4ACC_FP32 && g.nc <= 16); }
   size_t cplx_bytes() const { return precision == G4ACC_FP64 ? 16 : 8; }
 };
 
@@ -559,12 +562,15 @@ MtoGArgs<Real> mtog_args(g4acc_handle* h, int n_slots) {
 }
 
 template <typename Real>
-void run_mtog(g4acc_handle* h, int n_slots, hipStream_t st) {
+void run_mtog(g4acc_handle* h, int n_slots, hipStream_t st, bool half_g) {
   launch_sort(h->d_desc, h->g, n_slots, h->max_vertices, h->d_site_map, h->d_perm, h->d_off, h->d_err, st);
   if (h->non_dd)
     launch_sort(h->d_desc, h->g, n_slots, h->max_vertices, h->d_site_map, h->d_perm2, h->d_off2, h->d_err, st,
                 true);
-  launch_mtog<Real>(mtog_args<Real>(h, n_slots), st);
+  MtoGArgs<Real> a = mtog_args<Real>(h, n_slots);
+  if (half_g)
+    a.w_sum_min = h->g.nwE - 1;
+  launch_mtog<Real>(a, st);
 }
 
 // own_g: G is the handle's own (from M), not the caller's (g4acc_accumulate_G), which may lack the
@@ -602,8 +608,9 @@ void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
     // One walker's launch is the G4 read-modify-write, which half of the tiles with scattered
     // images does no faster (4x4, 8 transfers, three channels, 32 frequencies: 13.6 against 13.1 ms
     // for 64 measurements); from two walkers on the tiles' reads and products count.
-    a.half_g = h->g4_sym && own_g && h->conj_sym;
-    a.sym = a.half_g && n_walkers > 1 ? h->conj_sym : h->g4_sym && h->sym_ok ? SYM_TRANSPOSE : SYM_NONE;
+    a.half_g = own_g && h->half_g();
+    a.sym_few = h->g4_sym && h->sym_ok ? SYM_TRANSPOSE : SYM_NONE;
+    a.sym = a.half_g && n_walkers > 1 ? h->conj_sym : a.sym_few;
     a.k_neg = h->d_kneg;
     a.sym_tiles = h->d_stab[a.tile_order == 0 ? 0 : 1];
     a.n_sym_tiles = h->n_stab;
@@ -682,9 +689,9 @@ void launch_stage(g4acc_handle* h, int n_walkers, int stage, hipStream_t st) {
   }
   if (stage == 0) {
     if (h->precision == G4ACC_FP64)
-      run_mtog<double>(h, 2 * n_walkers, st);
+      run_mtog<double>(h, 2 * n_walkers, st, h->half_g());
     else
-      run_mtog<float>(h, 2 * n_walkers, st);
+      run_mtog<float>(h, 2 * n_walkers, st, h->half_g());
   }
   else if (h->precision == G4ACC_FP64)
     run_g4<double>(h, n_walkers);
@@ -919,13 +926,10 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
     h->chunk = static_cast<int>(W2);
   const size_t CH = h->chunk;
 
-  if ((rc = h->alloc(&h->d_kadd, nc2, "k_add")) || (rc = h->alloc(&h->d_ksub, nc2, "k_sub")) ||
-      (rc = h->alloc(&h->d_kex, g.nq, "k_ex")) || (rc = h->alloc(&h->d_wex, g.nv, "w_ex")) ||
-      (rc = h->alloc(&h->d_tperm, static_cast<size_t>(g.nw) * g.nw, "tile order")) ||
-      (rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_dft), cb * nc2, "dft")) ||
+  if ((rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_dft), cb * nc2, "dft")) ||
       (rc = h->alloc(&h->d_G0, static_cast<size_t>(g.nb) * g.nb * 2 * g.nc * g.nwE, "G0")) ||
       (rc = h->alloc(&h->d_perm, W2 * NM, "perm")) ||
-      (rc = h->alloc(&h->d_off, W2 * (g.n_orb + 1), "off")) || (rc = h->alloc(&h->d_err, 1, "err")) ||
+      (rc = h->alloc(&h->d_off, W2 * (g.n_orb + 1), "off")) ||
       (rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_T), cb * W2 * NM * g.nwE, "T")) ||
       (rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_B),
                      h->fused_mtog && !h->large_ok ? 1 : cb * CH * NM * D, "B")) ||
@@ -973,6 +977,13 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
                        cb * W2 / 2 * 4 * g.nq * g.nv * g.nc * g.nw, "UV")))
       return bail(rc);
   }
+  // The integer tables share one buffer, filled by one copy.
+  std::vector<int> tables;
+  std::vector<std::pair<int**, size_t>> table_at;
+  auto table = [&](int** p, const std::vector<int>& v) {
+    table_at.emplace_back(p, tables.size());
+    tables.insert(tables.end(), v.begin(), v.end());
+  };
   // Transpose symmetry of G4 over ((k1, w1), (k2, w2)): q = 0 (k + q = k for every k), v = 0 and
   // channels whose terms pair G(p1, p2) with G(p2, p1) only.
   {
@@ -998,18 +1009,12 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
       for (int q : h->k_ex)
         self = self && neg[q] == q;
       h->conj_sym = self && !has_pp ? SYM_CONJ_TRANSPOSE : SYM_CONJ;
-      // One buffer: the inversion, then the tiles w1 fastest and on diagonal strips of two.
-      std::vector<int> tab = neg;
-      for (int k = 0; k < 2; ++k) {
+      table(&h->d_kneg, neg);
+      for (int k = 0; k < 2; ++k) {  // w1 fastest, and on diagonal strips of two
         const std::vector<int> t = symmetric_tile_order(g.nw, 2 * k, h->w_ex, has_ph, has_pp, h->conj_sym);
         h->n_stab = static_cast<int>(t.size());
-        tab.insert(tab.end(), t.begin(), t.end());
+        table(&h->d_stab[k], t);
       }
-      if ((rc = h->alloc(&h->d_kneg, tab.size(), "symmetric tiles")) ||
-          (rc = h->check(hipMemcpy(h->d_kneg, tab.data(), sizeof(int) * tab.size(), hipMemcpyHostToDevice), "copy")))
-        return bail(rc);
-      for (int k = 0; k < 2; ++k)
-        h->d_stab[k] = h->d_kneg + g.nc + static_cast<size_t>(k) * h->n_stab;
     }
   }
   h->g4_sym = h->sym_ok || h->conj_sym ? 1 : 0;
@@ -1034,7 +1039,6 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
   // Constant tables. On a square cluster the sites are relabelled x + L y (the sort orders the
   // vertices by that label and the DFT columns follow it), so the right site DFT can run as two
   // L-point passes (G4ACC_DENSE_DFT=1 keeps the caller's labels and the dense DFT).
-  const std::vector<int> tperm = diagonal_tile_order(g.nw, 2);
   std::vector<double> dft_lab(gm->dft, gm->dft + 2 * static_cast<size_t>(nc2));
   if (h->grid_L) {
     for (int r = 0; r < g.nc; ++r)
@@ -1043,27 +1047,30 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
         dft_lab[2 * (k + static_cast<size_t>(g.nc) * xy[r]) + 1] =
             gm->dft[2 * (k + static_cast<size_t>(g.nc) * r) + 1];
       }
-    if ((rc = h->alloc(&h->d_site_map, g.nc, "site map")) || (rc = h->alloc(&h->d_kmap, g.nc, "k map")) ||
-        (rc = h->check(hipMemcpy(h->d_site_map, xy.data(), sizeof(int) * g.nc, hipMemcpyHostToDevice), "copy")) ||
-        (rc = h->check(hipMemcpy(h->d_kmap, kxy_to_k.data(), sizeof(int) * g.nc, hipMemcpyHostToDevice), "copy")))
-      return bail(rc);
+    table(&h->d_site_map, xy);
+    table(&h->d_kmap, kxy_to_k);
   }
   std::vector<unsigned char> dftbuf;
   if (h->precision == G4ACC_FP64)
     upload_dft<double>(dftbuf, dft_lab.data(), g.nc);
   else
     upload_dft<float>(dftbuf, dft_lab.data(), g.nc);
-  if ((rc = h->check(hipMemcpy(h->d_kadd, gm->k_add, sizeof(int) * nc2, hipMemcpyHostToDevice), "copy")) ||
-      (rc = h->check(hipMemcpy(h->d_ksub, gm->k_sub, sizeof(int) * nc2, hipMemcpyHostToDevice), "copy")) ||
-      (rc = h->check(hipMemcpy(h->d_kex, gm->k_ex, sizeof(int) * g.nq, hipMemcpyHostToDevice), "copy")) ||
-      (rc = h->check(hipMemcpy(h->d_wex, gm->w_ex, sizeof(int) * g.nv, hipMemcpyHostToDevice), "copy")) ||
-      (rc = h->check(hipMemcpy(h->d_tperm, tperm.data(), sizeof(int) * tperm.size(), hipMemcpyHostToDevice),
-                     "copy")) ||
+  table(&h->d_kadd, std::vector<int>(gm->k_add, gm->k_add + nc2));
+  table(&h->d_ksub, std::vector<int>(gm->k_sub, gm->k_sub + nc2));
+  table(&h->d_kex, h->k_ex);
+  table(&h->d_wex, h->w_ex);
+  table(&h->d_tperm, diagonal_tile_order(g.nw, 2));
+  table(&h->d_err, {0});
+  int* d_tables = nullptr;
+  if ((rc = h->alloc(&d_tables, tables.size(), "tables")))
+    return bail(rc);
+  for (const auto& t : table_at)
+    *t.first = d_tables + t.second;
+  if ((rc = h->check(hipMemcpy(d_tables, tables.data(), sizeof(int) * tables.size(), hipMemcpyHostToDevice), "copy")) ||
       (rc = h->check(hipMemcpy(h->d_dft, dftbuf.data(), dftbuf.size(), hipMemcpyHostToDevice), "copy")) ||
       (rc = h->check(hipMemcpy(h->d_G0, gm->g0,
                                sizeof(double2) * g.nb * g.nb * 2 * g.nc * g.nwE, hipMemcpyHostToDevice),
-                     "copy")) ||
-      (rc = h->check(hipMemset(h->d_err, 0, sizeof(int)), "memset")))
+                     "copy")))
     return bail(rc);
   if (gm->band_phase &&
       (rc = h->check(hipMemcpy(h->d_bphase, gm->band_phase, sizeof(double2) * g.nb * g.nc,
@@ -1447,9 +1454,9 @@ int compute_G_impl(g4acc_handle* h, const WalkerIn& w, bool general, int memory,
   G4_TRY(quiesce(h));
   G4_TRY(stage_walkers(h, &w, 1, memory, h->stream));
   if (h->precision == G4ACC_FP64)
-    run_mtog<double>(h, 2, h->stream);
+    run_mtog<double>(h, 2, h->stream, false);  // the caller gets all of G
   else
-    run_mtog<float>(h, 2, h->stream);
+    run_mtog<float>(h, 2, h->stream, false);
   double2* tmp = nullptr;
   const size_t n = g4acc_g_size(h);
   G4_TRY(h->check(hipMalloc(&tmp, sizeof(double2) * n), "hipMalloc(export)"));

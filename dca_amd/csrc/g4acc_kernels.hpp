@@ -41,6 +41,10 @@ struct MtoGArgs {
   // runs as two L-point passes; kmap[kx + L ky] is the caller's momentum index. L = 0: dense DFT.
   int grid_L;
   const int* kmap;
+  // Smallest w1 + w2 (extended frequencies) the consumer reads: nwE - 1 where G is conjugate
+  // symmetric and the tile kernel reads that half only, else 0. Blocks of G wholly below it are
+  // neither computed nor written.
+  int w_sum_min = 0;
 };
 
 // M = diag(exp_v - 1) N for one n x n matrix (column-major, leading dimensions ldn, ldm).
@@ -145,7 +149,7 @@ struct TiledArgs {
   int r1_slot[4];
   bool need_y, need_z, has_trans;
   // Symmetries of G4 used to compute a part of the tiles and write their images (G4Sym).
-  int sym = 0;
+  int sym = 0, sym_few = 0;  // sym_few: where the launch has few tiles
   // G is conjugate symmetric: only its half wa + wb >= nwE - 1 (extended frequencies) is read.
   bool half_g = false;
   const int* k_neg = nullptr;       // device [Nc], index(-k); half_g only

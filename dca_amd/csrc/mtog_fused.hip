@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(256) mtog_left_fused(const SlotDesc* __restric
 // workgroup's frequencies are staged once.
 template <typename Real, int NC, int TW, bool SEP>
 __global__ void __launch_bounds__(256) mtog_right_fused(const SlotDesc* __restrict__ desc, Geo g,
-                                                        int n_max, int slot0,
+                                                        int n_max, int slot0, int w_sum_min,
                                                         const int* __restrict__ off,
                                                         const Cplx<Real>* __restrict__ T,
                                                         const Cplx<Real>* __restrict__ A,
@@ -117,6 +117,8 @@ __global__ void __launch_bounds__(256) mtog_right_fused(const SlotDesc* __restri
   const int p1 = blockIdx.x * 64 + lane;
   const int w2wg = blockIdx.y * WT;           // first frequency of the workgroup
   const int w2b = w2wg + wave * TW;           // first frequency of this wave
+  if (w2wg + WT - 1 + (static_cast<int>(blockIdx.x) * 64 + 63) / NC < w_sum_min)
+    return;
   const int n = desc[slot].n;
   const bool active = p1 < g.D && w2b < g.nwE;
   const int* O = off + static_cast<size_t>(slot) * (NC + 1);
@@ -273,7 +275,7 @@ constexpr int mtog_mfma_max_vertices(int nc) { return 4 * (mtog_mfma_max_steps()
 // tiles of its rows, so the step table is built once per slot.
 template <int NC, bool SEP>
 __global__ void __launch_bounds__(256) mtog_right_mfma(const SlotDesc* __restrict__ desc, Geo g,
-                                                       int n_max, int slot0,
+                                                       int n_max, int slot0, int w_sum_min,
                                                        const int* __restrict__ off,
                                                        const float2* __restrict__ T,
                                                        const float2* __restrict__ A,
@@ -360,7 +362,10 @@ __global__ void __launch_bounds__(256) mtog_right_mfma(const SlotDesc* __restric
   const int pc = p_ok ? pl : g.D - 1;
 
   const int n_wt = (g.nwE + 15) / 16;
-  for (int wt = blockIdx.y; wt < n_wt; wt += gridDim.y) {
+  // The first frequency tile that reaches w_sum_min with the workgroup's highest row.
+  const int w_first = w_sum_min - 15 - static_cast<int>((blockIdx.x + 1) * (16 * TPW) - 1) / NC;
+  const int wt_first = w_first > 0 ? (w_first + 15) / 16 : 0;
+  for (int wt = wt_first + blockIdx.y; wt < n_wt; wt += gridDim.y) {
     const int w0 = wt * 16;
     __syncthreads();  // the previous tile's epilogue has read G0l and Xl
     for (int i = threadIdx.x; i < NC * 16; i += 256) {
@@ -552,10 +557,10 @@ void launch_fused_nc(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st) {
       const int rows = NC == 16 ? 32 : 64;  // p1 rows per workgroup (two waves per tile for Nc = 16)
       const dim3 grid((g.D + rows - 1) / rows, 1, ns);  // each workgroup walks all frequency tiles
       if (sep)
-        hipLaunchKernelGGL((mtog_right_mfma<NC, kSepM>), grid, dim3(256), 0, st, a.desc, g, a.n_max, s0, a.off,
+        hipLaunchKernelGGL((mtog_right_mfma<NC, kSepM>), grid, dim3(256), 0, st, a.desc, g, a.n_max, s0, a.w_sum_min, a.off,
                            a.T, a.A, a.dft, a.bphase, a.G0, a.kmap, a.G);
       else if constexpr (NC <= 8)
-        hipLaunchKernelGGL((mtog_right_mfma<NC, false>), grid, dim3(256), 0, st, a.desc, g, a.n_max, s0, a.off,
+        hipLaunchKernelGGL((mtog_right_mfma<NC, false>), grid, dim3(256), 0, st, a.desc, g, a.n_max, s0, a.w_sum_min, a.off,
                            a.T, a.A, a.dft, a.bphase, a.G0, nullptr, a.G);
       return;
     }
@@ -566,9 +571,9 @@ void launch_fused_nc(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st) {
   constexpr bool kSepRight = kSep && (NC != 64 || std::is_same<Real, double>::value);
   if (sep && kSepRight)
     hipLaunchKernelGGL((mtog_right_fused<Real, NC, TW, kSepRight>), grid, dim3(256), 0, st, a.desc, g, a.n_max,
-                       s0, a.off, a.T, a.A, a.dft, a.bphase, a.G0, a.kmap, a.G);
+                       s0, a.w_sum_min, a.off, a.T, a.A, a.dft, a.bphase, a.G0, a.kmap, a.G);
   else
-    hipLaunchKernelGGL((mtog_right_fused<Real, NC, TW, false>), grid, dim3(256), 0, st, a.desc, g, a.n_max, s0,
+    hipLaunchKernelGGL((mtog_right_fused<Real, NC, TW, false>), grid, dim3(256), 0, st, a.desc, g, a.n_max, s0, a.w_sum_min,
                        a.off, a.T, a.A, a.dft, a.bphase, a.G0, nullptr, a.G);
 }
 

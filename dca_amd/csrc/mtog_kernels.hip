@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(256) dft_left_kernel(const SlotDesc* __restric
 // over the column sort (off, T are the column order's arrays).
 template <typename Real>
 __global__ void __launch_bounds__(256) ndft_right_kernel(const SlotDesc* __restrict__ desc, Geo g,
-                                                         int n_max, int slot0,
+                                                         int n_max, int slot0, int w_sum_min,
                                                          const int* __restrict__ off,
                                                          const Cplx<Real>* __restrict__ T,
                                                          const Cplx<Real>* __restrict__ A,
@@ -184,6 +184,8 @@ __global__ void __launch_bounds__(256) ndft_right_kernel(const SlotDesc* __restr
   if (p1 >= g.D)
     return;
   const int o2 = q2 % g.n_orb, w2 = q2 / g.n_orb;
+  if (w2 + (static_cast<int>(blockIdx.x) * 256 + 255) / g.n_orb < w_sum_min)
+    return;
   const int* O = off + static_cast<size_t>(slot) * (g.n_orb + 1);
   const C* Ts = T + static_cast<size_t>(slot) * g.nwE * n_max;
   const C* As = A + static_cast<size_t>(blockIdx.z) * g.D * n_max;
@@ -199,7 +201,7 @@ __global__ void __launch_bounds__(256) ndft_right_kernel(const SlotDesc* __restr
 // NB bands as a compile-time constant: the nb x nb blocks M~(e, f) and the G0 factors stay in
 // registers (with a run-time band count they went to scratch memory).
 template <typename Real, int NB>
-__global__ void __launch_bounds__(256) dft_right_G_kernel(Geo g, int slot0,
+__global__ void __launch_bounds__(256) dft_right_G_kernel(Geo g, int slot0, int w_sum_min,
                                                           const Cplx<Real>* __restrict__ dft,
                                                           const double2* __restrict__ bphase,
                                                           const double2* __restrict__ G0,
@@ -222,7 +224,8 @@ __global__ void __launch_bounds__(256) dft_right_G_kernel(Geo g, int slot0,
   }
   const int kw1 = static_cast<int>(bx * blockDim.x + threadIdx.x);
   const int kw2 = static_cast<int>(by);
-  if (kw1 >= KW)
+  // Set for one band only, where the rows of a block are those of ndft_right_kernel's.
+  if (kw1 >= KW || kw2 / g.nc + (static_cast<int>(bx) * 256 + 255) / g.nc < w_sum_min)
     return;
   const int k1 = kw1 % g.nc, w1 = kw1 / g.nc;
   const int k2 = kw2 % g.nc, w2 = kw2 / g.nc;
@@ -343,14 +346,14 @@ void launch_mtog(const MtoGArgs<Real>& a, hipStream_t st) {
     hipLaunchKernelGGL(dft_left_kernel<Real>, dim3((g.D + 255) / 256, a.n_max, ns), dim3(256), 0, st,
                        a.desc, g, a.n_max, s0, a.dft, a.B, a.A);
     hipLaunchKernelGGL(ndft_right_kernel<Real>, dim3((g.D + 255) / 256, g.D, ns), dim3(256), 0, st,
-                       a.desc, g, a.n_max, s0, a.off2, a.T2, a.A, a.E);
+                       a.desc, g, a.n_max, s0, a.w_sum_min, a.off2, a.T2, a.A, a.E);
     const int KW = g.nc * g.nwE;
     const dim3 grid((KW + 255) / 256, KW, ns);
     switch (g.nb) {
-      case 1: hipLaunchKernelGGL((dft_right_G_kernel<Real, 1>), grid, dim3(256), 0, st, g, s0, a.dft, a.bphase, a.G0, a.E, a.G); break;
-      case 2: hipLaunchKernelGGL((dft_right_G_kernel<Real, 2>), grid, dim3(256), 0, st, g, s0, a.dft, a.bphase, a.G0, a.E, a.G); break;
-      case 3: hipLaunchKernelGGL((dft_right_G_kernel<Real, 3>), grid, dim3(256), 0, st, g, s0, a.dft, a.bphase, a.G0, a.E, a.G); break;
-      default: hipLaunchKernelGGL((dft_right_G_kernel<Real, 4>), grid, dim3(256), 0, st, g, s0, a.dft, a.bphase, a.G0, a.E, a.G); break;
+      case 1: hipLaunchKernelGGL((dft_right_G_kernel<Real, 1>), grid, dim3(256), 0, st, g, s0, a.w_sum_min, a.dft, a.bphase, a.G0, a.E, a.G); break;
+      case 2: hipLaunchKernelGGL((dft_right_G_kernel<Real, 2>), grid, dim3(256), 0, st, g, s0, a.w_sum_min, a.dft, a.bphase, a.G0, a.E, a.G); break;
+      case 3: hipLaunchKernelGGL((dft_right_G_kernel<Real, 3>), grid, dim3(256), 0, st, g, s0, a.w_sum_min, a.dft, a.bphase, a.G0, a.E, a.G); break;
+      default: hipLaunchKernelGGL((dft_right_G_kernel<Real, 4>), grid, dim3(256), 0, st, g, s0, a.w_sum_min, a.dft, a.bphase, a.G0, a.E, a.G); break;
     }
   }
 }

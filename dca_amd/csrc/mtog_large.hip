@@ -61,7 +61,7 @@ struct Mfma16<double> {
 // Loads past the site's vertices or the tile's edges read clamped, in-bounds addresses and are
 // zeroed before use.
 template <typename Real, int NC>
-__global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0,
+__global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0, int w_sum_min,
                                                     const int* __restrict__ off,
                                                     const Cplx<Real>* __restrict__ T,
                                                     const Cplx<Real>* __restrict__ A,
@@ -80,6 +80,8 @@ __global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0,
   const bool p_ok = pl < D;
   const int pc = p_ok ? pl : D - 1;
   const int w0 = blockIdx.y * 64;
+  // Tiles below the needed half: pairs are read by mtog_site_G in blocks of 64 rows and one w2.
+  const int w1_hi = (static_cast<int>(blockIdx.x) * 64 + 63) / NC;
   int wc[4];
   bool w_ok[4];
 #pragma unroll
@@ -88,6 +90,8 @@ __global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0,
     w_ok[t] = w < nwE;
     wc[t] = w_ok[t] ? w : nwE - 1;
   }
+  if (w0 + 63 + w1_hi < w_sum_min)
+    return;
   for (int r = 0; r < NC; ++r) {
     const int b = O[r], e = O[r + 1];
     V cr[4], ci[4];
@@ -134,7 +138,8 @@ __global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0,
 // the rows y = q, q + 4, ... over x into LDS; pass 2: it transforms the columns kx = q, q + 4, ...
 // over y and writes G for the L momenta (kx, ky) of each.
 template <typename Real, int L>
-__global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, const Cplx<Real>* __restrict__ E,
+__global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, int w_sum_min,
+                                                   const Cplx<Real>* __restrict__ E,
                                                    const double2* __restrict__ bphase,
                                                    const double2* __restrict__ G0,
                                                    const int* __restrict__ kmap,
@@ -151,6 +156,8 @@ __global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, const Cplx<
   const bool p_ok = p1 < D;
   const int pc = p_ok ? p1 : D - 1;
   const int w2 = blockIdx.y;
+  if (w2 + (static_cast<int>(blockIdx.x) * 64 + 63) / NC < w_sum_min)
+    return;
   const C* Eb = E + static_cast<size_t>(blockIdx.z) * D * D + static_cast<size_t>(D) * NC * w2 + pc;
   if (threadIdx.x < NC)
     Kl[threadIdx.x] = kmap[threadIdx.x];
@@ -214,6 +221,7 @@ __global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, const Cplx<
 // which keeps the per-step address arithmetic to one multiply-add per load.
 template <int L>
 __global__ void __launch_bounds__(64 * L, 4) mtog_right_block(Geo g, int n_max, int slot0, int n_wb, int xcd_map,
+                                                            int w_sum_min,
                                                             const int* __restrict__ off,
                                                             const Cplx<float>* __restrict__ T,
                                                             const Cplx<float>* __restrict__ A,
@@ -238,7 +246,17 @@ __global__ void __launch_bounds__(64 * L, 4) mtog_right_block(Geo g, int n_max, 
   unsigned lid = blockIdx.x;
   if (xcd_map)
     lid = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-  const int p0 = static_cast<int>(lid / n_wb) * 16, w0 = static_cast<int>(lid % n_wb) * 16;
+  int pb = static_cast<int>(lid / n_wb);
+  const int w0 = static_cast<int>(lid % n_wb) * 16;
+  if (w_sum_min > 0) {
+    // Only the blocks with w1 + w2 >= w_sum_min: alternating low and high rows gives every XCD's
+    // range the same share of them.
+    const int n_pb = static_cast<int>(gridDim.x) / n_wb;
+    pb = pb & 1 ? n_pb - 1 - (pb >> 1) : pb >> 1;
+    if (w0 + 15 + (pb * 16 + 15) / NC < w_sum_min)
+      return;
+  }
+  const int p0 = pb * 16;
   if (threadIdx.x < NC)
     Kl[threadIdx.x] = kmap[threadIdx.x];
   // Site offsets through LDS: reading them in the step loop then waits on LDS only, not on the
@@ -667,14 +685,14 @@ void launch_mtog_large(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st) 
       const int n_wb = (g.nwE + 15) / 16;
       const unsigned nblk = static_cast<unsigned>((g.D + 15) / 16) * n_wb;
       hipLaunchKernelGGL((mtog_right_block<L>), dim3(nblk, 1, ns), dim3(64 * L), 0, st, g, a.n_max, s0,
-                         n_wb, nblk % 8 == 0 ? 1 : 0, a.off, a.T, a.A, a.bphase, a.G0, a.kmap, a.G);
+                         n_wb, nblk % 8 == 0 ? 1 : 0, a.w_sum_min, a.off, a.T, a.A, a.bphase, a.G0, a.kmap, a.G);
       return;
     }
   }
   const dim3 g3((g.D + 63) / 64, (g.nwE + 63) / 64, ns);
-  hipLaunchKernelGGL((mtog_s3_mfma<Real, NC>), g3, dim3(256), 0, st, g, a.n_max, s0, a.off, a.T, a.A, a.E);
+  hipLaunchKernelGGL((mtog_s3_mfma<Real, NC>), g3, dim3(256), 0, st, g, a.n_max, s0, a.w_sum_min, a.off, a.T, a.A, a.E);
   const dim3 gs((g.D + 63) / 64, g.nwE, ns);
-  hipLaunchKernelGGL((mtog_site_G<Real, L>), gs, dim3(256), 0, st, g, s0, a.E, a.bphase, a.G0, a.kmap, a.G);
+  hipLaunchKernelGGL((mtog_site_G<Real, L>), gs, dim3(256), 0, st, g, s0, a.w_sum_min, a.E, a.bphase, a.G0, a.kmap, a.G);
 }
 
 template void launch_mtog_large<float, 36>(const MtoGArgs<float>&, int, int, hipStream_t);
