@@ -1,4 +1,4 @@
-// Device helpers shared by the single-band G4 tile kernels (g4_tiled.hip, g4_mfma.hip).
+// Device helpers of the G4 tile kernels (g4_tiled.hip, g4_band.hip).
 #ifndef G4ACC_G4_TILE_COMMON_HPP
 #define G4ACC_G4_TILE_COMMON_HPP
 

@@ -4,26 +4,37 @@
 // what the entries of one tile share. A workgroup owns the tile
 //     { (k1, w1, k2, w2, q, v) : all k1, k2;  w1, w2 fixed;  v fixed;  q in a group of QG }
 // and, per walker and spin, reads
-//   X(k1,k2)    = G[(k1, w1), (k2, w2)]                        directly (column segments)
-//   Yb(a,b)     = G[(a, w2+v), (b, w1+v)]                      into LDS: Y^q(k1,k2) = Yb(k2+q, k1+q)
-//   Zb(a,b)     = G[(a, v-w1), (b, v-w2)]                      into LDS: Z^q(k1,k2) = Zb(q-k1, q-k2)
-//   du,su(k1)   = a (u_0 -+ u_1),  u_s = G_s[(k1,w1), (k1+q, w1+v)]   precomputed (uv_kernel)
-//   dv,sv(k2)   =    v_0 -+ v_1,   v_s = G_s[(k2+q,w2+v), (k2,w2)]
-// so every G element a tile needs is fetched once per walker and reused by the QG momenta.
-//   MAGNETIC    += du dv - a (X_0 Y_0 + X_1 Y_1)
-//   CHARGE      += su sv - a (X_0 Y_0 + X_1 Y_1)
-//   PP_UP_DOWN  += a (X_0 Z_1 + X_1 Z_0)
-//   TRANSVERSE  -= a (X_0 Y_1 + X_1 Y_0)
-// Products are formed in the G precision and summed per term type over 8 walkers before they are
-// added to FP64 accumulators; G4 is read and written once per launch (FP64, or FP32 value + Kahan
-// compensation).
+//   X(k1,k2) = G[(k1, w1), (k2, w2)]            in registers: the thread's own pairs
+//   Yb(a,b)  = G[(a, w2+v), (b, w1+v)]          into LDS: Y^q(k1,k2) = Yb(k2+q, k1+q)
+//   Zb(a,b)  = G[(a, v-w1), (b, v-w2)]          into LDS: Z^q(k1,k2) = Zb(q-k1, q-k2)
+// so every G element a tile needs is fetched once per walker and reused by the QG momenta. Of the
+// walker loop's products
+//   xs = a (X_0 Y_0 + X_1 Y_1),  pz = a (X_0 Z_1 + X_1 Z_0),  tr = a (X_0 Y_1 + X_1 Y_0)
+// MAGNETIC and CHARGE share xs: MAGNETIC = R_m - xs, CHARGE = R_c - xs, PP_UP_DOWN = pz,
+// TRANSVERSE = -tr. The rank-one terms R_c(k1,k2) = sum_m U_c[m](k1) V_c[m](k2), with
+//   U = a (u_0 -+ u_1), u_s = G_s[(k1,w1), (k1+q, w1+v)],  V = v_0 -+ v_1, v_s = G_s[(k2+q,w2+v), (k2,w2)]
+// precomputed by uv_kernel, are a matrix product over the batch's walkers: each tile forms its own
+// 16 x 16 blocks of it on the matrix cores after the walker loop, so they cost no vector
+// instructions per walker and no buffer of G4's size.
+//
+// What bounds it: the blocks read from L2 and beyond (4x4, three channels, 256 walkers, 64
+// frequencies, 4 q, 3 v: 20 GB in 2.9 ms; the same block pattern alone reads 7.4 TB/s), with the
+// vector ALUs 60 % busy beside it. So each block is read once per walker for all the momenta whose
+// totals fit the registers. The next walkers' loads are in flight during a walker's products; every
+// load is issued (idle slots and walkers past the batch re-read valid elements).
+// Per batch (256 walkers) the stage went from 3.64 ms, with the rank-one terms in a buffer of G4's
+// size, to 3.0 ms; 6x6 (64 walkers, 64 frequencies, 4 q, 2 v) from 10.6 to 4.8 ms.
+// Products are formed in the G precision; with complex64 G, 256-thread tiles sum eight walkers in
+// FP32 before the FP64 totals, larger tiles (whose registers hold the totals) add every walker.
+// G4 is read and written once per launch (FP64, or FP32 value + Kahan compensation).
 #include <algorithm>
 #include <type_traits>
-#include <utility>
 
 #include "g4_tile_common.hpp"
 
 namespace g4acc {
+
+namespace {
 
 // Two values read together from LDS (one 16-byte read for complex64).
 template <typename C>
@@ -43,6 +54,57 @@ __device__ __forceinline__ void store_pair(CPair<C>& dst, C a, C b) {
     dst.b = b;
   }
 }
+
+typedef float pair_f32x4 __attribute__((ext_vector_type(4)));
+typedef double pair_f64x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ pair_f32x4 mma4(float a, float b, pair_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ pair_f64x4 mma4(double a, double b, pair_f64x4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Terms formed by the walker loop.
+constexpr int HAS_X = 1, HAS_Z = 2, HAS_T = 4;
+
+// Registers of a workgroup's threads. 704 threads hold 33..37-site clusters with two pairs each:
+// eleven waves leave 168 registers, enough for the totals of four momenta (6x6, magnetic and pp, 64
+// walkers, 64 frequencies: 4.8 ms per batch; two momenta 6.2, two in 1024 threads 7.6, since each
+// group of momenta reads the blocks again).
+template <typename Real, int TT, int PPT, int QG>
+struct PairShape {
+  static constexpr bool fp32 = sizeof(Real) == 4;
+  static constexpr int DEPTH = fp32 && TT == 1024 && PPT * QG <= 2 ? 2 : 1;  // walkers in flight
+  static constexpr int FLUSH = fp32 && TT == 256 ? 8 : 1;
+  static constexpr int WAVES = TT == 704 ? 3 : 4;  // per SIMD: 168 or 128 registers
+  // The compiler sinks the loads to their use, behind the products they are to overlap; kept in
+  // place they must fit beside everything else, which complex128 G in large tiles does not.
+  static constexpr bool HOLD = fp32 || TT == 256;
+};
+
+// G4[i] += v in two steps, so that a thread's loads are all issued before its stores.
+__device__ __forceinline__ void g4_put(void* g4, size_t i, float4 old, double2 acc, int sum_mode) {
+  if (sum_mode == SUM_FP64) {
+    double2 v = *reinterpret_cast<double2*>(&old);
+    v.x += acc.x;
+    v.y += acc.y;
+    static_cast<double2*>(g4)[i] = v;
+  }
+  else {
+    float4 v = old;
+    const float hx = static_cast<float>(acc.x), hy = static_cast<float>(acc.y);
+    const float lx = static_cast<float>(acc.x - hx), ly = static_cast<float>(acc.y - hy);
+    const float yx = hx - v.z, yy = hy - v.w;
+    const float tx = v.x + yx, ty = v.y + yy;
+    v.z = ((tx - v.x) - yx) - lx;
+    v.w = ((ty - v.y) - yy) - ly;
+    v.x = tx;
+    v.y = ty;
+    static_cast<float4*>(g4)[i] = v;
+  }
+}
+
+}  // namespace
 
 // UV[((m * 4 + plane) * nqv + qv) * P + p], planes: a(u0-u1), a(u0+u1), v0-v1, v0+v1.
 template <typename Real>
@@ -73,14 +135,14 @@ __global__ void __launch_bounds__(256) uv_kernel(TiledArgs<Real> a) {
   out[3 * plane] = C{v0.x + v1.x, v0.y + v1.y};
 }
 
-// MASK: compile-time channel set (bit 1 << type), or 0 to read the channel flags at run time.
-// RX: the rank-one terms of MAGNETIC and CHARGE come precomputed for the batch (a.R, g4_rank1.hip)
-// and are added at the G4 store; the kernel then stages no factors and forms no rank-one products.
-template <typename Real, int TT, int PPT, int QG, int NCH, int MASK, bool RX>
-__global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
+template <typename Real, int TT, int PPT, int QG, int SET>
+__global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_pair_kernel(TiledArgs<Real> a) {
   using C = Cplx<Real>;
+  using P2 = CPair<C>;
+  using Shape = PairShape<Real, TT, PPT, QG>;
+  constexpr bool HX = (SET & HAS_X) != 0, HZ = (SET & HAS_Z) != 0, HT = (SET & HAS_T) != 0, HY = HX || HT;
+  constexpr int DEPTH = Shape::DEPTH, FLUSH = Shape::FLUSH;
   extern __shared__ unsigned char smem_raw[];
-  C* lds = reinterpret_cast<C*>(smem_raw);
   const Geo& g = a.g;
   const int nc = g.nc, nw = g.nw, e = g.ext, P = nc * nw;
   const size_t D = g.D, DD = D * D;
@@ -89,16 +151,9 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
     return;
   const int iv = z / a.nqg, q0 = (z % a.nqg) * QG;
   const int nu = a.w_ex[iv];
-  const int ld = nc + 1, bs = nc * ld;
-  constexpr bool kStatic = MASK != 0;
-  constexpr int kY = (1 << PH_MAGNETIC) | (1 << PH_CHARGE) | (1 << 1);
-  const bool needY = kStatic ? (MASK & kY) != 0 : a.need_y;
-  const bool needZ = kStatic ? (MASK & (1 << PP_UP_DOWN)) != 0 : a.need_z;
-  // Both spins of a staged element side by side, and the two factors a thread reads together.
-  using P2 = CPair<C>;
-  P2* Yl = reinterpret_cast<P2*>(lds);  // [b][a] (a fastest): {spin 0, spin 1}
-  P2* Zl = Yl + (needY ? bs : 0);
-  P2* Ul = Zl + (needZ ? bs : 0);       // [side][qi][k]: side 0 {a(u0-u1), a(u0+u1)}, 1 {v0-v1, v0+v1}
+  const int ld = nc + 1, bs = nc * ld, ncc = nc * nc;
+  P2* Yl = reinterpret_cast<P2*>(smem_raw);  // [b][a] (a fastest): {spin 0, spin 1}
+  P2* Zl = Yl + (HY ? bs : 0);
   // Blocks (wa, wb) of G (extended frequencies). Of a conjugate symmetric G only the half
   // wa + wb >= nwE - 1 is read: another block is the conjugate of (-wa, -wb) at (-ka, -kb); its sign
   // is applied where the block is staged (Y, Z) or scaled by alpha (X).
@@ -109,531 +164,434 @@ __global__ void __launch_bounds__(TT) g4_tiled_kernel(TiledArgs<Real> a) {
   };
   const int wy = nu + e, wz = nu + nw - 1 + e;
   const bool xm = mirrored(w1 + e, w2 + e), ym = mirrored(w2 + wy, w1 + wy), zm = mirrored(wz - w1, wz - w2);
-  const size_t xoff = block(w1 + e, w2 + e), yoff = block(w2 + wy, w1 + wy), zoff = block(wz - w1, wz - w2);
+  // Wave-uniform block bases and, per thread, element offsets within a block (below nc D < 2^32).
+  const C* Xg = a.G + block(w1 + e, w2 + e);
+  const C* Yg = a.G + block(w2 + wy, w1 + wy);
+  const C* Zg = a.G + block(wz - w1, wz - w2);
   const Real xs_im = xm ? -1 : 1, ys_im = ym ? -1 : 1, zs_im = zm ? -1 : 1;
   auto element = [&](int ka, int kb, bool m) {
-    return (m ? a.k_neg[ka] : ka) + D * (m ? a.k_neg[kb] : kb);
+    return static_cast<unsigned>(m ? a.k_neg[ka] : ka) + static_cast<unsigned>(D) * static_cast<unsigned>(m ? a.k_neg[kb] : kb);
   };
-  const int nqv = g.nq * g.nv;
 
-  int k1[PPT], k2[PPT];
-  int yi[PPT][QG], zi[PPT][QG];
+  // The thread's pairs: element j is idx = tid + TT j of the block, (k1, k2) = (idx % nc, idx / nc)
+  // (pair 0 for idle ones). It loads X, Y and Z at the same idx.
   bool ok[PPT];
-  int qv[QG];
-  bool qok[QG];
-#pragma unroll
-  for (int qi = 0; qi < QG; ++qi) {
-    qok[qi] = q0 + qi < g.nq;
-    qv[qi] = (qok[qi] ? q0 + qi : 0) + g.nq * iv;
-  }
-#pragma unroll
-  for (int j = 0; j < PPT; ++j) {
-    const int pi = threadIdx.x + TT * j;
-    ok[j] = pi < nc * nc;
-    k1[j] = ok[j] ? pi % nc : 0;
-    k2[j] = ok[j] ? pi / nc : 0;
-#pragma unroll
-    for (int qi = 0; qi < QG; ++qi) {
-      const int q = a.k_ex[qok[qi] ? q0 + qi : 0];
-      yi[j][qi] = a.k_add[k1[j] + nc * q] * ld + a.k_add[k2[j] + nc * q];
-      zi[j][qi] = a.k_sub[k2[j] + nc * q] * ld + a.k_sub[k1[j] + nc * q];
-    }
-  }
-  // The rank-one factors: one staged element per thread (4 QG nc <= 256).
-  const int n_uv = 4 * QG * nc;
-  const int u_plane = threadIdx.x / (QG * nc), u_qi = (threadIdx.x / nc) % QG, u_k = threadIdx.x % nc;
-  const bool u_ok = threadIdx.x < n_uv;
-  const int u_dst = 2 * (((u_plane >> 1) * QG + u_qi) * nc + u_k) + (u_plane & 1);
-  const size_t plane = static_cast<size_t>(nqv) * P;
-  const size_t u_src = u_plane * plane + static_cast<size_t>(qv[0] + u_qi) * P + u_k +
-                       static_cast<size_t>(nc) * (u_plane < 2 ? w1 : w2);
-  const bool u_valid = !RX && u_ok && (q0 + u_qi < g.nq);
-
-  // Channel outputs are FP64 totals. With complex64 G the walker terms are first summed in FP32
-  // per term type for FLUSH walkers (relative rounding ~2^-24 per step), so the per-walker work
-  // is fused multiply-adds only:
-  //   xs = a(X0 Y0 + X1 Y1), pz = a(X0 Z1 + X1 Z0), tr = a(X0 Y1 + X1 Y0), dm = du dv, dc = su sv
-  //   MAGNETIC = dm - xs, CHARGE = dc - xs, PP = pz, TRANSVERSE = -tr,
-  // and the FP64 additions happen once per FLUSH walkers. With complex128 G every walker's
-  // channel term goes straight into the totals.
-  // 1024-thread tiles of two pairs per thread with precomputed rank-one terms (6x6 batches) run a
-  // two-walker pipeline (below): each walker's terms go straight into the FP64 totals, whose
-  // registers would otherwise hold FP32 partials.
-  constexpr bool kPipe = RX && TT == 1024 && PPT == 2;
-  // 1024-thread tiles of four pairs per thread (8x8) with complex64 G: every prefetch load is
-  // issued (clamped indices and walker) and the thread's X entries of the current walker are
-  // loaded before the next walker's prefetch, so the products wait for X only. Each walker's
-  // terms go straight into the FP64 totals, whose registers would otherwise hold FP32 partials.
-  constexpr bool kXFirst = !RX && TT == 1024 && PPT == 4 && sizeof(Real) == 4;
-  constexpr bool kChunk = sizeof(Real) == 4 && !kPipe && !kXFirst;
-  constexpr int FLUSH = 8;
-  constexpr int PC = kChunk ? PPT : 1, QC = kChunk ? QG : 1;
-  // Registers: with many pairs per thread (or 1024-thread workgroups, 128 VGPRs) X is read in place.
-  constexpr bool kPrefetchX = PPT * (TT / 256) <= 4 && !(TT > 256 && PPT > 1);
-  bool has_trans = a.has_trans, has_mag = false, has_chg = false;
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    has_mag |= a.ch[c] == PH_MAGNETIC;
-    has_chg |= a.ch[c] == PH_CHARGE;
-  }
-  if constexpr (kStatic) {
-    has_trans = (MASK & (1 << 1)) != 0;
-    has_mag = (MASK & (1 << PH_MAGNETIC)) != 0;
-    has_chg = (MASK & (1 << PH_CHARGE)) != 0;
-  }
-  double2 tot[PPT][QG][NCH];
-  C xs[PC][QC], pz[PC][QC], tr[PC][QC], dm[PC][QC], dc[PC][QC];
-#pragma unroll
-  for (int j = 0; j < PPT; ++j)
-#pragma unroll
-    for (int qi = 0; qi < QG; ++qi)
-#pragma unroll
-      for (int c = 0; c < NCH; ++c)
-        tot[j][qi][c] = double2{0, 0};
-#pragma unroll
-  for (int j = 0; j < PC; ++j)
-#pragma unroll
-    for (int qi = 0; qi < QC; ++qi)
-      xs[j][qi] = pz[j][qi] = tr[j][qi] = dm[j][qi] = dc[j][qi] = C{0, 0};
-  if constexpr (kPipe) {
-    // X, Y and Z (both spins) of walkers m + 1 and m + 2 are in flight while walker m is consumed.
-    // The elements a walker stages form one flat list, PS per thread, each stored with both spins
-    // in one 16-byte write; their source offsets (within the walker's G, below 2^31) and LDS
-    // places are fixed for the tile. Every load is issued (idle slots re-read element 0, walkers
-    // past the batch re-read the last one) and the loop is unrolled by two, so the loads in
-    // flight are counted exactly and staging waits only for the walker it writes.
-    constexpr int PS = 4;  // 3 nc^2 <= PS TT (the launcher takes this path for Nc <= 36 only)
-    constexpr int NBK = 1 + ((MASK & kY) != 0) + ((MASK & (1 << PP_UP_DOWN)) != 0);
-    P2* Xl = Yl + (NBK - 1) * bs;  // after Y and Z
-    const int ncc = nc * nc, n_items = NBK * ncc, n_walk = a.n_walkers;
-    int psrc[PS], pdst[PS];
-    bool puse[PS];
-    Real pim[PS];  // sign of the imaginary part
-#pragma unroll
-    for (int j = 0; j < PS; ++j) {
-      const int f = threadIdx.x + TT * j;
-      puse[j] = f < n_items;
-      const int blk = puse[j] ? f / ncc : 0, idx = f % ncc;
-      // Blocks in LDS order: Y (if staged), Z (if staged), X.
-      const bool isx = blk == NBK - 1, isy = !isx && needY && blk == 0;
-      const size_t boff = isx ? xoff : (isy ? yoff : zoff);
-      psrc[j] = puse[j] ? static_cast<int>(boff + element(idx % nc, idx / nc, isx ? xm : (isy ? ym : zm))) : 0;
-      pim[j] = isx ? xs_im : (isy ? ys_im : zs_im);
-      pdst[j] = blk * bs + (idx / nc) * ld + idx % nc;
-    }
-    C pre[2][PS][2];
-    auto fetch = [&](int m, C (&pr)[PS][2]) {
-      const C* H = a.G + (2 * static_cast<size_t>(m < n_walk ? m : n_walk - 1)) * DD;
-#pragma unroll
-      for (int j = 0; j < PS; ++j) {
-        pr[j][0] = H[psrc[j]];
-        pr[j][1] = H[DD + psrc[j]];
-      }
-    };
-    auto stage = [&](const C (&cur)[PS][2]) {
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < PS; ++j)
-        if (puse[j])
-          store_pair(Yl[pdst[j]], C{cur[j][0].x, cur[j][0].y * pim[j]}, C{cur[j][1].x, cur[j][1].y * pim[j]});
-      __syncthreads();
-    };
-    auto consume = [&](int m) {
-      const Real alpha = static_cast<Real>(0.5 * a.desc[2 * m].sign);
-#pragma unroll
-      for (int j = 0; j < PPT; ++j) {
-        if (!ok[j])
-          continue;
-        const P2 xx = Xl[k2[j] * ld + k1[j]];
-        const C x0{alpha * xx.a.x, alpha * xx.a.y}, x1{alpha * xx.b.x, alpha * xx.b.y};
-#pragma unroll
-        for (int qi = 0; qi < QG; ++qi) {
-          if (!qok[qi])
-            continue;
-          C cross{0, 0}, ppz{0, 0};
-          if (needY) {
-            const P2 yy = Yl[yi[j][qi]];
-            cross = cmul(x0, yy.a);
-            cfma(cross, x1, yy.b);
-          }
-          if (needZ) {
-            const P2 zz = Zl[zi[j][qi]];
-            ppz = cmul(x0, zz.b);
-            cfma(ppz, x1, zz.a);
-          }
-#pragma unroll
-          for (int c = 0; c < NCH; ++c) {
-            const int ch = a.ch[c];
-            const C t = ch == PP_UP_DOWN ? ppz : C{-cross.x, -cross.y};
-            tot[j][qi][c].x += static_cast<double>(t.x);
-            tot[j][qi][c].y += static_cast<double>(t.y);
-          }
-        }
-      }
-    };
-    if (n_walk > 0) {
-      fetch(0, pre[0]);
-      fetch(1, pre[1]);
-      for (int m = 0; m < n_walk; m += 2) {
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          stage(pre[d]);
-          fetch(m + d + 2, pre[d]);
-          if (m + d < n_walk)
-            consume(m + d);
-        }
-      }
-    }
-  }
-  else {
-  // Everything walker m needs is loaded into registers while walker m - 1 is consumed: the
-  // staged blocks (each thread stages at most PPT elements per block, nc^2 <= 256 PPT), the
-  // rank-one factors and (for few pairs per thread) the thread's own X entries.
-  C pre[4][PPT], pre_uv, pre_x[2][kPrefetchX ? PPT : 1];
-  size_t ysrc[PPT], zsrc[PPT], xsrc[PPT];  // this thread's elements of the three blocks
+  unsigned xo[PPT], yo[PPT], zo[PPT];
+  int li[PPT];
+  int yz[PPT][QG];  // LDS places of Y^q and Z^q, 16 bits each (bs <= 64 * 65)
 #pragma unroll
   for (int j = 0; j < PPT; ++j) {
     const int idx = threadIdx.x + TT * j;
-    const int idc = idx < nc * nc ? idx : 0;
-    ysrc[j] = yoff + element(idc % nc, idc / nc, ym);
-    zsrc[j] = zoff + element(idc % nc, idc / nc, zm);
-    xsrc[j] = xoff + element(k1[j], k2[j], xm);  // pair 0 for idle pairs
-  }
-  auto prefetch = [&](int m) {
-    if constexpr (kXFirst) {
-      const int mc = m < a.n_walkers ? m : a.n_walkers - 1;
-      const C* H0 = a.G + (2 * static_cast<size_t>(mc)) * DD;
-      const C* H1 = H0 + DD;
-#pragma unroll
-      for (int j = 0; j < PPT; ++j) {
-        if (needY) {
-          pre[0][j] = H0[ysrc[j]];
-          pre[1][j] = H1[ysrc[j]];
-        }
-        if (needZ) {
-          pre[2][j] = H0[zsrc[j]];
-          pre[3][j] = H1[zsrc[j]];
-        }
-      }
-      pre_uv = a.UV[static_cast<size_t>(mc) * 4 * plane + (u_valid ? u_src : 0)];
-      return;
-    }
-    const C* H0 = a.G + (2 * static_cast<size_t>(m)) * DD;
-    const C* H1 = H0 + DD;
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-      const int idx = threadIdx.x + TT * j;
-      if (idx < nc * nc) {
-        if (needY) {
-          pre[0][j] = H0[ysrc[j]];
-          pre[1][j] = H1[ysrc[j]];
-        }
-        if (needZ) {
-          pre[2][j] = H0[zsrc[j]];
-          pre[3][j] = H1[zsrc[j]];
-        }
-      }
-      if constexpr (kPrefetchX) {
-        if (ok[j]) {
-          pre_x[0][j] = H0[xsrc[j]];
-          pre_x[1][j] = H1[xsrc[j]];
-        }
-      }
-    }
-    if (u_valid)
-      pre_uv = a.UV[static_cast<size_t>(m) * 4 * plane + u_src];
-  };
-  if (a.n_walkers > 0)
-    prefetch(0);
-  for (int m = 0; m < a.n_walkers; ++m) {
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-      const int idx = threadIdx.x + TT * j;
-      if (idx < nc * nc) {
-        const int li = (idx / nc) * ld + (idx % nc);
-        if (needY)
-          store_pair(Yl[li], C{pre[0][j].x, pre[0][j].y * ys_im}, C{pre[1][j].x, pre[1][j].y * ys_im});
-        if (needZ)
-          store_pair(Zl[li], C{pre[2][j].x, pre[2][j].y * zs_im}, C{pre[3][j].x, pre[3][j].y * zs_im});
-      }
-    }
-    if (u_valid)
-      reinterpret_cast<C*>(Ul)[u_dst] = pre_uv;
-    C xw[2][kPrefetchX ? PPT : 1];
-    if constexpr (kPrefetchX) {
-#pragma unroll
-      for (int j = 0; j < PPT; ++j) {
-        xw[0][j] = pre_x[0][j];
-        xw[1][j] = pre_x[1][j];
-      }
-    }
-    __syncthreads();
-    const Real alpha = static_cast<Real>(0.5 * a.desc[2 * m].sign);
-    const C* G0m = a.G + (2 * static_cast<size_t>(m)) * DD;
-    C xr[kXFirst ? PPT : 1][2];
-    if constexpr (kXFirst) {
-#pragma unroll
-      for (int j = 0; j < PPT; ++j) {
-        xr[j][0] = G0m[xsrc[j]];
-        xr[j][1] = G0m[DD + xsrc[j]];
-      }
-      prefetch(m + 1);
-    }
-    else if (m + 1 < a.n_walkers) {
-      prefetch(m + 1);
-    }
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-      if (!ok[j])
-        continue;
-      C x0, x1;
-      if constexpr (kXFirst) {
-        x0 = xr[j][0];
-        x1 = xr[j][1];
-      }
-      else if constexpr (kPrefetchX) {
-        x0 = xw[0][j];
-        x1 = xw[1][j];
-      }
-      else {
-        x0 = G0m[xsrc[j]];
-        x1 = G0m[DD + xsrc[j]];
-      }
-      x0.x *= alpha;
-      x0.y *= alpha * xs_im;
-      x1.x *= alpha;
-      x1.y *= alpha * xs_im;
-#pragma unroll
-      for (int qi = 0; qi < QG; ++qi) {
-        if (!qok[qi])
-          continue;
-        const P2* uq = Ul + qi * nc;
-        if constexpr (kChunk) {
-          const int jj = kChunk ? j : 0, qq = kChunk ? qi : 0;
-          if (needY) {
-            const P2 yy = Yl[yi[j][qi]];
-            const C y0 = yy.a, y1 = yy.b;
-            cfma(xs[jj][qq], x0, y0);
-            cfma(xs[jj][qq], x1, y1);
-            if (has_trans) {
-              cfma(tr[jj][qq], x0, y1);
-              cfma(tr[jj][qq], x1, y0);
-            }
-          }
-          if (needZ) {
-            const P2 zz = Zl[zi[j][qi]];
-            cfma(pz[jj][qq], x0, zz.b);
-            cfma(pz[jj][qq], x1, zz.a);
-          }
-          if (!RX && (has_mag || has_chg)) {
-            const P2 uu = uq[k1[j]], vv = uq[QG * nc + k2[j]];
-            if (has_mag)
-              cfma(dm[jj][qq], uu.a, vv.a);
-            if (has_chg)
-              cfma(dc[jj][qq], uu.b, vv.b);
-          }
-        }
-        else {
-          C cross{0, 0}, ppz{0, 0}, trans{0, 0};
-          if (needY) {
-            const C y0 = Yl[yi[j][qi]].a, y1 = Yl[yi[j][qi]].b;  // members: no 32-byte temporary
-            cross = cmul(x0, y0);
-            cfma(cross, x1, y1);
-            if (has_trans) {
-              trans = cmul(x0, y1);
-              cfma(trans, x1, y0);
-            }
-          }
-          if (needZ) {
-            ppz = cmul(x0, Zl[zi[j][qi]].b);
-            cfma(ppz, x1, Zl[zi[j][qi]].a);
-          }
-#pragma unroll
-          for (int c = 0; c < NCH; ++c) {
-            const int ch = a.ch[c];
-            C t;
-            if (ch == PH_MAGNETIC) {
-              t = csub(C{0, 0}, cross);
-              if (!RX)
-                cfma(t, uq[k1[j]].a, uq[QG * nc + k2[j]].a);
-            }
-            else if (ch == PH_CHARGE) {
-              t = csub(C{0, 0}, cross);
-              if (!RX)
-                cfma(t, uq[k1[j]].b, uq[QG * nc + k2[j]].b);
-            }
-            else if (ch == PP_UP_DOWN)
-              t = ppz;
-            else
-              t = C{-trans.x, -trans.y};
-            tot[j][qi][c].x += static_cast<double>(t.x);
-            tot[j][qi][c].y += static_cast<double>(t.y);
-          }
-        }
-      }
-    }
-    if constexpr (kChunk) {
-      if ((m + 1) % FLUSH == 0 || m + 1 == a.n_walkers) {
-#pragma unroll
-        for (int j = 0; j < PC; ++j)
-#pragma unroll
-          for (int qi = 0; qi < QC; ++qi) {
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-              const int ch = a.ch[c];
-              C t;
-              if (ch == PH_MAGNETIC)
-                t = csub(dm[j][qi], xs[j][qi]);
-              else if (ch == PH_CHARGE)
-                t = csub(dc[j][qi], xs[j][qi]);
-              else if (ch == PP_UP_DOWN)
-                t = pz[j][qi];
-              else
-                t = C{-tr[j][qi].x, -tr[j][qi].y};
-              tot[j][qi][c].x += static_cast<double>(t.x);
-              tot[j][qi][c].y += static_cast<double>(t.y);
-            }
-            xs[j][qi] = pz[j][qi] = tr[j][qi] = dm[j][qi] = dc[j][qi] = C{0, 0};
-          }
-      }
-    }
-  }
-  }
-  auto store = [&](int c, size_t idx, double2 v) {
-    if constexpr (RX) {
-      if (a.r1_slot[c] >= 0) {
-        const size_t plane = static_cast<size_t>(nqv) * P * P;
-        const float2 r = static_cast<const float2*>(a.R)[a.r1_slot[c] * plane + idx];
-        v.x += static_cast<double>(r.x);
-        v.y += static_cast<double>(r.y);
-      }
-    }
-    g4_store_t(a.g4[c], idx, v, a.sum_mode);
-  };
-  auto g4_index = [&](int ka, int wa, int kb, int wb, int qvi) {
-    return ka + static_cast<size_t>(nc) *
-                    (wa + static_cast<size_t>(nw) * (kb + static_cast<size_t>(nc) * (wb + static_cast<size_t>(nw) * qvi)));
-  };
-#pragma unroll
-  for (int j = 0; j < PPT; ++j) {
-    if (!ok[j])
-      continue;
+    ok[j] = idx < ncc;
+    const int k1 = ok[j] ? idx % nc : 0, k2 = ok[j] ? idx / nc : 0;
+    xo[j] = element(k1, k2, xm);
+    yo[j] = element(k1, k2, ym);
+    zo[j] = element(k1, k2, zm);
+    li[j] = k2 * ld + k1;
 #pragma unroll
     for (int qi = 0; qi < QG; ++qi) {
-      if (!qok[qi])
-        continue;
-      const size_t idx = g4_index(k1[j], w1, k2[j], w2, qv[qi]);
-#pragma unroll
-      for (int c = 0; c < NCH; ++c)
-        store(c, idx, tot[j][qi][c]);
+      const int q = a.k_ex[q0 + qi < g.nq ? q0 + qi : 0];
+      yz[j][qi] = (a.k_add[k1 + nc * q] * ld + a.k_add[k2 + nc * q]) |
+                  ((a.k_sub[k2 + nc * q] * ld + a.k_sub[k1 + nc * q]) << 16);
     }
   }
-  if (a.sym == SYM_NONE)
-    return;
-  // Images of the tile (G4Sym) that no workgroup computes. P keeps the order of k1 up to a
-  // permutation of its Nc entries and is stored directly; T, C and both together (v = 0) go through
-  // LDS (the staging area is free now), so that the stores run along k1 of the image. Thread
-  // (k1, k2) of an image takes the tile's pair (src1, src2) below.
-  const bool ht = a.need_y, hp = a.need_z;
+
+  double2 tx[PPT][QG], tz[PPT][QG], tt[PPT][QG];  // FP64 totals
+  C fx[PPT][QG], fz[PPT][QG], ft[PPT][QG];         // partial sums (FLUSH > 1)
+#pragma unroll
+  for (int j = 0; j < PPT; ++j)
+#pragma unroll
+    for (int qi = 0; qi < QG; ++qi) {
+      tx[j][qi] = tz[j][qi] = tt[j][qi] = double2{0, 0};
+      fx[j][qi] = fz[j][qi] = ft[j][qi] = C{0, 0};
+    }
+  const int n_walk = a.n_walkers;
+  C px[DEPTH][PPT][2], py[DEPTH][PPT][2], pz[DEPTH][PPT][2];
+  double sign[DEPTH];
+  auto fetch = [&](int m, int d) {
+    const int mc = m < n_walk ? m : n_walk - 1;
+    const size_t mo = 2 * static_cast<size_t>(mc) * DD;
+    sign[d] = a.desc[2 * mc].sign;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const C* X = Xg + mo + s * DD;
+      const C* Y = Yg + mo + s * DD;
+      const C* Z = Zg + mo + s * DD;
+#pragma unroll
+      for (int j = 0; j < PPT; ++j) {
+        if (HY)
+          py[d][j][s] = Y[yo[j]];
+        if (HZ)
+          pz[d][j][s] = Z[zo[j]];
+      }
+#pragma unroll
+      for (int j = 0; j < PPT; ++j)
+        px[d][j][s] = X[xo[j]];
+    }
+  };
+  auto flush = [&]() {
+#pragma unroll
+    for (int j = 0; j < PPT; ++j)
+#pragma unroll
+      for (int qi = 0; qi < QG; ++qi) {
+        if (HX)
+          tx[j][qi] = double2{tx[j][qi].x + static_cast<double>(fx[j][qi].x), tx[j][qi].y + static_cast<double>(fx[j][qi].y)};
+        if (HZ)
+          tz[j][qi] = double2{tz[j][qi].x + static_cast<double>(fz[j][qi].x), tz[j][qi].y + static_cast<double>(fz[j][qi].y)};
+        if (HT)
+          tt[j][qi] = double2{tt[j][qi].x + static_cast<double>(ft[j][qi].x), tt[j][qi].y + static_cast<double>(ft[j][qi].y)};
+        fx[j][qi] = fz[j][qi] = ft[j][qi] = C{0, 0};
+      }
+  };
+  auto walker = [&](int m, int d) {
+    __syncthreads();  // the previous walker's blocks have been read
+#pragma unroll
+    for (int j = 0; j < PPT; ++j)
+      if (ok[j]) {
+        if (HY)
+          store_pair(Yl[li[j]], C{py[d][j][0].x, py[d][j][0].y * ys_im}, C{py[d][j][1].x, py[d][j][1].y * ys_im});
+        if (HZ)
+          store_pair(Zl[li[j]], C{pz[d][j][0].x, pz[d][j][0].y * zs_im}, C{pz[d][j][1].x, pz[d][j][1].y * zs_im});
+      }
+    const Real al = static_cast<Real>(0.5 * sign[d]), ali = al * xs_im;
+    C x0[PPT], x1[PPT];
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+      x0[j] = C{al * px[d][j][0].x, ali * px[d][j][0].y};
+      x1[j] = C{al * px[d][j][1].x, ali * px[d][j][1].y};
+    }
+    __syncthreads();
+    fetch(m + DEPTH, d);
+    if constexpr (Shape::HOLD)
+      asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+#pragma unroll
+      for (int qi = 0; qi < QG; ++qi) {
+        if (HY) {
+          const P2& yy = Yl[yz[j][qi] & 0xffff];
+          const C y0 = yy.a, y1 = yy.b;
+          if (HX) {
+            cfma(fx[j][qi], x0[j], y0);
+            cfma(fx[j][qi], x1[j], y1);
+          }
+          if (HT) {
+            cfma(ft[j][qi], x0[j], y1);
+            cfma(ft[j][qi], x1[j], y0);
+          }
+        }
+        if (HZ) {
+          const P2& zz = Zl[static_cast<unsigned>(yz[j][qi]) >> 16];
+          const C z0 = zz.a, z1 = zz.b;
+          cfma(fz[j][qi], x0[j], z1);
+          cfma(fz[j][qi], x1[j], z0);
+        }
+      }
+    }
+    if (FLUSH == 1 || (m + 1) % FLUSH == 0)
+      flush();
+  };
+  if (n_walk > 0) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      fetch(d, d);
+    int m = 0;
+    for (; m + DEPTH <= n_walk; m += DEPTH)
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d)
+        walker(m + d, d);
+    if constexpr (DEPTH > 1)
+      if (m < n_walk)
+        walker(m, 0);
+    if (FLUSH > 1)
+      flush();
+  }
+
+  // Rank-one terms, totals and G4, for RB momenta at a time: rank-one blocks of both channels into
+  // LDS, then each thread's channel totals, its G4 entries and the images (G4Sym) that no workgroup
+  // computes. P keeps the order of k1 up to a permutation of its Nc entries and is stored directly;
+  // T, C and both together (v = 0) go through LDS, so that the stores run along k1 of the image:
+  // thread (k1, k2) of an image takes the tile's pair below.
+  // LDS holds the particle-hole channels of those momenta together, or one channel at a time where a
+  // plane is large (PPT = 4: up to 66.5 KB).
+  constexpr int RB = TT == 256 && PPT == 1 ? QG : 1;
+  constexpr bool kOneCh = PPT == 4;
   auto left_out = [&](int wa, int wb) {
-    return wa >= 0 && wa < nw && wb >= 0 && wb < nw && !sym_tile_computed(nw, nu, wa, wb, ht, hp, a.sym);
+    return wa >= 0 && wa < nw && wb >= 0 && wb < nw && !sym_tile_computed(nw, nu, wa, wb, HY, HZ, a.sym);
   };
   const int c1 = nw - 1 - nu - w2, c2 = nw - 1 - nu - w1;  // C
   const int p1 = nw - 1 + nu - w1, p2 = nw - 1 + nu - w2;  // P
   const bool img_t = (a.sym & 1) && w1 != w2;
   const bool img_c = a.sym == SYM_CONJ ? left_out(c1, c2) : a.sym == SYM_CONJ_TRANSPOSE && w1 + w2 != nw - 1;
-  const bool img_p = a.sym == SYM_CONJ && left_out(p1, p2);
-  double2* tl = reinterpret_cast<double2*>(lds);
+  const bool img_p = HZ && a.sym == SYM_CONJ && left_out(p1, p2);
+  double2* Rl = reinterpret_cast<double2*>(smem_raw);  // [momentum][particle-hole channel][k2][k1]
+  auto g4_index = [&](int ka, int wa, int kb, int wb, int qv) {
+    return ka + static_cast<size_t>(nc) *
+                    (wa + static_cast<size_t>(nw) * (kb + static_cast<size_t>(nc) * (wb + static_cast<size_t>(nw) * qv)));
+  };
+  // Index arithmetic below starts from an opaque copy of the thread id per group of entries: held
+  // for all pairs at once it would not fit beside the totals.
+  auto own_index = [&](int tid, int j, int qv) {
+    const int idx = tid + TT * j;
+    return g4_index(idx % nc, w1, idx / nc, w2, qv);
+  };
+  auto swap_index = [&](int tid, int j, int qv, int q) {
+    const int idx = tid + TT * j;
+    return g4_index(a.k_sub[idx % nc + nc * q], p1, a.k_sub[idx / nc + nc * q], p2, qv);
+  };
+  // Below four walkers a matrix-core step would be mostly padding, and the launch is the G4
+  // read-modify-write: each thread forms its entries' rank-one terms itself (to its own LDS places,
+  // ahead of the G4 loads and stores).
+  const bool direct = n_walk < 4;
+  const size_t uv_row = static_cast<size_t>(g.nq) * g.nv * P;  // between the planes of one walker
+  auto rank_one = [&](int j, int qv, int pl) {
+    const int idx = threadIdx.x + TT * j;
+    const C* U = a.UV + pl * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w1) + idx % nc;
+    const C* V = a.UV + (pl + 2) * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w2) + idx / nc;
+    double2 r{0, 0};
+    for (int m = 0; m < n_walk; ++m)
+      cfma(r, to_d(V[4 * uv_row * m]), to_d(U[4 * uv_row * m]));
+    return r;
+  };
+  constexpr int GS = RB * PPT >= 4 ? 4 : RB * PPT >= 2 ? 2 : 1;  // G4 entries per channel in flight
+  // Channels whose entries are in flight together (one where four groups of momenta are unrolled: the
+  // loop over them must unroll for the totals to stay in registers).
+  constexpr int CG = kOneCh || QG / RB > 2 ? 1 : 3;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-  for (int qi = 0; qi < QG; ++qi) {
-    if (!qok[qi])
+  for (int r0 = 0; r0 < QG; r0 += RB) {
+    if (q0 + r0 >= g.nq)
+      break;
+    const int nr = min(RB, g.nq - q0 - r0);
+    for (int c_lo = 0; c_lo < a.n_ch; c_lo += kOneCh ? 1 : a.n_ch) {
+    const int c_hi = kOneCh ? c_lo + 1 : a.n_ch;
+    int n_ph = 0, n_r = 0;  // particle-hole channels, and those of them with a rank-one term
+    for (int c = c_lo; c < c_hi; ++c) {
+      n_ph += a.ch[c] != PP_UP_DOWN;
+      n_r += a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE;
+    }
+    __syncthreads();
+    if (HX && n_r > 0 && direct) {
+      int ph = 0;
+      for (int c = c_lo; c < c_hi; ph += a.ch[c] != PP_UP_DOWN, ++c)
+        if (a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE)
+#pragma unroll
+          for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int j = 0; j < PPT; ++j)
+              if (r < nr && ok[j])
+                Rl[(r * n_ph + ph) * bs + li[j]] =
+                    rank_one(j, q0 + r0 + r + g.nq * iv, a.ch[c] == PH_MAGNETIC ? 0 : 1);
+    }
+    else if (HX && n_r > 0) {
+      // R(k2, k1) blocks of 16 x 16: lane l supplies V[m0 + l/16][k2] and U[m0 + l/16][k1] and holds
+      // rows k2 = 4 (l/16) + i (FP32) or l/16 + 4 i (FP64) of column k1 = l % 16.
+      // complex64 G: 256-thread tiles add eight walkers' FP32 products to FP64 sums, as their walker
+      // loop does; larger tiles, whose walker loop adds every walker, multiply in FP64.
+      constexpr bool kR32 = Shape::fp32 && TT == 256;
+      using RT = std::conditional_t<kR32, float, double>;
+      using V4 = std::conditional_t<kR32, pair_f32x4, pair_f64x4>;
+      const int nt = (nc + 15) / 16, n_items = nr * n_r * nt * nt;
+      const size_t row = uv_row;
+      for (int it = wave; it < n_items; it += TT / 64) {
+        const int ta = it % nt, tb = (it / nt) % nt, cr = (it / (nt * nt)) % n_r, rq = it / (nt * nt * n_r);
+        int c = c_lo, ph = 0;  // the cr-th channel with a rank-one term
+        for (int left = cr;; ++c) {
+          const bool has = a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE;
+          if (has && left-- == 0)
+            break;
+          ph += a.ch[c] != PP_UP_DOWN;
+        }
+        const int k1 = ta * 16 + (lane & 15), k2 = tb * 16 + (lane & 15), kl = lane >> 4;
+        const int pl = a.ch[c] == PH_MAGNETIC ? 0 : 1;
+        const C* U = a.UV + pl * row + static_cast<size_t>(q0 + r0 + rq + g.nq * iv) * P +
+                     nc * static_cast<size_t>(w1) + (k1 < nc ? k1 : 0);
+        const C* V = a.UV + (pl + 2) * row + static_cast<size_t>(q0 + r0 + rq + g.nq * iv) * P +
+                     nc * static_cast<size_t>(w2) + (k2 < nc ? k2 : 0);
+        V4 fr{0, 0, 0, 0}, fi{0, 0, 0, 0};
+        double dr[4] = {0, 0, 0, 0}, di[4] = {0, 0, 0, 0};
+        constexpr int RU = 4;  // steps of four walkers loaded together
+        for (int m0 = 0; m0 < n_walk; m0 += 4 * RU) {
+          C u[RU], v[RU];
+          bool live[RU];
+#pragma unroll
+          for (int i = 0; i < RU; ++i) {
+            const int m = m0 + 4 * i + kl;
+            live[i] = m < n_walk;
+            const size_t mo = 4 * row * static_cast<size_t>(m < n_walk ? m : n_walk - 1);
+            u[i] = U[mo];
+            v[i] = V[mo];
+          }
+#pragma unroll
+          for (int i = 0; i < RU; ++i) {
+            if (m0 + 4 * i >= n_walk)
+              break;
+            // R += V U = (Vx Ux - Vy Uy) + i (Vy Ux + Vx Uy)
+            const C vv = live[i] ? v[i] : C{0, 0}, uu = live[i] ? u[i] : C{0, 0};
+            const RT vr = vv.x, vi = vv.y, ur = uu.x, ui = uu.y;
+            fr = mma4(vr, ur, fr);
+            fi = mma4(vi, ur, fi);
+            fr = mma4(-vi, ui, fr);
+            fi = mma4(vr, ui, fi);
+            if (kR32 && (i % 2 == 1 || m0 + 4 * i + 4 >= n_walk)) {  // eight walkers per FP32 sum
+#pragma unroll
+              for (int h = 0; h < 4; ++h) {
+                dr[h] += static_cast<double>(fr[h]);
+                di[h] += static_cast<double>(fi[h]);
+              }
+              fr = fi = V4{0, 0, 0, 0};
+            }
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int kr = tb * 16 + (kR32 ? 4 * kl + h : kl + 4 * h);
+          if (k1 < nc && kr < nc)
+            Rl[(rq * n_ph + ph) * bs + kr * ld + k1] =
+                kR32 ? double2{dr[h], di[h]} : double2{static_cast<double>(fr[h]), static_cast<double>(fi[h])};
+        }
+      }
+      __syncthreads();
+    }
+    // The tile's own entries, CG channels' loads in flight before their stores.
+    int ph0 = 0;
+    for (int c0 = c_lo; c0 < c_hi; c0 += CG) {
+#pragma unroll
+      for (int i0 = 0; i0 < RB * PPT; i0 += GS) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        float4 old[CG][GS], oldp[HZ ? GS : 1];  // at most one pp channel
+#pragma unroll
+        for (int k = 0; k < CG; ++k)
+          if (c0 + k < c_hi)
+#pragma unroll
+            for (int i = 0; i < GS; ++i) {
+              const int r = (i0 + i) / PPT, j = (i0 + i) % PPT;
+              if (r >= nr || !ok[j])
+                continue;
+              const int qv = q0 + r0 + r + g.nq * iv;
+              old[k][i] = static_cast<const float4*>(a.g4[c0 + k])[own_index(tid, j, qv)];
+              if (img_p && a.ch[c0 + k] == PP_UP_DOWN)
+                oldp[HZ ? i : 0] =
+                    static_cast<const float4*>(a.g4[c0 + k])[swap_index(tid, j, qv, a.k_ex[q0 + r0 + r])];
+            }
+        int ph = ph0;
+#pragma unroll
+        for (int k = 0; k < CG; ++k)
+          if (c0 + k < c_hi) {
+            const int type = a.ch[c0 + k];
+            const bool is_pp = HZ && type == PP_UP_DOWN;
+            void* g4 = a.g4[c0 + k];
+#pragma unroll
+            for (int i = 0; i < GS; ++i) {
+              const int r = (i0 + i) / PPT, j = (i0 + i) % PPT;
+              if (r >= nr || !ok[j])
+                continue;
+              const int qv = q0 + r0 + r + g.nq * iv;
+              double2 v;
+              if (is_pp)
+                v = tz[j][r0 + r];
+              else if (HX && (type == PH_MAGNETIC || type == PH_CHARGE)) {
+                v = Rl[(r * n_ph + ph) * bs + li[j]];
+                v.x -= tx[j][r0 + r].x;
+                v.y -= tx[j][r0 + r].y;
+              }
+              else
+                v = double2{-tt[j][r0 + r].x, -tt[j][r0 + r].y};
+              g4_put(g4, own_index(tid, j, qv), old[k][i], v, a.sum_mode);
+              if (!is_pp && (img_t || img_c))
+                Rl[(r * n_ph + ph) * bs + li[j]] = v;
+              if (is_pp && img_p)
+                g4_put(g4, swap_index(tid, j, qv, a.k_ex[q0 + r0 + r]), oldp[HZ ? i : 0], v, a.sum_mode);
+            }
+            ph += !is_pp;
+          }
+      }
+      for (int k = 0; k < CG && c0 + k < c_hi; ++k)
+        ph0 += a.ch[c0 + k] != PP_UP_DOWN;
+    }
+    if (n_ph == 0 || (!img_t && !img_c))
       continue;
-    const int q = a.k_ex[q0 + qi];
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      if (a.ch[c] == PP_UP_DOWN) {
-        if (img_p)
-#pragma unroll
-          for (int j = 0; j < PPT; ++j)
-            if (ok[j])
-              store(c, g4_index(a.k_sub[k1[j] + nc * q], p1, a.k_sub[k2[j] + nc * q], p2, qv[qi]), tot[j][qi][c]);
+    __syncthreads();
+    // Images of the particle-hole channels.
+    for (int kind = 0; kind < 3; ++kind) {  // T, C, both
+      if (!(kind == 0 ? img_t : kind == 1 ? img_c : img_t && img_c))
         continue;
-      }
-      if (!img_t && !img_c)
-        continue;
-      __syncthreads();
+      const int wa = kind == 0 ? w2 : kind == 1 ? c1 : c2, wb = kind == 0 ? w1 : kind == 1 ? c2 : c1;
+      int ph0 = 0;
+      for (int c0 = c_lo; c0 < c_hi; c0 += CG) {
 #pragma unroll
-      for (int j = 0; j < PPT; ++j)
-        if (ok[j])
-          tl[k1[j] + ld * k2[j]] = tot[j][qi][c];
-      __syncthreads();
+        for (int i0 = 0; i0 < RB * PPT; i0 += GS) {
+          int tid = threadIdx.x;
+          asm volatile("" : "+v"(tid));
+          float4 old[CG][GS];
 #pragma unroll
-      for (int j = 0; j < PPT; ++j) {
-        if (!ok[j])
-          continue;
-        if (img_t)
-          store(c, g4_index(k1[j], w2, k2[j], w1, qv[qi]),
-                tl[a.k_sub[q + nc * k2[j]] + ld * a.k_sub[q + nc * k1[j]]]);
-        if (img_c) {
-          double2 v = tl[a.k_neg[a.k_add[k2[j] + nc * q]] + ld * a.k_neg[a.k_add[k1[j] + nc * q]]];
-          v.y = -v.y;
-          store(c, g4_index(k1[j], c1, k2[j], c2, qv[qi]), v);
+          for (int k = 0; k < CG; ++k)
+            if (c0 + k < c_hi && a.ch[c0 + k] != PP_UP_DOWN)
+#pragma unroll
+              for (int i = 0; i < GS; ++i) {
+                const int r = (i0 + i) / PPT, j = (i0 + i) % PPT, idx = tid + TT * j;
+                if (r < nr && ok[j])
+                  old[k][i] = static_cast<const float4*>(
+                      a.g4[c0 + k])[g4_index(idx % nc, wa, idx / nc, wb, q0 + r0 + r + g.nq * iv)];
+              }
+          int ph = ph0;
+#pragma unroll
+          for (int k = 0; k < CG; ++k)
+            if (c0 + k < c_hi && a.ch[c0 + k] != PP_UP_DOWN) {
+#pragma unroll
+              for (int i = 0; i < GS; ++i) {
+                const int r = (i0 + i) / PPT, j = (i0 + i) % PPT;
+                if (r >= nr || !ok[j])
+                  continue;
+                const int idx = tid + TT * j, k1 = idx % nc, k2 = idx / nc;
+                const int q = a.k_ex[q0 + r0 + r];
+                int s1, s2;
+                if (kind == 0) {
+                  s1 = a.k_sub[q + nc * k2];
+                  s2 = a.k_sub[q + nc * k1];
+                }
+                else if (kind == 1) {
+                  s1 = a.k_neg[a.k_add[k2 + nc * q]];
+                  s2 = a.k_neg[a.k_add[k1 + nc * q]];
+                }
+                else {
+                  s1 = a.k_neg[k1];
+                  s2 = a.k_neg[k2];
+                }
+                double2 v = Rl[(r * n_ph + ph) * bs + s2 * ld + s1];
+                if (kind != 0)
+                  v.y = -v.y;
+                g4_put(a.g4[c0 + k], g4_index(k1, wa, k2, wb, q0 + r0 + r + g.nq * iv), old[k][i], v, a.sum_mode);
+              }
+              ++ph;
+            }
         }
-        if (img_t && img_c) {
-          double2 v = tl[a.k_neg[k1[j]] + ld * a.k_neg[k2[j]]];
-          v.y = -v.y;
-          store(c, g4_index(k1[j], c2, k2[j], c1, qv[qi]), v);
-        }
+        for (int k = 0; k < CG && c0 + k < c_hi; ++k)
+          ph0 += a.ch[c0 + k] != PP_UP_DOWN;
       }
+    }
     }
   }
 }
 
 namespace {
 
-template <typename Real, int TT, int PPT, int QG, int NCH, int MASK>
-void launch_tiled_fixed(TiledArgs<Real> a, size_t lds, hipStream_t st) {
+template <typename Real, int TT, int PPT, int QG, int SET>
+void launch_pair_set(TiledArgs<Real> a, size_t lds, hipStream_t st) {
   const unsigned tiles = tile_schedule(a);
-  constexpr bool kRX = std::is_same<Real, float>::value && MASK != 0 &&
-                       (MASK & ((1 << PH_MAGNETIC) | (1 << PH_CHARGE))) != 0;
-  if constexpr (kRX) {
-    if (a.R) {
-      launch_g4_rank1(a, st);
-      if constexpr (TT == 1024 && PPT == 2) {
-        // The pipelined tile stages X beside Y and Z (both spins each).
-        constexpr int kY = (1 << PH_MAGNETIC) | (1 << PH_CHARGE) | (1 << PH_TRANSVERSE);
-        constexpr int NBK = 1 + ((MASK & kY) != 0) + ((MASK & (1 << PP_UP_DOWN)) != 0);
-        lds = sizeof(Cplx<Real>) * 2 * NBK * static_cast<size_t>(a.g.nc) * (a.g.nc + 1);
-      }
-      hipLaunchKernelGGL((g4_tiled_kernel<Real, TT, PPT, QG, NCH, MASK, true>), dim3(tiles), dim3(TT), lds, st, a);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((g4_tiled_kernel<Real, TT, PPT, QG, NCH, MASK, false>), dim3(tiles), dim3(TT), lds, st, a);
+  hipLaunchKernelGGL((g4_pair_kernel<Real, TT, PPT, QG, SET>), dim3(tiles), dim3(TT), lds, st, a);
 }
 
-// Channel sets of the measured workloads get their own instantiations (registers sized for the
-// terms they need); any other set reads the channel flags at run time.
 template <typename Real, int TT, int PPT, int QG>
-bool launch_tiled_nch(const TiledArgs<Real>& a, size_t lds, hipStream_t st) {
-  int mask = 0;
-  for (int c = 0; c < a.n_ch; ++c)
-    mask |= 1 << a.ch[c];
-  constexpr int M = 1 << PH_MAGNETIC, Q = 1 << PH_CHARGE, P = 1 << PP_UP_DOWN;
-  switch (mask) {
-    case M | Q | P: launch_tiled_fixed<Real, TT, PPT, QG, 3, M | Q | P>(a, lds, st); return true;
-    case M | P: launch_tiled_fixed<Real, TT, PPT, QG, 2, M | P>(a, lds, st); return true;
-    case Q: launch_tiled_fixed<Real, TT, PPT, QG, 1, Q>(a, lds, st); return true;
-    case M: launch_tiled_fixed<Real, TT, PPT, QG, 1, M>(a, lds, st); return true;
-    default: break;
-  }
-  switch (a.n_ch) {
-    case 1: launch_tiled_fixed<Real, TT, PPT, QG, 1, 0>(a, lds, st); return true;
-    case 2: launch_tiled_fixed<Real, TT, PPT, QG, 2, 0>(a, lds, st); return true;
-    case 3: launch_tiled_fixed<Real, TT, PPT, QG, 3, 0>(a, lds, st); return true;
-    case 4: launch_tiled_fixed<Real, TT, PPT, QG, 4, 0>(a, lds, st); return true;
-    default: return false;
+void launch_pair_shape(const TiledArgs<Real>& a, int set, size_t lds, hipStream_t st) {
+  switch (set) {
+    case HAS_X: launch_pair_set<Real, TT, PPT, QG, HAS_X>(a, lds, st); break;
+    case HAS_Z: launch_pair_set<Real, TT, PPT, QG, HAS_Z>(a, lds, st); break;
+    case HAS_X | HAS_Z: launch_pair_set<Real, TT, PPT, QG, HAS_X | HAS_Z>(a, lds, st); break;
+    case HAS_T:
+    case HAS_X | HAS_T: launch_pair_set<Real, TT, PPT, QG, HAS_X | HAS_T>(a, lds, st); break;
+    default: launch_pair_set<Real, TT, PPT, QG, HAS_X | HAS_Z | HAS_T>(a, lds, st); break;
   }
 }
 
@@ -650,6 +608,8 @@ TileShape tile_shape(int nc) {
     return {256, 2};
   if (pairs <= 1024)
     return {1024, 1};
+  if (pairs <= 1408)
+    return {704, 2};
   if (pairs <= 2048)
     return {1024, 2};
   if (pairs <= 4096)
@@ -724,9 +684,13 @@ std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>&
   return out;
 }
 
-size_t tiled_lds_bytes(const Geo& g, bool need_y, bool need_z, size_t cplx_bytes, int qg) {
+// LDS of a workgroup: the staged blocks (both spins), or the rank-one planes of the particle-hole
+// channels that are finished together.
+size_t tiled_lds_bytes(const Geo& g, int n_ph, bool need_z, size_t cplx_bytes, int qg) {
   const size_t bs = static_cast<size_t>(g.nc) * (g.nc + 1);
-  return cplx_bytes * (bs * 2 * ((need_y ? 1 : 0) + (need_z ? 1 : 0)) + 4 * static_cast<size_t>(qg) * g.nc);
+  const TileShape ts = tile_shape(g.nc);
+  const int planes = (ts.threads == 256 && ts.ppt == 1 ? qg : 1) * (ts.ppt == 4 ? std::min(n_ph, 1) : n_ph);
+  return bs * std::max(cplx_bytes * 2 * ((n_ph > 0 ? 1 : 0) + (need_z ? 1 : 0)), sizeof(double2) * planes);
 }
 
 template <typename Real>
@@ -736,33 +700,23 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
   const int ppt = ts.ppt;
   if (g.nb != 1 || ppt == 0 || a.n_ch < 1 || a.n_ch > 4)
     return false;
-  // Momenta per workgroup: as many as fit 16 FP64 accumulators per thread (and as the
-  // instantiated shapes provide: 4 for one pair per thread, 2 for two, else 1).
-  int qg = g.nq >= 4 ? 4 : (g.nq >= 2 ? 2 : 1);
-  if (ppt == 2 && qg > 2)
+  int set = 0, n_ph = 0;
+  for (int c = 0; c < a.n_ch; ++c) {
+    set |= a.ch[c] == PP_UP_DOWN ? HAS_Z : a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE ? HAS_X : HAS_T;
+    n_ph += a.ch[c] != PP_UP_DOWN;
+  }
+  // Momenta per workgroup: as many as keep the FP64 totals (pairs x momenta x terms, four registers
+  // each) at 64 registers; at 32 where the loads in flight need the others (complex128 G or four
+  // pairs per thread in a 1024-thread workgroup, 128 registers).
+  const int terms = set == (HAS_X | HAS_Z) ? 2 : set == HAS_X || set == HAS_Z ? 1 : set & HAS_Z ? 3 : 2;
+  const int budget = ts.threads == 1024 && (sizeof(Real) == 8 || ppt == 4) ? 8 : 16;
+  int qg = g.nq >= 3 ? 4 : g.nq;
+  if (ppt == 4 && qg > 2)
     qg = 2;
-  if (ppt > 2)
-    qg = 1;
-  // FP64 accumulators per thread: 16 for 256-thread workgroups, 4 for 1024-thread ones (8 when
-  // the batch's rank-one terms come precomputed, which frees the factor staging and partials).
-  int mask = 0;
-  for (int c = 0; c < a.n_ch; ++c)
-    mask |= 1 << a.ch[c];
-  constexpr int kM = 1 << PH_MAGNETIC, kQ = 1 << PH_CHARGE, kP = 1 << PP_UP_DOWN;
-  // The pipelined 1024 x 2 tile (the rank-one path of that shape) addresses a walker's G with
-  // 32-bit offsets and stages at most 4 x 1024 elements per walker (3 nc^2: Nc <= 36).
-  if (ts.threads == 1024 && ppt == 2 &&
-      (2 * static_cast<size_t>(g.D) * g.D >= (size_t(1) << 31) || 3 * g.nc * g.nc > 4 * 1024))
-    a.R = nullptr;
-  const bool rx = std::is_same<Real, float>::value && a.R != nullptr &&
-                  (mask == (kM | kQ | kP) || mask == (kM | kP) || mask == kQ || mask == kM);
-  const int acc_budget = ts.threads == 256 ? 16 : (rx ? 8 : 4);
-  while (qg > 1 && ppt * qg * a.n_ch > acc_budget)
+  while (qg > 1 && ppt * qg * terms > budget)
     qg /= 2;
   while (a.qg_cap > 0 && qg > a.qg_cap)
     qg /= 2;
-  if (ppt * qg * a.n_ch > 16 || 4 * qg * g.nc > ts.threads)
-    return false;  // accumulators would not fit in registers / one staged factor per thread
   a.nqg = (g.nq + qg - 1) / qg;
   // Where every tile is resident at once (four 256-thread workgroups per CU, one of 1024), half of
   // them take as long as all, and writing the images comes on top: 6x6, 16 walkers, 16 frequencies
@@ -770,37 +724,36 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
   if (a.sym >= SYM_CONJ &&
       static_cast<size_t>(g.nw) * g.nw * g.nv * a.nqg <= (ts.threads == 256 ? size_t(1024) : size_t(256)))
     a.sym = a.sym_few;
-  const size_t lds = tiled_lds_bytes(g, a.need_y, a.need_z, sizeof(Cplx<Real>), qg);
-  const dim3 ug((g.nc * g.nw + 255) / 256, g.nq * g.nv, a.n_walkers);
-  hipLaunchKernelGGL(uv_kernel<Real>, ug, dim3(256), 0, st, a);
-  if constexpr (std::is_same<Real, float>::value) {
-    if (a.mfma && ts.threads == 256 && ppt == 1) {
-      TiledArgs<float> b = a;
-      b.sym = SYM_NONE;  // the matrix-core tile computes every tile and reads all of G
-      b.half_g = false;
-      if (launch_g4_mfma(b, qg, st))
-        return true;
-    }
+  const size_t lds = tiled_lds_bytes(g, n_ph, a.need_z, sizeof(Cplx<Real>), qg);
+  if (set & HAS_X) {
+    const dim3 ug((g.nc * g.nw + 255) / 256, g.nq * g.nv, a.n_walkers);
+    hipLaunchKernelGGL(uv_kernel<Real>, ug, dim3(256), 0, st, a);
   }
   auto by_qg = [&](auto tt, auto pp) {
     constexpr int TT = decltype(tt)::value, PP = decltype(pp)::value;
     if (qg == 4)
-      return launch_tiled_nch<Real, TT, PP, (PP == 1 ? 4 : 1)>(a, lds, st);
-    if (qg == 2)
-      return launch_tiled_nch<Real, TT, PP, (PP <= 2 ? 2 : 1)>(a, lds, st);
-    return launch_tiled_nch<Real, TT, PP, 1>(a, lds, st);
+      launch_pair_shape<Real, TT, PP, (PP <= 2 ? 4 : 2)>(a, set, lds, st);
+    else if (qg == 2)
+      launch_pair_shape<Real, TT, PP, 2>(a, set, lds, st);
+    else
+      launch_pair_shape<Real, TT, PP, 1>(a, set, lds, st);
   };
   using I256 = std::integral_constant<int, 256>;
+  using I704 = std::integral_constant<int, 704>;
   using I1024 = std::integral_constant<int, 1024>;
-  if (ts.threads == 256)
-    return ppt == 1 ? by_qg(I256{}, std::integral_constant<int, 1>{})
-                    : by_qg(I256{}, std::integral_constant<int, 2>{});
-  switch (ppt) {
-    case 1: return by_qg(I1024{}, std::integral_constant<int, 1>{});
-    case 2: return by_qg(I1024{}, std::integral_constant<int, 2>{});
-    case 4: return by_qg(I1024{}, std::integral_constant<int, 4>{});
-    default: return false;
-  }
+  if (ts.threads == 256 && ppt == 1)
+    by_qg(I256{}, std::integral_constant<int, 1>{});
+  else if (ts.threads == 256)
+    by_qg(I256{}, std::integral_constant<int, 2>{});
+  else if (ts.threads == 704)
+    by_qg(I704{}, std::integral_constant<int, 2>{});
+  else if (ppt == 1)
+    by_qg(I1024{}, std::integral_constant<int, 1>{});
+  else if (ppt == 2)
+    by_qg(I1024{}, std::integral_constant<int, 2>{});
+  else
+    by_qg(I1024{}, std::integral_constant<int, 4>{});
+  return true;
 }
 
 template bool launch_g4_tiled<double>(TiledArgs<double>, hipStream_t);

@@ -133,7 +133,6 @@ struct g4acc_handle {
   int mtog_large = 0;
   bool large_ok = false, large_e = false, right_fused_ok = false;
   int g4_qg = 0;                   // tuning: momenta per G4 workgroup (0: register limit)
-  int g4_mfma = 0;                 // tuning: rank-one G4 terms on the matrix cores (FP32 G, Nc <= 16)
   // tuning: g4_sym = 0 computes every G4 tile. sym_ok: the transpose symmetry alone applies (one
   // q = 0, one v = 0, channels among magnetic, charge, transverse). conj_sym: G4Sym of handles
   // whose G is conjugate symmetric (SYM_NONE otherwise), their inversion table and tile tables in
@@ -143,15 +142,9 @@ struct g4acc_handle {
   int conj_sym = SYM_NONE;
   int *d_kneg = nullptr, *d_stab[2] = {nullptr, nullptr};
   int n_stab = 0;
-  // tuning: rank-one MAGNETIC / CHARGE terms of a batch as one matrix-core GEMM (g4_rank1.hip),
-  // stored in d_R (complex64, one G4-sized plane per channel) and added by the tile kernel.
-  int g4_rank1 = 0;
-  void* d_R = nullptr;
   // This device's address of the static workspace of g4acc_compute_G_noalloc.
   unsigned char* d_scratch = nullptr;
   std::string scratch_err;
-  int* d_r1_planes = nullptr;
-  int n_r1 = 0, r1_slot[4] = {-1, -1, -1, -1};
   // Single-particle accumulator (g4acc_sp_enable): sorted by caller orbital, exact M_r_w sums.
   bool sp = false;
   bool sp_sqr = false;
@@ -192,9 +185,8 @@ struct g4acc_handle {
     *p = static_cast<T*>(q);
     return G4ACC_OK;
   }
-  // The G4 stage reads the half w1 + w2 >= nwE - 1 of G only (the matrix-core tile kernel of
-  // g4_mfma reads all of it), so M -> G forms that half.
-  bool half_g() const { return g4_sym && conj_sym && !(g4_mfma && precision == G4ACC_FP32 && g.nc <= 16); }
+  // The G4 stage reads the half w1 + w2 >= nwE - 1 of G only, so M -> G forms that half.
+  bool half_g() const { return g4_sym && conj_sym; }
   size_t cplx_bytes() const { return precision == G4ACC_FP64 ? 16 : 8; }
 };
 
@@ -585,13 +577,12 @@ void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
     a.desc = h->d_desc;
     a.n_walkers = n_walkers;
     a.n_ch = static_cast<int>(h->channels.size());
-    a.need_y = a.need_z = a.has_trans = false;
+    a.need_y = a.need_z = false;
     for (int c = 0; c < a.n_ch; ++c) {
       a.ch[c] = h->channels[c];
       a.g4[c] = h->d_g4[c];
       a.need_y |= a.ch[c] != G4ACC_PARTICLE_PARTICLE_UP_DOWN;
       a.need_z |= a.ch[c] == G4ACC_PARTICLE_PARTICLE_UP_DOWN;
-      a.has_trans |= a.ch[c] == G4ACC_PARTICLE_HOLE_TRANSVERSE;
     }
     a.k_add = h->d_kadd;
     a.k_sub = h->d_ksub;
@@ -604,7 +595,6 @@ void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
     a.tile_order = h->tile_order >= 0 ? h->tile_order : (n_walkers > 1 ? 2 : 0);
     a.tile_perm = h->d_tperm;
     a.sum_mode = h->sum_mode;
-    a.mfma = h->g4_mfma;
     // One walker's launch is the G4 read-modify-write, which half of the tiles with scattered
     // images does no faster (4x4, 8 transfers, three channels, 32 frequencies: 13.6 against 13.1 ms
     // for 64 measurements); from two walkers on the tiles' reads and products count.
@@ -614,12 +604,6 @@ void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
     a.k_neg = h->d_kneg;
     a.sym_tiles = h->d_stab[a.tile_order == 0 ? 0 : 1];
     a.n_sym_tiles = h->n_stab;
-    const bool r1 = std::is_same<Real, float>::value && h->g4_rank1 && h->d_R;
-    a.R = r1 ? h->d_R : nullptr;
-    a.n_r1 = h->n_r1;
-    a.r1_planes = h->d_r1_planes;
-    for (int c = 0; c < 4; ++c)
-      a.r1_slot[c] = h->r1_slot[c];
     if (launch_g4_tiled<Real>(a, h->stream))
       return;
   }
@@ -951,15 +935,16 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
   // The LDS-tiled G4 kernel covers one band, Nc >= 8 and tiles whose staged G blocks fit the
   // workgroup's LDS.
   {
-    bool need_y = false, need_z = false;
+    int n_ph = 0;
+    bool need_z = false;
     for (int c : h->channels) {
-      need_y |= c != G4ACC_PARTICLE_PARTICLE_UP_DOWN;
+      n_ph += c != G4ACC_PARTICLE_PARTICLE_UP_DOWN;
       need_z |= c == G4ACC_PARTICLE_PARTICLE_UP_DOWN;
     }
     int max_lds = 0;
     if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, h->device) != hipSuccess)
       max_lds = 65536;
-    const size_t lds = tiled_lds_bytes(g, need_y, need_z, cb, 4);
+    const size_t lds = tiled_lds_bytes(g, n_ph, need_z, cb, 4);
     if (const char* to = getenv("G4ACC_TILE_ORDER"))
       h->tile_order = atoi(to);
     if (const char* gr = getenv("G4ACC_GRAPH"))
@@ -1081,19 +1066,10 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
     launch_zero16(p, h->g4_entries, h->stream);
   if ((rc = h->check(hipStreamSynchronize(h->stream), "hipStreamSynchronize")))
     return bail(rc);
-  // Default launch shapes for callers that do not tune (the C++ drop-in): the matrix-core forms
-  // where they were measured faster, complex64 G on 16-site clusters with batches of 8 or more.
-  if (h->precision != G4ACC_FP64 && g.nb == 1 && g.nc == 16 && !h->general()) {
+  // Default for callers that do not tune (the C++ drop-in): the matrix-core right half of M -> G
+  // where it was measured faster, complex64 G on 16-site clusters.
+  if (h->precision != G4ACC_FP64 && g.nb == 1 && g.nc == 16 && !h->general())
     h->mtog_mfma = 1;
-    int mask = 0;
-    for (int c : h->channels)
-      mask |= 1 << c;
-    constexpr int M = 1 << G4ACC_PARTICLE_HOLE_MAGNETIC, Q = 1 << G4ACC_PARTICLE_HOLE_CHARGE,
-                  P = 1 << G4ACC_PARTICLE_PARTICLE_UP_DOWN;
-    if (h->use_tiled && h->max_walkers >= 8 && (mask == (M | Q | P) || mask == (M | P) || mask == M || mask == Q) &&
-        (rc = g4acc_set_tuning(h, "g4_rank1", 1)) != G4ACC_OK)
-      return bail(rc);
-  }
   *out = h;
   return G4ACC_OK;
 }
@@ -1657,8 +1633,10 @@ int g4acc_set_tuning(g4acc_handle* h, const char* key, int value) {
     h->g4_qg = value;
   else if (k == "g4_tile_order" && value >= -1 && value <= 2)
     h->tile_order = value;
-  else if (k == "g4_mfma" && (value == 0 || value == 1))
-    h->g4_mfma = value;
+  else if ((k == "g4_mfma" || k == "g4_rank1") && (value == 0 || value == 1)) {
+    // Accepted for callers that set them: the tile kernel always forms the rank-one terms on the
+    // matrix cores, after its walker loop.
+  }
   else if (k == "g4_tile_strip" && value >= 1 && value <= 16) {
     // Diagonal positions per group of schedule 2 (table uploaded now, outside any batch).
     const std::vector<int> tperm = diagonal_tile_order(h->g.nw, value);
@@ -1667,33 +1645,6 @@ int g4acc_set_tuning(g4acc_handle* h, const char* key, int value) {
         (rs = h->check(hipMemcpy(h->d_tperm, tperm.data(), tperm.size() * sizeof(int), hipMemcpyHostToDevice),
                        "hipMemcpy")))
       return rs;
-  }
-  else if (k == "g4_rank1" && (value == 0 || value == 1)) {
-    if (value && !h->d_R && h->use_tiled && h->precision != G4ACC_FP64) {
-      int rs;
-      if ((rs = h->check(hipSetDevice(h->device), "hipSetDevice")))
-        return rs;
-      // One complex64 plane of G4's (k1, w1, k2, w2, q, v) size per rank-one channel.
-      std::vector<int> planes;
-      for (size_t c = 0; c < h->channels.size(); ++c) {
-        const int ch = h->channels[c];
-        if (ch == G4ACC_PARTICLE_HOLE_MAGNETIC || ch == G4ACC_PARTICLE_HOLE_CHARGE) {
-          h->r1_slot[c] = static_cast<int>(planes.size());
-          planes.push_back(ch == G4ACC_PARTICLE_HOLE_MAGNETIC ? 0 : 1);  // U plane of uv_kernel
-        }
-      }
-      if (!planes.empty()) {
-        int rc;
-        if ((rc = h->alloc(reinterpret_cast<float2**>(&h->d_R), planes.size() * h->g4_entries, "R")) ||
-            (rc = h->alloc(&h->d_r1_planes, planes.size(), "r1_planes")))
-          return rc;
-        if ((rc = h->check(hipMemcpy(h->d_r1_planes, planes.data(), planes.size() * sizeof(int),
-                                     hipMemcpyHostToDevice), "hipMemcpy")))
-          return rc;
-        h->n_r1 = static_cast<int>(planes.size());
-      }
-    }
-    h->g4_rank1 = value;
   }
   else if (k == "graph" && (value == 0 || value == 1))
     h->use_graph = value != 0;

@@ -123,7 +123,7 @@ template <typename Real>
 struct TiledArgs {
   Geo g;
   const Cplx<Real>* G;         // [n_slots][D][D]
-  Cplx<Real>* UV;              // [walkers][4][nq*nv][Nc*nw]
+  Cplx<Real>* UV;              // [walkers][4][nq*nv][Nc*nw] rank-one factors
   const SlotDesc* desc;
   int n_walkers;
   int n_ch;
@@ -139,15 +139,7 @@ struct TiledArgs {
   int super_tile, n_super, n_xcd;  // tile schedule (set by the launcher)
   const int* tile_perm;        // schedule 2: (w1 | w2 << 16) in dispatch order, nw * nw entries
   int sum_mode;
-  int mfma;                    // 1: rank-one terms on the matrix cores where a kernel provides it
-  // Rank-one terms precomputed for the batch (complex64 G, 256-thread tiles): R[c][q,v][p2][p1] for
-  // the n_r1 channels with r1_planes[c] their U plane, and r1_slot[ch] the R plane of G4 channel
-  // slot ch (-1: none). R == nullptr: the tile kernel forms them itself.
-  void* R;
-  int n_r1;
-  const int* r1_planes;  // device, n_r1 entries
-  int r1_slot[4];
-  bool need_y, need_z, has_trans;
+  bool need_y, need_z;         // particle-hole channels, pp
   // Symmetries of G4 used to compute a part of the tiles and write their images (G4Sym).
   int sym = 0, sym_few = 0;  // sym_few: where the launch has few tiles
   // G is conjugate symmetric: only its half wa + wb >= nwE - 1 (extended frequencies) is read.
@@ -159,12 +151,6 @@ struct TiledArgs {
 
 template <typename Real>
 bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st);
-// The matrix-core form of the single-band tile kernel (FP32 G, Nc <= 16, one pair per thread);
-// false if it does not cover the geometry or channel set. The caller has run uv_kernel and set
-// a.nqg for momentum groups of qg.
-bool launch_g4_mfma(const TiledArgs<float>& a, int qg, hipStream_t st);
-// R of the batch from the rank-one factors (g4_rank1.hip); the caller has run uv_kernel.
-void launch_g4_rank1(const TiledArgs<float>& a, hipStream_t st);
 // Multiband LDS-tiled G4 update (g4_band.hip); false if the band count, cluster or channel set
 // is not covered (the generic kernel then runs).
 template <typename Real>
@@ -176,8 +162,8 @@ std::vector<int> diagonal_tile_order(int nw, int strip);
 // (strip > 0) or w1 fastest (strip = 0).
 std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>& w_ex, bool has_ph, bool has_pp,
                                       int sym);
-// LDS of one tile workgroup with momentum groups of qg (staged blocks and rank-one factors).
-size_t tiled_lds_bytes(const Geo& g, bool need_y, bool need_z, size_t cplx_bytes, int qg);
+// LDS of one tile workgroup with momentum groups of qg and n_ph particle-hole channels.
+size_t tiled_lds_bytes(const Geo& g, int n_ph, bool need_z, size_t cplx_bytes, int qg);
 
 // Single-particle accumulator (sp_acc.hip): exact FP64 M_r_w of the batch's slots added to acc
 // (and M_ij^2's to acc_sqr when squared_too), acc laid out [s][(b1 + nb (b2 + nb r)) n_w + w].

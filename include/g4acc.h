@@ -272,21 +272,18 @@ int g4acc_set_timing(g4acc_handle* h, int enable);
  * 0 = as many as registers allow, 1, 2, 4), "g4_tile_order" (-1 by batch size: 2 for batches, 0 for
  * one walker; 0 natural,
  * 1 XCD-aware super-tiles, 2 XCD-aware diagonal strips with their mirror images),
- * "g4_tile_strip" (diagonal positions per group of schedule 2: 1..16, default 2), "g4_mfma"
- * (1: rank-one G4 terms on the matrix cores where available, FP32 G and Nc <= 16; 0: vector ALUs),
- * "g4_rank1" (1: the batch's rank-one MAGNETIC / CHARGE terms as one matrix-core GEMM into a
- * complex64 buffer of G4's size per such channel, allocated when the key is set; FP32 G,
- * 256-thread tiles, measured channel sets; 0: formed per walker in the tile kernel),
+ * "g4_tile_strip" (diagonal positions per group of schedule 2: 1..16, default 2), "g4_mfma" and
+ * "g4_rank1" (accepted and without effect: the single-band tile kernel always forms the rank-one
+ * MAGNETIC / CHARGE terms on the matrix cores),
  * "graph" (1: replay captured batch sequences, 0: launch eagerly), "mtog_large" (6x6 and 8x8 tori:
  * 0 register-fused M -> G kernels; 1 matrix-core S1/S3 with a D x D workspace per slot of a chunk
  * for S3's output, the FP64 default, in FP32 only when the environment variable G4ACC_MTOG_E was
  * set at creation; 2 FP32 only, S3, the right site transform and the epilogue in one kernel with
  * that output kept in LDS, the FP32 default), "mtog_chunk" (slots per M -> G pass, below the
  * number the workspace was sized for; 0: that number, a whole batch where its workspace fits
- * 24 GiB), "g4_sym" (1: transpose-symmetric G4 tiles where the geometry allows them, the default
- * there; 0: all tiles).
- * Defaults: mtog_mfma = 1 and, with max_walkers >= 8 and a measured channel set, g4_rank1 = 1 for
- * complex64 G on single-band 16-site clusters; 0 elsewhere.
+ * 24 GiB), "g4_sym" (0: all G4 tiles and all of G, instead of the part that the symmetries of the
+ * handle's G leave; 1, accepted where the transpose symmetry alone applies: back to the default).
+ * Defaults: mtog_mfma = 1 for complex64 G on single-band 16-site clusters; 0 elsewhere.
  * Results do not depend on the tuning beyond FP32 summation order. */
 int g4acc_set_tuning(g4acc_handle* h, const char* key, int value);
 int g4acc_get_timing(const g4acc_handle* h, double* mtog_ms, double* g4_ms, long long* batches);
