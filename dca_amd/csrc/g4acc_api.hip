@@ -308,12 +308,13 @@ int detect_grid(int nc, const double* dft, std::vector<int>& xy, std::vector<int
   return 0;
 }
 
-// Finds the inversion k -> -k of the caller's momenta and whether G(-p1, -p2) = conj G(p1, p2)
-// holds for real M: the tables are those of an abelian group, dft(-k, r) = conj dft(k, r) and
-// G0(-p) = conj G0(p) (and the band phases likewise). The last must hold to `tol` of |G0|: the
-// conjugate then stands for an entry that differs from it by less than G's own rounding. A G0
-// without the symmetry (or holding a NaN) fails the test, and every tile is computed.
-bool conjugate_symmetric(const Geo& g, const g4acc_geometry* gm, double tol, double dft_tol, std::vector<int>& neg) {
+bool conjugate_pair(const double* x, const double* y, double bound) {  // y = conj x
+  return std::abs(y[0] - x[0]) <= bound && std::abs(y[1] + x[1]) <= bound;
+}
+
+// Finds the inversion k -> -k of the caller's momenta: the tables are those of an abelian group and
+// dft(-k, r) = conj dft(k, r).
+bool find_inversion(const Geo& g, const g4acc_geometry* gm, double dft_tol, std::vector<int>& neg) {
   const int nc = g.nc;
   auto add = [&](int a, int b) { return gm->k_add[a + static_cast<size_t>(nc) * b]; };
   auto sub = [&](int a, int b) { return gm->k_sub[a + static_cast<size_t>(nc) * b]; };  // k_b - k_a
@@ -340,24 +341,29 @@ bool conjugate_symmetric(const Geo& g, const g4acc_geometry* gm, double tol, dou
       if (add(a, b) != add(b, a) || neg[add(a, b)] != add(neg[a], neg[b]) || sub(a, b) != add(b, neg[a]) ||
           sub(a, add(b, a)) != b || sub(sub(a, b), b) != a)
         return false;
-  auto pair = [&](const double* x, const double* y, double bound) {  // y = conj x
-    return std::abs(y[0] - x[0]) <= bound && std::abs(y[1] + x[1]) <= bound;
-  };
   for (int r = 0; r < nc; ++r)
     for (int k = 0; k < nc; ++k)
-      if (!pair(gm->dft + 2 * (k + static_cast<size_t>(nc) * r), gm->dft + 2 * (neg[k] + static_cast<size_t>(nc) * r),
-                dft_tol))
+      if (!conjugate_pair(gm->dft + 2 * (k + static_cast<size_t>(nc) * r),
+                          gm->dft + 2 * (neg[k] + static_cast<size_t>(nc) * r), dft_tol))
         return false;
+  return true;
+}
+
+// Whether G(-p1, -p2) = conj G(p1, p2) for real M: G0(-p) = conj G0(p) and the band phases likewise, to
+// `tol` of |G0|, so that the conjugate stands for an entry that differs from it by less than G's own
+// rounding. A G0 without the symmetry (or holding a NaN) fails the test, and every tile is computed.
+bool conjugate_symmetric(const Geo& g, const g4acc_geometry* gm, double tol, const std::vector<int>& neg) {
+  const int nc = g.nc;
   if (gm->band_phase)
     for (int k = 0; k < nc; ++k)
-      if (!pair(gm->band_phase + 2 * k, gm->band_phase + 2 * neg[k], tol))
+      if (!conjugate_pair(gm->band_phase + 2 * k, gm->band_phase + 2 * neg[k], tol))
         return false;
   for (int w = 0; w < g.nwE; ++w)
     for (int k = 0; k < nc; ++k)
       for (int s = 0; s < 2; ++s) {
         const double* x = gm->g0 + 2 * (s + 2 * (k + static_cast<size_t>(nc) * w));
         const double* y = gm->g0 + 2 * (s + 2 * (neg[k] + static_cast<size_t>(nc) * (g.nwE - 1 - w)));
-        if (!pair(x, y, tol * std::hypot(x[0], x[1])))
+        if (!conjugate_pair(x, y, tol * std::hypot(x[0], x[1])))
           return false;
       }
   return true;
@@ -550,6 +556,7 @@ MtoGArgs<Real> mtog_args(g4acc_handle* h, int n_slots) {
   a.G0 = h->d_G0;
   a.grid_L = h->grid_L;
   a.kmap = h->d_kmap;
+  a.kneg = h->d_kneg;
   return a;
 }
 
@@ -980,21 +987,24 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
                   c == G4ACC_PARTICLE_HOLE_TRANSVERSE);
     h->sym_ok = ok && getenv("G4ACC_NO_SYM") == nullptr;
   }
-  // Conjugate symmetry of G (single band, real M). Tolerances: complex64 G rounds at 2^-24, so
-  // 2^-30 of G0 does not show; complex128 G allows 16 roundings of G0 itself. The DFT table enters
-  // M -> G only for clusters without the L x L transforms.
-  if (h->use_tiled && getenv("G4ACC_NO_SYM") == nullptr) {
+  // Inversion of the momenta and conjugate symmetry of G (single band, real M). Tolerances: complex64
+  // G rounds at 2^-24, so 2^-30 of G0 does not show; complex128 G allows 16 roundings of G0 itself.
+  // The DFT table enters M -> G only for clusters without the L x L transforms.
+  if (g.nb == 1 && !h->general()) {
     const bool dp = h->precision == G4ACC_FP64;
     const double eps = 2.220446049250313e-16;
     std::vector<int> neg;
-    if (conjugate_symmetric(g, gm, dp ? 16 * eps : 0x1p-30, dp && !h->grid_L ? 64 * eps : 1e-9, neg)) {
+    const bool inv = find_inversion(g, gm, dp && !h->grid_L ? 64 * eps : 1e-9, neg);
+    if (inv)
+      table(&h->d_kneg, neg);
+    if (inv && h->use_tiled && getenv("G4ACC_NO_SYM") == nullptr &&
+        conjugate_symmetric(g, gm, dp ? 16 * eps : 0x1p-30, neg)) {
       bool has_ph = false, has_pp = false, self = g.nv == 1 && gm->w_ex[0] == 0;
       for (int c : h->channels)
         (c == G4ACC_PARTICLE_PARTICLE_UP_DOWN ? has_pp : has_ph) = true;
       for (int q : h->k_ex)
         self = self && neg[q] == q;
       h->conj_sym = self && !has_pp ? SYM_CONJ_TRANSPOSE : SYM_CONJ;
-      table(&h->d_kneg, neg);
       for (int k = 0; k < 2; ++k) {  // w1 fastest, and on diagonal strips of two
         const std::vector<int> t = symmetric_tile_order(g.nw, 2 * k, h->w_ex, has_ph, has_pp, h->conj_sym);
         h->n_stab = static_cast<int>(t.size());
@@ -1066,10 +1076,8 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
     launch_zero16(p, h->g4_entries, h->stream);
   if ((rc = h->check(hipStreamSynchronize(h->stream), "hipStreamSynchronize")))
     return bail(rc);
-  // Default for callers that do not tune (the C++ drop-in): the matrix-core right half of M -> G
-  // where it was measured faster, complex64 G on 16-site clusters.
-  if (h->precision != G4ACC_FP64 && g.nb == 1 && g.nc == 16 && !h->general())
-    h->mtog_mfma = 1;
+  // The matrix-core M -> G of the 4-, 8- and 16-site clusters, measured faster in both precisions.
+  h->mtog_mfma = h->fused_mtog && g.nc <= 16 ? 1 : 0;
   *out = h;
   return G4ACC_OK;
 }

@@ -14,7 +14,7 @@ struct MtoGArgs {
   int chunk;              // slots whose S1..S4 workspaces exist at once
   bool fused;             // use the register-fused single-band kernels
   int tw;                 // frequencies per thread in the fused right kernel (0: default)
-  int mfma;               // fused right kernel on the matrix cores (complex64, Nc <= 16)
+  int mfma;               // 4, 8 and 16 sites: the matrix-core kernels of mtog_small.hip
   // 6x6 and 8x8 clusters: the whole M -> G on the matrix cores with the B, E and Ms workspaces
   // (mtog_large.hip), instead of the register-fused kernels.
   bool large = false;
@@ -41,6 +41,7 @@ struct MtoGArgs {
   // runs as two L-point passes; kmap[kx + L ky] is the caller's momentum index. L = 0: dense DFT.
   int grid_L;
   const int* kmap;
+  const int* kneg = nullptr;  // index(-k), where dft(-k, r) = conj dft(k, r): A(-k, -w) = conj A(k, w)
   // Smallest w1 + w2 (extended frequencies) the consumer reads: nwE - 1 where G is conjugate
   // symmetric and the tile kernel reads that half only, else 0. Blocks of G wholly below it are
   // neither computed nor written.
@@ -66,6 +67,10 @@ void launch_mtog(const MtoGArgs<Real>& a, hipStream_t st);
 template <typename Real>
 bool launch_mtog_fused(const MtoGArgs<Real>& a, hipStream_t st);
 bool mtog_fused_covers(const Geo& g);
+// Matrix-core M -> G of the 4-, 8- and 16-site clusters (mtog_small.hip) on slots [s0, s0 + ns); false
+// where it does not apply (the register-fused kernels then run).
+template <typename Real>
+bool launch_mtog_small(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st);
 // M -> G for single-band 6x6 (NC = 36) and 8x8 (NC = 64) clusters with site labels x + L y, on
 // slots [s0, s0 + ns) of a chunk (needs the Ms, B and E workspaces).
 template <typename Real, int NC>

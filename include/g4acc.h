@@ -266,9 +266,9 @@ int g4acc_set_timing(g4acc_handle* h, int enable);
 
 /* Launch-shape tuning (no counterpart in the reference, whose launch shapes are fixed; set by
  * the autotuner's table, dca_amd/autotune.py). Keys: "mtog_tw" (frequencies per thread of the
- * fused single-band M -> G kernel: 0 default, 1, 2, 4, 8), "mtog_mfma" (1: its right half on the
- * matrix cores where available, FP32 G, Nc <= 8 or a 4x4 torus, max_vertices <= 4 (128 - Nc);
- * 0: vector ALUs), "g4_qg" (momenta per G4 workgroup:
+ * fused single-band M -> G kernel: 0 default, 1, 2, 4, 8), "mtog_mfma" (1: M -> G on the matrix
+ * cores for 4 and 8 sites and the 4x4 torus, max_vertices <= 4 (128 - Nc), the default there;
+ * 0: the fused kernel), "g4_qg" (momenta per G4 workgroup:
  * 0 = as many as registers allow, 1, 2, 4), "g4_tile_order" (-1 by batch size: 2 for batches, 0 for
  * one walker; 0 natural,
  * 1 XCD-aware super-tiles, 2 XCD-aware diagonal strips with their mirror images),
@@ -283,7 +283,6 @@ int g4acc_set_timing(g4acc_handle* h, int enable);
  * number the workspace was sized for; 0: that number, a whole batch where its workspace fits
  * 24 GiB), "g4_sym" (0: all G4 tiles and all of G, instead of the part that the symmetries of the
  * handle's G leave; 1, accepted where the transpose symmetry alone applies: back to the default).
- * Defaults: mtog_mfma = 1 for complex64 G on single-band 16-site clusters; 0 elsewhere.
  * Results do not depend on the tuning beyond FP32 summation order. */
 int g4acc_set_tuning(g4acc_handle* h, const char* key, int value);
 int g4acc_get_timing(const g4acc_handle* h, double* mtog_ms, double* g4_ms, long long* batches);
