@@ -28,23 +28,26 @@
 namespace g4acc {
 
 // ---------------------------------------------------------------------------------------------
-// Counting sort of the vertices of each slot by orbital, stable in the vertex index: the order of
+// Sort of the vertices of each slot by orbital, stable in the vertex index: the order of
 // details::Triple (tp/ndft/triple.hpp:23-30). perm[slot][rank] = vertex index, off[slot][o] =
 // first rank of orbital o (n_orb + 1 entries). Invalid site/band indices raise *err_flag.
-__global__ void __launch_bounds__(256) sort_kernel(const SlotDesc* __restrict__ desc, Geo g,
-                                                   int n_max, const int* __restrict__ site_map,
-                                                   int* __restrict__ perm,
-                                                   int* __restrict__ off, int* __restrict__ err_flag,
-                                                   bool left) {
+// Ranks within an orbital: a wave takes every (waves)-th orbital and walks the vertices 64 at a time,
+// a ballot giving each member its place (N n_orb / 64 lane steps per slot; one thread per vertex
+// counting its predecessors took N steps each, 130 us at N ~ 2000 and 64 orbitals against 17).
+__global__ void __launch_bounds__(1024) sort_kernel(const SlotDesc* __restrict__ desc, Geo g,
+                                                    int n_max, const int* __restrict__ site_map,
+                                                    int* __restrict__ perm,
+                                                    int* __restrict__ off, int* __restrict__ err_flag,
+                                                    bool left) {
   extern __shared__ int lds[];
   int* orb = lds;               // n_max
-  int* cnt = lds + n_max;       // n_orb + 1
+  int* cnt = lds + n_max;       // n_orb: vertices per orbital
   const int slot = blockIdx.x;
   const SlotDesc d = desc[slot];
   const int n = d.n;
   int* P = perm + static_cast<size_t>(slot) * n_max;
   int* O = off + static_cast<size_t>(slot) * (g.n_orb + 1);
-  for (int o = threadIdx.x; o <= g.n_orb; o += blockDim.x)
+  for (int o = threadIdx.x; o < g.n_orb; o += blockDim.x)
     cnt[o] = 0;
   __syncthreads();
   const int* bands = left && d.band_l ? d.band_l : d.band;
@@ -57,22 +60,29 @@ __global__ void __launch_bounds__(256) sort_kernel(const SlotDesc* __restrict__ 
     else
       o = b + g.nb * (site_map ? site_map[r] : r);
     orb[i] = o;
-    atomicAdd(&cnt[o + 1], 1);
+    atomicAdd(&cnt[o], 1);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int o = 1; o <= g.n_orb; ++o)
-      cnt[o] += cnt[o - 1];
-  }
-  __syncthreads();
-  for (int o = threadIdx.x; o <= g.n_orb; o += blockDim.x)
-    O[o] = cnt[o];
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const int o = orb[i];
-    int rank = cnt[o];
-    for (int j = 0; j < i; ++j)
-      rank += (orb[j] == o);
-    P[rank] = i;
+  const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  for (int o = threadIdx.x >> 6; o < g.n_orb; o += waves) {
+    int base = 0;  // vertices of the orbitals before o, summed over the lanes
+    for (int r = lane; r < o; r += 64)
+      base += cnt[r];
+    for (int s = 32; s > 0; s >>= 1)
+      base += __shfl_xor(base, s);
+    if (lane == 0) {
+      O[o] = base;
+      if (o == g.n_orb - 1)
+        O[g.n_orb] = n;
+    }
+    for (int i0 = 0; i0 < n; i0 += 64) {
+      const int i = i0 + lane;
+      const bool mine = i < n && orb[i] == o;
+      const unsigned long long members = __ballot(mine);
+      if (mine)
+        P[base + __popcll(members & ((1ull << lane) - 1))] = i;
+      base += __popcll(members);
+    }
   }
 }
 
@@ -317,8 +327,9 @@ void launch_compute_m(int n, const double* exp_v, const double* N, int ldn, doub
 
 void launch_sort(const SlotDesc* desc, const Geo& g, int n_slots, int n_max, const int* site_map,
                  int* perm, int* off, int* err_flag, hipStream_t st, bool left) {
-  const size_t lds = sizeof(int) * (n_max + g.n_orb + 1);
-  hipLaunchKernelGGL(sort_kernel, dim3(n_slots), dim3(256), lds, st, desc, g, n_max, site_map, perm, off,
+  const size_t lds = sizeof(int) * (n_max + g.n_orb);
+  const int threads = static_cast<size_t>(n_max) * g.n_orb > 256 * 64 ? 1024 : 256;
+  hipLaunchKernelGGL(sort_kernel, dim3(n_slots), dim3(threads), lds, st, desc, g, n_max, site_map, perm, off,
                      err_flag, left);
 }
 
