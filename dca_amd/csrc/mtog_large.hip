@@ -4,6 +4,9 @@
 //   mtog_s1_mfma    S1: B[jj][r][w] = sum_{ii in site r} Ms[ii][jj] T[w, ii]
 //   mtog_left_site  S2: A[(k, w)][jj] = sum_r exp(+i k.r) B[jj][r][w]
 //
+// formed for the upper half of the frequencies where the momenta have their inverses: M is real, so
+// A(-k, -w) = conj A(k, w).
+//
 // Right half, in two kernels (FP64, or FP32 with E as a workspace):
 //
 //   mtog_s3_mfma  S3 on the matrix cores: for every site r of the column sort
@@ -29,12 +32,12 @@
 
 namespace g4acc {
 
-// One workgroup owns 64 rows p1 (16 per wave) and 64 frequencies w2 (four 16 x 16 tiles per wave)
-// and walks the sites. A step takes four vertices of one site: lane l supplies conj-T[w][jj0 + l/16]
-// for w = w0 + 16 t + l%16 and A[p0 + l%16][jj0 + l/16], and after the site holds
-// E[w0 + 16 t + row(l/16, i)][p0 + l%16], i = 0..3, which it stores as 16-entry runs of p1.
-// Loads past the site's vertices or the tile's edges read clamped, in-bounds addresses and are
-// zeroed before use.
+// One workgroup owns 64 rows p1 (16 per wave) and 64 frequencies w2 (four 16 x 16 tiles per wave, of
+// which those below the needed half are left out). The sites' steps form one stream, a step being four
+// vertices of one site: lane l supplies conj-T[w][jj0 + l/16] for w = w0 + 16 t + l%16 and
+// A[p0 + l%16][jj0 + l/16], and after the site holds E[w0 + 16 t + row(l/16, i)][p0 + l%16], i = 0..3,
+// which it stores as 16-entry runs of p1. Two steps are in flight (as in mtog_s1_mfma below): every
+// load is issued, at clamped, in-bounds addresses, and A is zeroed past the site's vertices.
 template <typename Real, int NC>
 __global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0, int w_sum_min,
                                                     const int* __restrict__ off,
@@ -46,7 +49,13 @@ __global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0,
   const int slot = slot0 + blockIdx.z;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int D = g.D, nwE = g.nwE;
-  const int* O = off + static_cast<size_t>(slot) * (NC + 1);
+  const int w0 = blockIdx.y * 64;
+  // Frequency tiles t_lo <= t < t_hi: mtog_site_G reads blocks of 64 rows and one w2.
+  const int w1_hi = (static_cast<int>(blockIdx.x) * 64 + 63) / NC;
+  const int below = w_sum_min - 15 - w1_hi - w0;
+  const int t_lo = below > 0 ? (below + 15) / 16 : 0, t_hi = min(4, (nwE - w0 + 15) / 16);
+  if (t_lo >= t_hi)
+    return;
   const C* Ts = T + static_cast<size_t>(slot) * nwE * n_max;
   const C* Ab = A + static_cast<size_t>(blockIdx.z) * D * n_max;
   C* Eb = E + static_cast<size_t>(blockIdx.z) * D * D;
@@ -54,70 +63,105 @@ __global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0,
   const int pl = blockIdx.x * 64 + 16 * wave + (lane & 15);
   const bool p_ok = pl < D;
   const int pc = p_ok ? pl : D - 1;
-  const int w0 = blockIdx.y * 64;
-  // Tiles below the needed half: pairs are read by mtog_site_G in blocks of 64 rows and one w2.
-  const int w1_hi = (static_cast<int>(blockIdx.x) * 64 + 63) / NC;
   int wc[4];
-  bool w_ok[4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int w = w0 + 16 * t + (lane & 15);
-    w_ok[t] = w < nwE;
-    wc[t] = w_ok[t] ? w : nwE - 1;
-  }
-  if (w0 + 63 + w1_hi < w_sum_min)
-    return;
-  for (int r = 0; r < NC; ++r) {
-    const int b = O[r], e = O[r + 1];
-    V cr[4], ci[4];
+  for (int t = 0; t < 4; ++t)
+    wc[t] = min(w0 + 16 * t + (lane & 15), nwE - 1);
+  __shared__ int Os[NC + 1];
+  if (threadIdx.x <= NC)
+    Os[threadIdx.x] = off[static_cast<size_t>(slot) * (NC + 1) + threadIdx.x];
+  __syncthreads();
+  int cs = NC, cj = 0, ce = 0;  // cursor (uniform): site of the next step, its first vertex, site end
+  auto open_site = [&](int from) {
+    cs = NC;
+    for (int r = from; r < NC; ++r)
+      if (Os[r] < Os[r + 1]) {
+        cs = r;
+        cj = Os[r];
+        ce = Os[r + 1];
+        break;
+      }
+  };
+  open_site(0);
+  C av[2], tv[2][4];
+  int sv[2];  // site of the step in the ring position (NC: none)
+  Real mv[2];
+  auto fetch = [&](int k) {
+    sv[k] = cs;
+    const int jj = cj + jl;
+    const bool j_ok = cs < NC && jj < ce;
+    const int jc = j_ok ? jj : 0;
+    mv[k] = static_cast<Real>(j_ok ? 1 : 0);
+    av[k] = Ab[pc + static_cast<size_t>(D) * jc];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
-      cr[t] = ci[t] = V{0, 0, 0, 0};
-    for (int j0 = b; j0 < e; j0 += 4) {
-      const int jj = j0 + jl;
-      const bool j_ok = jj < e;
-      const int jc = j_ok ? jj : b;
-      C a = Ab[pc + static_cast<size_t>(D) * jc];
-      if (!(j_ok && p_ok))
-        a = C{0, 0};
-      C tt[4];
+      tv[k][t] = Ts[wc[t] + static_cast<size_t>(nwE) * jc];
+    if (cs < NC) {
+      cj += 4;
+      if (cj >= ce)
+        open_site(cs + 1);
+    }
+  };
+  V cr[4], ci[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    cr[t] = ci[t] = V{0, 0, 0, 0};
+  int cur = 0;  // site being accumulated
+  // Stores the accumulated site cur and zeros for the sites without vertices up to (excluding) s.
+  auto store_to = [&](int s) {
+    for (; cur < s; ++cur) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        tt[t] = Ts[wc[t] + static_cast<size_t>(nwE) * jc];
-        if (!(j_ok && w_ok[t]))
-          tt[t] = C{0, 0};
-      }
-      // E += conj(T) A = (Tx Ax + Ty Ay) + i (Tx Ay - Ty Ax)
+        if (t >= t_lo && t < t_hi && p_ok)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        cr[t] = Mfma16<Real>::mma(tt[t].x, a.x, cr[t]);
-        ci[t] = Mfma16<Real>::mma(tt[t].x, a.y, ci[t]);
-        cr[t] = Mfma16<Real>::mma(tt[t].y, a.y, cr[t]);
-        ci[t] = Mfma16<Real>::mma(-tt[t].y, a.x, ci[t]);
+          for (int i = 0; i < 4; ++i) {
+            const int w = w0 + 16 * t + Mfma16<Real>::row(jl, i);
+            if (w < nwE)
+              Eb[pl + static_cast<size_t>(D) * (cur + NC * w)] = C{cr[t][i], ci[t][i]};
+          }
+        cr[t] = ci[t] = V{0, 0, 0, 0};
       }
     }
-    if (p_ok) {
+  };
+  fetch(0);
+  fetch(1);
+  while (sv[0] < NC) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+    for (int k = 0; k < 2; ++k) {
+      if (sv[k] < NC) {
+        if (sv[k] != cur)
+          store_to(sv[k]);
+        // Lanes past the site's vertices hold vertex 0 (finite), scaled by 0.
+        const C a{av[k].x * mv[k], av[k].y * mv[k]};
+        // E += conj(T) A = (Tx Ax + Ty Ay) + i (Tx Ay - Ty Ax)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int w = w0 + 16 * t + Mfma16<Real>::row(jl, i);
-          if (w < nwE)
-            Eb[pl + static_cast<size_t>(D) * (r + NC * w)] = C{cr[t][i], ci[t][i]};
-        }
+        for (int t = 0; t < 4; ++t)
+          if (t >= t_lo && t < t_hi) {
+            cr[t] = Mfma16<Real>::mma(tv[k][t].x, a.x, cr[t]);
+            ci[t] = Mfma16<Real>::mma(tv[k][t].x, a.y, ci[t]);
+            cr[t] = Mfma16<Real>::mma(tv[k][t].y, a.y, cr[t]);
+            ci[t] = Mfma16<Real>::mma(-tv[k][t].y, a.x, ci[t]);
+          }
+      }
+      fetch(k);
     }
   }
+  store_to(NC);
 }
 
 // One workgroup owns 64 rows p1 (one per lane) and one frequency w2. Pass 1: wave q transforms
 // the rows y = q, q + 4, ... over x into LDS; pass 2: it transforms the columns kx = q, q + 4, ...
-// over y and writes G for the L momenta (kx, ky) of each.
+// over y and writes G for the L momenta (kx, ky) of each. mirror: E holds the pairs w1 + w2 >= nwE - 1
+// only and the caller wants all of G (G0 without the conjugate symmetry): M~(-p1, -p2) =
+// conj M~(p1, p2) for real M, so each pair above that diagonal also writes its image with the image's
+// own G0 and band phases.
 template <typename Real, int L>
-__global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, int w_sum_min,
+__global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, int w_sum_min, bool mirror,
                                                    const Cplx<Real>* __restrict__ E,
                                                    const double2* __restrict__ bphase,
                                                    const double2* __restrict__ G0,
                                                    const int* __restrict__ kmap,
+                                                   const int* __restrict__ kneg,
                                                    Cplx<Real>* __restrict__ G) {
   using C = Cplx<Real>;
   constexpr int NC = L * L;
@@ -147,13 +191,19 @@ __global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, int w_sum_m
       F[(kx + L * y) * 64 + lane] = v[kx];
   }
   __syncthreads();
-  if (!p_ok)
+  const int k1 = pc % NC, w1 = pc / NC;
+  // With mirror every entry of G has one writer: pairs below the diagonal are images.
+  if (!p_ok || (mirror && w1 + w2 < g.nwE - 1))
     return;
-  const int k1 = p1 % NC, w1 = p1 / NC;
-  const double2 ga = G0[s + 2 * (k1 + static_cast<size_t>(NC) * w1)];
   const double inv_nc = 1.0 / NC;
+  auto g0 = [&](int k, int w) { return G0[s + 2 * (k + static_cast<size_t>(NC) * w)]; };
+  const double2 ga = g0(k1, w1);
   const double2 gneg{-ga.x * inv_nc, -ga.y * inv_nc};  // -G0(p1) / Nc
-  C* Gs = G + static_cast<size_t>(slot) * D * D + p1;
+  C* Gs = G + static_cast<size_t>(slot) * D * D;
+  const bool image = mirror && w1 + w2 > g.nwE - 1;
+  const int m1 = image ? kneg[k1] : 0, v1 = g.nwE - 1 - w1, v2 = g.nwE - 1 - w2;
+  const double2 gm = image ? g0(m1, v1) : double2{0, 0};
+  const double2 gmneg{-gm.x * inv_nc, -gm.y * inv_nc};
   for (int kx = wave; kx < L; kx += 4) {
     C v[L];
 #pragma unroll
@@ -166,13 +216,26 @@ __global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, int w_sum_m
       double2 m = to_d(v[ky]);
       if (bphase)
         m = cmulc(cmul(m, bphase[k1]), bphase[k2]);
-      double2 val = cmul(cmul(gneg, m), G0[s + 2 * (k2 + static_cast<size_t>(NC) * w2)]);
+      double2 val = cmul(cmul(gneg, m), g0(k2, w2));
       const int p2 = k2 + NC * w2;
       if (p1 == p2) {
         val.x = fma(ga.x, g.beta, val.x);
         val.y = fma(ga.y, g.beta, val.y);
       }
-      Gs[static_cast<size_t>(D) * p2] = from_d<C>(val);
+      Gs[p1 + static_cast<size_t>(D) * p2] = from_d<C>(val);
+      if (image) {
+        const int m2 = kneg[k2];
+        double2 c = to_d(v[ky]);
+        c.y = -c.y;
+        if (bphase)
+          c = cmulc(cmul(c, bphase[m1]), bphase[m2]);
+        double2 w = cmul(cmul(gmneg, c), g0(m2, v2));
+        if (p1 == p2) {
+          w.x = fma(gm.x, g.beta, w.x);
+          w.y = fma(gm.y, g.beta, w.y);
+        }
+        Gs[m1 + NC * v1 + static_cast<size_t>(D) * (m2 + NC * v2)] = from_d<C>(w);
+      }
     }
   }
 }
@@ -458,14 +521,15 @@ __global__ void __launch_bounds__(256) mtog_permute_m(const SlotDesc* __restrict
 }
 
 // Left half, step 1 (S1 on the matrix cores): for every site r of the sort,
-//     B[jj][r][w] = sum_{ii in site r} Ms[ii][jj] T[w, ii].
+//     B[jj][r][w] = sum_{ii in site r} Ms[ii][jj] T[w, ii],  w >= w_lo
+// (the upper half: M is real, and the lower half of A is the conjugate of the upper one).
 // A workgroup owns 64 columns jj (16 per wave) and 64 frequencies w (four 16 x 16 tiles per wave)
 // and walks the sites; a step takes four vertices of one site. Lane l supplies Ms[ii0 + l/16][jj]
 // for jj = j0 + l%16 and T[w0 + 16 t + l%16][ii0 + l/16], and holds
 // B[j0 + row(l/16, i)][r][w0 + 16 t + l%16], stored as 16-entry runs of w.
 template <typename Real, int NC>
 __global__ void __launch_bounds__(256) mtog_s1_mfma(const SlotDesc* __restrict__ desc, Geo g, int n_max,
-                                                    int slot0, const int* __restrict__ off,
+                                                    int slot0, int w_lo, const int* __restrict__ off,
                                                     const Cplx<Real>* __restrict__ T,
                                                     const Real* __restrict__ Ms, Cplx<Real>* __restrict__ B) {
   using C = Cplx<Real>;
@@ -485,7 +549,8 @@ __global__ void __launch_bounds__(256) mtog_s1_mfma(const SlotDesc* __restrict__
   const int jq = j0 + (lane & 15);
   const bool j_ok = jq < n;
   const int jc = j_ok ? jq : n - 1;
-  const int w0 = blockIdx.y * 64;
+  const int w0 = w_lo + blockIdx.y * 64;
+  const int t_hi = min(4, (nwE - w0 + 15) / 16);
   int wc[4];
   bool w_ok[4];
 #pragma unroll
@@ -499,7 +564,7 @@ __global__ void __launch_bounds__(256) mtog_s1_mfma(const SlotDesc* __restrict__
   // (clamped indices, finite data; past the stream's end a dummy step) and no load sits under a
   // branch, so the wait before a step covers only that step's loads. The lane's M value (row j,
   // step vertex i) is scaled by 0 past the site's vertices or the column count, which zeroes those
-  // products; columns past nwE (clamped T reads) are computed but not stored. A site's B rows are
+  // products; columns past nwE (clamped T reads) are not stored, and whole tiles past it not computed. A site's B rows are
   // stored when the stream moves past it (zeros for sites without vertices).
   __shared__ int Os[NC + 1];
   if (threadIdx.x <= NC)
@@ -567,10 +632,11 @@ __global__ void __launch_bounds__(256) mtog_s1_mfma(const SlotDesc* __restrict__
         if (sv[k] != cur)
           store_to(sv[k]);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          cr[t] = Mfma16<Real>::mma(mv[k], tv[k][t].x, cr[t]);
-          ci[t] = Mfma16<Real>::mma(mv[k], tv[k][t].y, ci[t]);
-        }
+        for (int t = 0; t < 4; ++t)
+          if (t < t_hi) {
+            cr[t] = Mfma16<Real>::mma(mv[k], tv[k][t].x, cr[t]);
+            ci[t] = Mfma16<Real>::mma(mv[k], tv[k][t].y, ci[t]);
+          }
       }
       fetch(k);
     }
@@ -584,24 +650,27 @@ __global__ void __launch_bounds__(256) mtog_s1_mfma(const SlotDesc* __restrict__
 // frequency, caller momentum order) is copied out through LDS as one contiguous run.
 template <typename Real, int L>
 __global__ void __launch_bounds__(256) mtog_left_site(const SlotDesc* __restrict__ desc, Geo g, int n_max,
-                                                      int slot0, const Cplx<Real>* __restrict__ B,
-                                                      const int* __restrict__ kmap, Cplx<Real>* __restrict__ A) {
+                                                      int slot0, int w_lo, const Cplx<Real>* __restrict__ B,
+                                                      const int* __restrict__ kmap, const int* __restrict__ kneg,
+                                                      Cplx<Real>* __restrict__ A) {
   using C = Cplx<Real>;
   constexpr int NC = L * L;
   __shared__ C F[NC * 64];  // [kx + L y][lane], then [k][lane]
-  __shared__ int Kl[NC];
+  __shared__ int Kl[NC], Nl[NC];
   const int slot = slot0 + blockIdx.z;
   const int jj = blockIdx.y;
   if (jj >= desc[slot].n)
     return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nwE = g.nwE;
-  const int w0 = blockIdx.x * 64;
+  const int w0 = w_lo + blockIdx.x * 64;
   const int w = w0 + lane;
   const int wc = w < nwE ? w : nwE - 1;
   const C* Bj = B + static_cast<size_t>(blockIdx.z) * g.D * n_max + static_cast<size_t>(nwE) * NC * jj + wc;
-  if (threadIdx.x < NC)
+  if (threadIdx.x < NC) {
     Kl[threadIdx.x] = kmap[threadIdx.x];
+    Nl[threadIdx.x] = kneg ? kneg[threadIdx.x] : 0;
+  }
   for (int y = wave; y < L; y += 4) {
     C v[L];
 #pragma unroll
@@ -636,10 +705,18 @@ __global__ void __launch_bounds__(256) mtog_left_site(const SlotDesc* __restrict
   }
   __syncthreads();
   const int nw = min(64, nwE - w0);
-  C* Aj = A + static_cast<size_t>(blockIdx.z) * g.D * n_max + static_cast<size_t>(g.D) * jj +
-          static_cast<size_t>(NC) * w0;
+  C* Aj = A + static_cast<size_t>(blockIdx.z) * g.D * n_max + static_cast<size_t>(g.D) * jj;
+  C* Au = Aj + static_cast<size_t>(NC) * w0;
   for (int e = threadIdx.x; e < NC * nw; e += 256)
-    Aj[e] = F[(e % NC) * 64 + e / NC];
+    Au[e] = F[(e % NC) * 64 + e / NC];
+  if (w_lo == 0)
+    return;
+  // A(-k, -w) = conj A(k, w): the mirrored run, from frequency nwE - w0 - nw on.
+  C* Am = Aj + static_cast<size_t>(NC) * (nwE - w0 - nw);
+  for (int e = threadIdx.x; e < NC * nw; e += 256) {
+    const C v = F[Nl[e % NC] * 64 + (nw - 1 - e / NC)];
+    Am[e] = C{v.x, -v.y};
+  }
 }
 
 template <typename Real, int NC>
@@ -650,10 +727,12 @@ void launch_mtog_large(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st) 
   Real* Ms = reinterpret_cast<Real*>(a.Ms);
   const int nt = (a.n_max + 63) / 64;
   hipLaunchKernelGGL((mtog_permute_m<Real>), dim3(nt, nt, ns), dim3(256), 0, st, a.desc, a.n_max, s0, a.perm, Ms);
-  hipLaunchKernelGGL((mtog_s1_mfma<Real, NC>), dim3(nt, (g.nwE + 63) / 64, ns), dim3(256), 0, st, a.desc, g,
-                     a.n_max, s0, a.off, a.T, Ms, a.B);
-  hipLaunchKernelGGL((mtog_left_site<Real, L>), dim3((g.nwE + 63) / 64, a.n_max, ns), dim3(256), 0, st, a.desc,
-                     g, a.n_max, s0, a.B, a.kmap, a.A);
+  const int w_lo = a.kneg ? g.nwE / 2 : 0;  // nwE is even
+  const int nwt = (g.nwE - w_lo + 63) / 64;
+  hipLaunchKernelGGL((mtog_s1_mfma<Real, NC>), dim3(nt, nwt, ns), dim3(256), 0, st, a.desc, g, a.n_max, s0, w_lo,
+                     a.off, a.T, Ms, a.B);
+  hipLaunchKernelGGL((mtog_left_site<Real, L>), dim3(nwt, a.n_max, ns), dim3(256), 0, st, a.desc, g, a.n_max, s0,
+                     w_lo, a.B, a.kmap, a.kneg, a.A);
   if constexpr (std::is_same<Real, float>::value) {
     // Set by the handle only where a slot's A, T and G fit 32-bit offsets.
     if (a.right_fused) {
@@ -664,10 +743,13 @@ void launch_mtog_large(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st) 
       return;
     }
   }
+  const bool mirror = a.kneg && a.w_sum_min == 0;
+  const int sum_min = mirror ? g.nwE - 1 : a.w_sum_min;
   const dim3 g3((g.D + 63) / 64, (g.nwE + 63) / 64, ns);
-  hipLaunchKernelGGL((mtog_s3_mfma<Real, NC>), g3, dim3(256), 0, st, g, a.n_max, s0, a.w_sum_min, a.off, a.T, a.A, a.E);
+  hipLaunchKernelGGL((mtog_s3_mfma<Real, NC>), g3, dim3(256), 0, st, g, a.n_max, s0, sum_min, a.off, a.T, a.A, a.E);
   const dim3 gs((g.D + 63) / 64, g.nwE, ns);
-  hipLaunchKernelGGL((mtog_site_G<Real, L>), gs, dim3(256), 0, st, g, s0, a.w_sum_min, a.E, a.bphase, a.G0, a.kmap, a.G);
+  hipLaunchKernelGGL((mtog_site_G<Real, L>), gs, dim3(256), 0, st, g, s0, sum_min, mirror, a.E, a.bphase, a.G0,
+                     a.kmap, a.kneg, a.G);
 }
 
 template void launch_mtog_large<float, 36>(const MtoGArgs<float>&, int, int, hipStream_t);

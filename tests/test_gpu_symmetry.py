@@ -95,6 +95,42 @@ def test_asymmetric_g0_takes_every_tile(oracle_lib, name, precision, tol, scale)
         assert _linf(r, x) < tol
 
 
+@pytest.mark.parametrize("name", ["6x6", "8x8"])
+@pytest.mark.parametrize("scale", [0.0, 0.3])
+def test_all_of_g_from_half_of_the_pairs(oracle_lib, name, scale):
+    """G of the FP64 6x6 and 8x8 kernels: the pairs below the anti-diagonal are images formed with
+    their own G0 (asymmetric by `scale`); an odd number of 16-frequency tiles."""
+    L, _, wex, kex, channels = CASES[name]
+    for n_freq in (2, 18, 34 if L == 6 else 20):
+        wl = synth.tiny_workload(L=L, n_freq=n_freq, w_ex=wex, k_ex=kex, channels=list(channels), n_range=(30, 90),
+                                 seed_cfg=780 + n_freq, zeeman=0.37)
+        g = wl.geometry
+        g.g0[0, 0, 0, 1, 0] *= 1.0 + scale
+        meas = wl.draw(1)[0]
+        ora = oracle_lib.OracleAccumulator(g)
+        ora.compute_G(meas)
+        acc = g4acc.TpAccumulator(g, precision="fp64", max_vertices=wl.n_max)
+        assert _linf(ora.get_G(), acc.compute_G(meas)) < 1e-12
+        acc.close()
+
+
+@pytest.mark.parametrize("nb,n_range", [(1, (0, 5)), (2, (60, 70)), (1, (500, 530)), (3, (90, 140))])
+def test_sort_order_through_g(oracle_lib, nb, n_range):
+    """The device sort at vertex counts around a wave and both workgroup sizes, empty orbitals among them
+    (FP64 G against the oracle)."""
+    wl = synth.tiny_workload(nb=nb, L=6 if n_range[0] == 500 else 2, n_freq=4, channels=[MAG], n_range=n_range,
+                             seed_cfg=790 + nb)
+    g = wl.geometry
+    for meas in wl.draw(2):
+        if sum(meas.n) == 0:
+            continue
+        ora = oracle_lib.OracleAccumulator(g)
+        ora.compute_G(meas)
+        acc = g4acc.TpAccumulator(g, precision="fp64", max_vertices=wl.n_max)
+        assert _linf(ora.get_G(), acc.compute_G(meas)) < 1e-12
+        acc.close()
+
+
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 1e-6)])
 def test_given_g_and_own_g_on_one_handle(oracle_lib, precision, tol):
     """accumulate_G (a caller's G without the conjugate symmetry) between batches of the same handle."""
