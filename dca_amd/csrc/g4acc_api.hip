@@ -102,27 +102,38 @@ struct g4acc_handle {
   bool use_band = false;           // LDS-tiled multiband G4 kernel (G4ACC_GENERIC_G4=1 disables)
   int tile_order = -1;             // G4 tile schedule (G4ACC_TILE_ORDER); -1 = by batch size
   SlotDesc* d_desc = nullptr;
-  SlotDesc* h_desc = nullptr;      // pinned
-  double* d_stage_f = nullptr;     // device staging of host inputs (M, tau)
-  int* d_stage_i = nullptr;        // (site, band)
-  double* h_stage_f = nullptr;     // pinned
-  int* h_stage_i = nullptr;
-  size_t stage_f_cap = 0, stage_i_cap = 0;
-  // Queue of g4acc_accumulate_queued: owned copies of host inputs; device inputs are copied
+  // Staging of a batch: the slot descriptors, then the walkers' host arrays one after the other, in one
+  // block, so that a batch is one copy. The device has one such block (d_desc is its start), the host
+  // two page-locked ones: the queue fills one while the other's copy may still be in flight (the second
+  // is allocated when the queue first takes host arrays).
+  struct StageBlock {
+    unsigned char* h = nullptr;
+    hipEvent_t done = nullptr;     // its last copy
+    bool pending = false;
+    SlotDesc* desc() const { return reinterpret_cast<SlotDesc*>(h); }
+  };
+  StageBlock stage[2];
+  unsigned char* d_stage = nullptr;
+  size_t stage_cap = 0, desc_bytes = 0;
+  // Queue of g4acc_accumulate_queued: host inputs are packed into a staging block, device inputs copied
   // into d_qm (M), d_qtau, d_qsb (site, band) slot by slot.
   struct Queued {
     int n[2] = {0, 0};
     double sign = 1;
-    std::vector<double> m[2], tau[2];
+    std::vector<double> tau[2];
     std::vector<int> site[2], band[2];
   };
-  std::vector<Queued> queue;
+  std::vector<Queued> queue;       // device arrays (G4ACC_DEVICE_M keeps its host configuration here)
   int queue_kind = G4ACC_HOST;
+  // Host measurements are packed where the batch's copy reads them: block q_block, q_bytes used by
+  // q_n walkers; q_error holds the first packing error, reported when the queue runs.
+  int q_block = -1, q_n = 0, q_error = G4ACC_OK, q_next = 0;
+  size_t q_bytes = 0;
+  std::string q_err_text;
   double* d_qm = nullptr;
   double* d_qtau = nullptr;
   int* d_qsb = nullptr;
-  hipEvent_t staged = nullptr;     // staging buffers free once this event completes
-  bool staged_pending = false;
+  bool dirty = true;               // kernels that may raise d_err were launched since it was read
   // Captured launch sequences, one per batch size (G4ACC_GRAPH=0 disables them).
   bool use_graph = true;
   int mtog_tw = 0;                 // tuning: frequencies per thread of the fused M -> G kernel
@@ -420,111 +431,140 @@ WalkerIn walker_in(const g4acc_handle* h, const g4acc_walker_general& w) {
   return x;
 }
 
-// Resolves the walkers of one chunk into slot descriptors; host inputs are packed into the
-// pinned staging buffer and copied once. Returns the number of slots. exp(V) values live where M
-// does; left labels where the configuration does.
-int stage_walkers(g4acc_handle* h, const WalkerIn* ws, int nw_, int memory, hipStream_t st) {
-  const int nb = h->g.nb, nc = h->g.nc;
-  // The pinned descriptor and staging buffers are reused: wait until the previous copies are done.
-  if (h->staged_pending) {
-    G4_TRY(h->check(hipEventSynchronize(h->staged), "hipEventSynchronize"));
-    h->staged_pending = false;
+// A staging block that no copy reads any more and the queue does not hold; block 1 is allocated when
+// first asked for.
+int claim_block(g4acc_handle* h, int b) {
+  g4acc_handle::StageBlock& k = h->stage[b];
+  if (!k.h) {
+    G4_TRY(h->check(hipHostMalloc(reinterpret_cast<void**>(&k.h), h->stage_cap), "hipHostMalloc"));
+    G4_TRY(h->check(hipEventCreateWithFlags(&k.done, hipEventDisableTiming), "hipEventCreate"));
   }
-  size_t of = 0, oi = 0;
-  for (int w = 0; w < nw_; ++w) {
-    const WalkerIn& wk = ws[w];
-    for (int s = 0; s < 2; ++s) {
-      SlotDesc& d = h->h_desc[2 * w + s];
-      const int n = wk.n[s];
-      d.n = n;
-      d.sign = wk.sign;
-      d.sign_im = wk.sign_im;
-      d.m_cplx = wk.m_cplx ? 1 : 0;
-      d.expv = nullptr;
-      d.site_l = d.band_l = nullptr;
-      if (n == 0) {
-        d.m = nullptr;
-        d.tau = nullptr;
-        d.site = nullptr;
-        d.band = nullptr;
-        d.ld = 1;
-        continue;
-      }
-      const size_t per = wk.m_cplx ? 2 : 1;  // doubles per element of M
-      if (!(memory & 1)) {  // M in host memory: packed column by column
-        of += of & (per - 1);  // complex entries start on a 16-byte boundary
-        double* fm = h->h_stage_f + of;
+  if (k.pending) {
+    G4_TRY(h->check(hipEventSynchronize(k.done), "hipEventSynchronize"));
+    k.pending = false;
+  }
+  return G4ACC_OK;
+}
+
+// Copies the first `bytes` of block b to `dst` and marks it in flight.
+int send_block(g4acc_handle* h, int b, void* dst, size_t bytes, hipStream_t st) {
+  G4_TRY(h->check(hipMemcpyAsync(dst, h->stage[b].h, bytes, hipMemcpyHostToDevice, st), "hipMemcpyAsync(stage)"));
+  G4_TRY(h->check(hipEventRecord(h->stage[b].done, st), "hipEventRecord"));
+  h->stage[b].pending = true;
+  return G4ACC_OK;
+}
+
+// Resolves walker w of a batch into the slot descriptors of block b, appending host arrays at byte
+// `used`. exp(V) values live where M does; left labels where the configuration does.
+int pack_walker(g4acc_handle* h, int b, int w, const WalkerIn& wk, int memory, size_t& used) {
+  const int nb = h->g.nb, nc = h->g.nc;
+  unsigned char* const hb = h->stage[b].h;
+  auto take = [&](size_t bytes, size_t& at) {
+    at = used;
+    used += bytes;
+    return hb + at;
+  };
+  for (int s = 0; s < 2; ++s) {
+    SlotDesc& d = h->stage[b].desc()[2 * w + s];
+    const int n = wk.n[s];
+    d.n = n;
+    d.sign = wk.sign;
+    d.sign_im = wk.sign_im;
+    d.m_cplx = wk.m_cplx ? 1 : 0;
+    d.expv = nullptr;
+    d.site_l = d.band_l = nullptr;
+    if (n == 0) {
+      d.m = nullptr;
+      d.tau = nullptr;
+      d.site = nullptr;
+      d.band = nullptr;
+      d.ld = 1;
+      continue;
+    }
+    size_t at;
+    used = (used + 15) / 16 * 16;
+    const size_t col = sizeof(double) * n * (wk.m_cplx ? 2 : 1);  // bytes of a column of M
+    if (!(memory & 1)) {  // M in host memory: packed column by column
+      unsigned char* fm = take(col * n, at);
+      const unsigned char* src = reinterpret_cast<const unsigned char*>(wk.m[s]);
+      if (wk.ld[s] == n)
+        std::memcpy(fm, src, col * n);
+      else
         for (int j = 0; j < n; ++j)
-          std::memcpy(fm + per * n * j, wk.m[s] + per * wk.ld[s] * j, sizeof(double) * per * n);
-        d.m = h->d_stage_f + of;
-        d.ld = n;
-        of += per * n * n;
+          std::memcpy(fm + col * j, src + col / n * wk.ld[s] * j, col);
+      d.m = reinterpret_cast<double*>(h->d_stage + at);
+      d.ld = n;
+    }
+    else {
+      d.m = wk.m[s];
+      d.ld = wk.ld[s];
+    }
+    if (wk.n_form) {
+      const double* xv = wk.expv[s];
+      if (!xv)
+        return h->fail(G4ACC_INVALID_ARG, "exp_v missing for a non-empty spin sector");
+      if (!(memory & 1)) {
+        std::memcpy(take(sizeof(double) * n, at), xv, sizeof(double) * n);
+        d.expv = reinterpret_cast<double*>(h->d_stage + at);
       }
-      else {
-        d.m = wk.m[s];
-        d.ld = wk.ld[s];
-      }
-      if (wk.n_form) {
-        const double* xv = wk.expv[s];
-        if (!xv)
-          return h->fail(G4ACC_INVALID_ARG, "exp_v missing for a non-empty spin sector");
-        if (!(memory & 1)) {
-          std::memcpy(h->h_stage_f + of, xv, sizeof(double) * n);
-          d.expv = h->d_stage_f + of;
-          of += n;
-        }
-        else
-          d.expv = xv;
-      }
-      const bool left = wk.site_l[s] != nullptr;
-      if (!(memory & 2)) {  // configuration in host memory: validated and packed
-        std::memcpy(h->h_stage_f + of, wk.tau[s], sizeof(double) * n);
-        int* im = h->h_stage_i + oi;
-        for (int i = 0; i < n; ++i) {
-          const int r = wk.site[s][i], b = wk.band[s][i];
-          if (r < 0 || r >= nc || b < 0 || b >= nb)
-            return h->fail(G4ACC_INVALID_ARG, "vertex site or band index out of range");
-          im[i] = r;
-          im[n + i] = b;
-          if (left) {
-            const int rl = wk.site_l[s][i], bl = wk.band_l[s][i];
-            if (rl < 0 || rl >= nc || bl < 0 || bl >= nb)
-              return h->fail(G4ACC_INVALID_ARG, "vertex left site or band index out of range");
-            im[2 * n + i] = rl;
-            im[3 * n + i] = bl;
-          }
-        }
-        d.tau = h->d_stage_f + of;
-        d.site = h->d_stage_i + oi;
-        d.band = h->d_stage_i + oi + n;
+      else
+        d.expv = xv;
+    }
+    const bool left = wk.site_l[s] != nullptr;
+    if (!(memory & 2)) {  // configuration in host memory: validated and packed
+      std::memcpy(take(sizeof(double) * n, at), wk.tau[s], sizeof(double) * n);
+      d.tau = reinterpret_cast<double*>(h->d_stage + at);
+      int* im = reinterpret_cast<int*>(take(sizeof(int) * (left ? 4 : 2) * n, at));
+      const int* di = reinterpret_cast<int*>(h->d_stage + at);
+      for (int i = 0; i < n; ++i) {
+        const int r = wk.site[s][i], bd = wk.band[s][i];
+        if (r < 0 || r >= nc || bd < 0 || bd >= nb)
+          return h->fail(G4ACC_INVALID_ARG, "vertex site or band index out of range");
+        im[i] = r;
+        im[n + i] = bd;
         if (left) {
-          d.site_l = h->d_stage_i + oi + 2 * n;
-          d.band_l = h->d_stage_i + oi + 3 * n;
+          const int rl = wk.site_l[s][i], bl = wk.band_l[s][i];
+          if (rl < 0 || rl >= nc || bl < 0 || bl >= nb)
+            return h->fail(G4ACC_INVALID_ARG, "vertex left site or band index out of range");
+          im[2 * n + i] = rl;
+          im[3 * n + i] = bl;
         }
-        of += n;
-        oi += (left ? 4 : 2) * static_cast<size_t>(n);
       }
-      else {
-        d.tau = wk.tau[s];
-        d.site = wk.site[s];
-        d.band = wk.band[s];
-        d.site_l = wk.site_l[s];
-        d.band_l = wk.band_l[s];
+      d.site = di;
+      d.band = di + n;
+      if (left) {
+        d.site_l = di + 2 * n;
+        d.band_l = di + 3 * n;
       }
     }
+    else {
+      d.tau = wk.tau[s];
+      d.site = wk.site[s];
+      d.band = wk.band[s];
+      d.site_l = wk.site_l[s];
+      d.band_l = wk.band_l[s];
+    }
   }
-  const int n_slots = 2 * nw_;
-  if (of)
-    G4_TRY(h->check(hipMemcpyAsync(h->d_stage_f, h->h_stage_f, of * sizeof(double),
-                                   hipMemcpyHostToDevice, st), "hipMemcpyAsync(M, tau)"));
-  if (oi)
-    G4_TRY(h->check(hipMemcpyAsync(h->d_stage_i, h->h_stage_i, oi * sizeof(int),
-                                   hipMemcpyHostToDevice, st), "hipMemcpyAsync(config)"));
-  G4_TRY(h->check(hipMemcpyAsync(h->d_desc, h->h_desc, sizeof(SlotDesc) * n_slots,
-                                 hipMemcpyHostToDevice, st), "hipMemcpyAsync(desc)"));
-  G4_TRY(h->check(hipEventRecord(h->staged, st), "hipEventRecord"));
-  h->staged_pending = true;
   return G4ACC_OK;
+}
+
+// Copies block b's descriptors of nw_ walkers, and the host arrays behind them, to the device.
+int send_walkers(g4acc_handle* h, int b, int nw_, size_t used, hipStream_t st) {
+  return send_block(h, b, h->d_stage, used > h->desc_bytes ? used : 2 * sizeof(SlotDesc) * nw_, st);
+}
+
+// The block that calls other than the queue stage in.
+int free_block(const g4acc_handle* h) { return h->q_block == 0 ? 1 : 0; }
+
+// Resolves the walkers of one chunk into slot descriptors on the device; host inputs travel with them
+// in one copy.
+int stage_walkers(g4acc_handle* h, const WalkerIn* ws, int nw_, int memory, hipStream_t st) {
+  const int b = free_block(h);
+  G4_TRY(claim_block(h, b));
+  size_t used = h->desc_bytes;
+  for (int w = 0; w < nw_; ++w)
+    G4_TRY(pack_walker(h, b, w, ws[w], memory, used));
+  return send_walkers(h, b, nw_, used, st);
 }
 
 template <typename Real>
@@ -729,6 +769,7 @@ int run_stage(g4acc_handle* h, int n_walkers, int stage, hipStream_t st) {
 // Runs the staged batch: M -> G, then the G4 update, on the handle's stream.
 int run_batch(g4acc_handle* h, int n_walkers) {
   hipStream_t st = h->stream;
+  h->dirty = true;
   if (h->timing)
     G4_TRY(h->check(hipEventRecord(h->ev[0], st), "hipEventRecord"));
   G4_TRY(run_stage(h, n_walkers, 0, st));
@@ -755,7 +796,7 @@ int run_batch(g4acc_handle* h, int n_walkers) {
 // Waits for all work of the handle.
 int quiesce(g4acc_handle* h) {
   G4_TRY(h->check(hipStreamSynchronize(h->stream), "hipStreamSynchronize"));
-  h->staged_pending = false;
+  h->stage[0].pending = h->stage[1].pending = false;
   return G4ACC_OK;
 }
 
@@ -859,8 +900,6 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
   }
   if ((rc = h->check(hipStreamCreate(&h->stream), "hipStreamCreate")) != G4ACC_OK)
     return bail(rc);
-  if ((rc = h->check(hipEventCreateWithFlags(&h->staged, hipEventDisableTiming), "hipEventCreate")) != G4ACC_OK)
-    return bail(rc);
   for (auto& e : h->ev)
     if ((rc = h->check(hipEventCreate(&e), "hipEventCreate")) != G4ACC_OK)
       return bail(rc);
@@ -929,8 +968,7 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
       (rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_A), cb * CH * NM * D, "A")) ||
       (rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_E),
                      h->fused_mtog && !h->large_e ? 1 : cb * CH * D * D, "E")) ||
-      (rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_G), cb * W2 * D * D, "G")) ||
-      (rc = h->alloc(&h->d_desc, W2, "desc")))
+      (rc = h->alloc(reinterpret_cast<unsigned char**>(&h->d_G), cb * W2 * D * D, "G")))
     return bail(rc);
   if (gm->band_phase && (rc = h->alloc(&h->d_bphase, static_cast<size_t>(g.nb) * g.nc, "band_phase")))
     return bail(rc);
@@ -1017,19 +1055,14 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
   for (auto& p : h->d_g4)
     if ((rc = h->alloc(reinterpret_cast<double2**>(&p), h->g4_entries, "G4")))
       return bail(rc);
-  // Per slot: M (or N; complex M takes two doubles per entry), tau and exp(V); right and left labels.
-  h->stage_f_cap = W2 * ((h->complex_m ? 2 : 1) * NM * NM + 2 * NM);
-  h->stage_i_cap = W2 * (h->non_dd ? 4 : 2) * NM;
-  if ((rc = h->alloc(&h->d_stage_f, h->stage_f_cap, "stage_f")) ||
-      (rc = h->alloc(&h->d_stage_i, h->stage_i_cap, "stage_i")))
+  // Per slot: M (or N; complex M takes two doubles per entry), tau and exp(V); right and left labels;
+  // 16-byte alignment.
+  h->desc_bytes = (sizeof(SlotDesc) * W2 + 15) / 16 * 16;
+  h->stage_cap = h->desc_bytes + W2 * (sizeof(double) * ((h->complex_m ? 2 : 1) * NM * NM + 2 * NM) +
+                                       sizeof(int) * (h->non_dd ? 4 : 2) * NM + 16);
+  if ((rc = h->alloc(&h->d_stage, h->stage_cap, "stage")) || (rc = claim_block(h, 0)))
     return bail(rc);
-  if ((rc = h->check(hipHostMalloc(reinterpret_cast<void**>(&h->h_desc), sizeof(SlotDesc) * W2),
-                     "hipHostMalloc")) ||
-      (rc = h->check(hipHostMalloc(reinterpret_cast<void**>(&h->h_stage_f), sizeof(double) * h->stage_f_cap),
-                     "hipHostMalloc")) ||
-      (rc = h->check(hipHostMalloc(reinterpret_cast<void**>(&h->h_stage_i), sizeof(int) * h->stage_i_cap),
-                     "hipHostMalloc")))
-    return bail(rc);
+  h->d_desc = reinterpret_cast<SlotDesc*>(h->d_stage);
 
   // Constant tables. On a square cluster the sites are relabelled x + L y (the sort orders the
   // vertices by that label and the DFT columns follow it), so the right site DFT can run as two
@@ -1091,14 +1124,12 @@ int g4acc_destroy(g4acc_handle* h) {
     (void)hipGraphExecDestroy(e.second);
   for (void* p : h->allocations)
     (void)hipFree(p);
-  if (h->h_desc)
-    (void)hipHostFree(h->h_desc);
-  if (h->h_stage_f)
-    (void)hipHostFree(h->h_stage_f);
-  if (h->h_stage_i)
-    (void)hipHostFree(h->h_stage_i);
-  if (h->staged)
-    (void)hipEventDestroy(h->staged);
+  for (auto& k : h->stage) {
+    if (k.h)
+      (void)hipHostFree(k.h);
+    if (k.done)
+      (void)hipEventDestroy(k.done);
+  }
   for (auto e : h->ev)
     if (e)
       (void)hipEventDestroy(e);
@@ -1113,6 +1144,7 @@ int g4acc_reset(g4acc_handle* h) {
     return G4ACC_INVALID_ARG;
   G4_TRY(h->check(hipSetDevice(h->device), "hipSetDevice"));
   h->queue.clear();
+  h->q_block = -1;
   for (auto* p : h->d_g4)
     launch_zero16(p, h->g4_entries, h->stream);
   if (h->sp) {
@@ -1220,6 +1252,17 @@ int g4acc_accumulate(g4acc_handle* h, const g4acc_walker* walker, int memory) {
 int g4acc_flush(g4acc_handle* h) {
   if (!h)
     return G4ACC_INVALID_ARG;
+  if (h->q_block >= 0) {  // host measurements, packed as they came
+    const int b = h->q_block, n = h->q_n;
+    h->q_block = -1;
+    if (h->q_error != G4ACC_OK)
+      return h->fail(h->q_error, h->q_err_text);
+    if (!h->g4_present)
+      return G4ACC_OK;
+    G4_TRY(h->check(hipSetDevice(h->device), "hipSetDevice"));
+    G4_TRY(send_walkers(h, b, n, h->q_bytes, h->stream));
+    return run_batch(h, n);
+  }
   if (h->queue.empty())
     return G4ACC_OK;
   const size_t NM = h->max_vertices, NM2 = NM * NM;
@@ -1239,7 +1282,7 @@ int g4acc_flush(g4acc_handle* h) {
         w.site[s] = w.band[s] = nullptr;
         continue;
       }
-      w.m[s] = kind == G4ACC_HOST ? q.m[s].data() : h->d_qm + sl * NM2;
+      w.m[s] = h->d_qm + sl * NM2;
       if (kind == G4ACC_DEVICE) {
         w.tau[s] = h->d_qtau + sl * NM;
         w.site[s] = h->d_qsb + 2 * sl * NM;
@@ -1252,7 +1295,7 @@ int g4acc_flush(g4acc_handle* h) {
       }
     }
   }
-  // The batch reads host copies before it returns and device copies in stream order, so the
+  // The batch reads host configurations before it returns and device copies in stream order, so the
   // queue slots are free for the next measurements.
   const int rc = g4acc_accumulate_batch(h, ws.data(), static_cast<int>(ws.size()), kind);
   h->queue.clear();
@@ -1273,10 +1316,27 @@ int g4acc_accumulate_queued(g4acc_handle* h, const g4acc_walker* walker, int mem
   G4_TRY(check_walker(h, w));
   if (w.n[0] + w.n[1] == 0)
     return G4ACC_OK;  // empty configuration: no-op (tp_accumulator_cpu.hpp:238-239)
-  if (!h->queue.empty() && h->queue_kind != memory)
+  if ((h->q_block >= 0 && memory != G4ACC_HOST) || (!h->queue.empty() && h->queue_kind != memory))
     G4_TRY(g4acc_flush(h));
+  if (memory == G4ACC_HOST) {
+    if (h->q_block < 0) {
+      const int b = h->q_next;
+      G4_TRY(claim_block(h, b));
+      h->q_next = 1 - b;
+      h->q_block = b;
+      h->q_n = 0;
+      h->q_bytes = h->desc_bytes;
+      h->q_error = G4ACC_OK;
+    }
+    if (h->q_error == G4ACC_OK) {
+      h->q_error = pack_walker(h, h->q_block, h->q_n, walker_in(w), memory, h->q_bytes);
+      if (h->q_error != G4ACC_OK)
+        h->q_err_text = h->err;
+    }
+    return ++h->q_n == h->max_walkers ? g4acc_flush(h) : G4ACC_OK;
+  }
   const size_t NM = h->max_vertices, NM2 = NM * NM, W2 = 2 * static_cast<size_t>(h->max_walkers);
-  if (memory != G4ACC_HOST && !h->d_qm)
+  if (!h->d_qm)
     G4_TRY(h->alloc(&h->d_qm, W2 * NM2, "queue M"));
   if (memory == G4ACC_DEVICE && !h->d_qtau) {
     G4_TRY(h->alloc(&h->d_qtau, W2 * NM, "queue tau"));
@@ -1291,16 +1351,8 @@ int g4acc_accumulate_queued(g4acc_handle* h, const g4acc_walker* walker, int mem
     if (n == 0)
       continue;
     const size_t sl = 2 * slot + s;
-    if (memory == G4ACC_HOST) {
-      q.m[s].resize(static_cast<size_t>(n) * n);
-      for (int j = 0; j < n; ++j)
-        std::memcpy(q.m[s].data() + static_cast<size_t>(n) * j, w.m[s] + static_cast<size_t>(w.ld[s]) * j,
-                    sizeof(double) * n);
-    }
-    else
-      G4_TRY(h->check(hipMemcpy2DAsync(h->d_qm + sl * NM2, sizeof(double) * n, w.m[s],
-                                       sizeof(double) * w.ld[s], sizeof(double) * n, n,
-                                       hipMemcpyDeviceToDevice, h->stream), "queue M copy"));
+    G4_TRY(h->check(hipMemcpy2DAsync(h->d_qm + sl * NM2, sizeof(double) * n, w.m[s], sizeof(double) * w.ld[s],
+                                     sizeof(double) * n, n, hipMemcpyDeviceToDevice, h->stream), "queue M copy"));
     if (memory == G4ACC_DEVICE) {
       G4_TRY(h->check(hipMemcpyAsync(h->d_qtau + sl * NM, w.tau[s], sizeof(double) * n,
                                      hipMemcpyDeviceToDevice, h->stream), "queue tau copy"));
@@ -1339,6 +1391,9 @@ int g4acc_sync(g4acc_handle* h) {
   G4_TRY(h->check(hipSetDevice(h->device), "hipSetDevice"));
   G4_TRY(g4acc_flush(h));
   G4_TRY(quiesce(h));
+  if (!h->dirty)
+    return G4ACC_OK;
+  h->dirty = false;
   int flag = 0;
   G4_TRY(h->check(hipMemcpy(&flag, h->d_err, sizeof(int), hipMemcpyDeviceToHost), "read error flag"));
   if (flag) {
@@ -1436,6 +1491,7 @@ int compute_G_impl(g4acc_handle* h, const WalkerIn& w, bool general, int memory,
   G4_TRY(h->check(hipSetDevice(h->device), "hipSetDevice"));
   G4_TRY(check_walker(h, w, general));
   G4_TRY(quiesce(h));
+  h->dirty = true;
   G4_TRY(stage_walkers(h, &w, 1, memory, h->stream));
   if (h->precision == G4ACC_FP64)
     run_mtog<double>(h, 2, h->stream, false);  // the caller gets all of G
@@ -1554,14 +1610,12 @@ int g4acc_compute_G_noalloc(g4acc_handle* h, const g4acc_walker* walker, double*
     return h->fail(G4ACC_INVALID_ARG, "compute_G_noalloc: this measurement needs " + std::to_string(l.total) +
                                           " B of workspace, more than the static " +
                                           std::to_string(G4ACC_NOALLOC_SCRATCH_BYTES) + " B");
-  // The pinned descriptor buffer is reused: wait until its previous copy has been read. Measurements
-  // queued by g4acc_accumulate_queued stay queued (their copies are not touched here).
-  if (h->staged_pending) {
-    G4_TRY(h->check(hipEventSynchronize(h->staged), "hipEventSynchronize"));
-    h->staged_pending = false;
-  }
+  // Measurements queued by g4acc_accumulate_queued stay queued (their block is not touched here).
+  const int blk = free_block(h);
+  G4_TRY(claim_block(h, blk));
+  h->dirty = true;
   for (int s = 0; s < 2; ++s) {
-    SlotDesc& d = h->h_desc[s];
+    SlotDesc& d = h->stage[blk].desc()[s];
     d.n = walker->n[s];
     d.ld = walker->ld[s];
     d.sign = walker->sign;
@@ -1574,10 +1628,7 @@ int g4acc_compute_G_noalloc(g4acc_handle* h, const g4acc_walker* walker, double*
     d.site = d.n ? walker->site[s] : nullptr;
     d.band = d.n ? walker->band[s] : nullptr;
   }
-  G4_TRY(h->check(hipMemcpyAsync(h->d_scratch + l.desc, h->h_desc, 2 * sizeof(SlotDesc), hipMemcpyHostToDevice,
-                                 h->stream), "hipMemcpyAsync(desc)"));
-  G4_TRY(h->check(hipEventRecord(h->staged, h->stream), "hipEventRecord"));
-  h->staged_pending = true;
+  G4_TRY(send_block(h, blk, h->d_scratch + l.desc, 2 * sizeof(SlotDesc), h->stream));
   if (h->precision == G4ACC_FP64)
     launch_mtog_noalloc<double>(h, l, n_max, G_dev);
   else
@@ -1601,11 +1652,14 @@ int g4acc_accumulate_G(g4acc_handle* h, const double* G_ref, double sign) {
   G4_TRY(h->check(hipMalloc(&tmp, sizeof(double2) * n), "hipMalloc(import)"));
   int rc = h->check(hipMemcpyAsync(tmp, G_ref, sizeof(double2) * n, hipMemcpyHostToDevice, h->stream),
                     "copy G");
+  const int blk = free_block(h);
+  if (rc == G4ACC_OK)
+    rc = claim_block(h, blk);
   if (rc == G4ACC_OK) {
-    h->h_desc[0] = SlotDesc{nullptr, nullptr, nullptr, nullptr, 1, 1, sign, nullptr, nullptr, nullptr, 0.0, 0};
-    h->h_desc[1] = h->h_desc[0];
-    rc = h->check(hipMemcpyAsync(h->d_desc, h->h_desc, 2 * sizeof(SlotDesc), hipMemcpyHostToDevice,
-                                 h->stream), "copy desc");
+    SlotDesc* d = h->stage[blk].desc();
+    d[0] = SlotDesc{nullptr, nullptr, nullptr, nullptr, 1, 1, sign, nullptr, nullptr, nullptr, 0.0, 0};
+    d[1] = d[0];
+    rc = send_block(h, blk, h->d_desc, 2 * sizeof(SlotDesc), h->stream);
   }
   if (rc == G4ACC_OK) {
     if (h->precision == G4ACC_FP64) {
