@@ -596,6 +596,7 @@ MtoGArgs<Real> mtog_args(g4acc_handle* h, int n_slots) {
   a.G0 = h->d_G0;
   a.grid_L = h->grid_L;
   a.kmap = h->d_kmap;
+  a.real_m = !h->complex_m;
   a.kneg = h->d_kneg;
   return a;
 }
@@ -1025,14 +1026,14 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
                   c == G4ACC_PARTICLE_HOLE_TRANSVERSE);
     h->sym_ok = ok && getenv("G4ACC_NO_SYM") == nullptr;
   }
-  // Inversion of the momenta and conjugate symmetry of G (single band, real M). Tolerances: complex64
+  // Inversion of the momenta (real M) and conjugate symmetry of G (single band). Tolerances: complex64
   // G rounds at 2^-24, so 2^-30 of G0 does not show; complex128 G allows 16 roundings of G0 itself.
-  // The DFT table enters M -> G only for clusters without the L x L transforms.
-  if (g.nb == 1 && !h->general()) {
+  // The L x L transforms of the fused kernels do not read the DFT table; the others do.
+  if (!h->complex_m) {
     const bool dp = h->precision == G4ACC_FP64;
     const double eps = 2.220446049250313e-16;
     std::vector<int> neg;
-    const bool inv = find_inversion(g, gm, dp && !h->grid_L ? 64 * eps : 1e-9, neg);
+    const bool inv = find_inversion(g, gm, dp && !(h->fused_mtog && h->grid_L) ? 64 * eps : 1e-9, neg);
     if (inv)
       table(&h->d_kneg, neg);
     if (inv && h->use_tiled && getenv("G4ACC_NO_SYM") == nullptr &&

@@ -41,7 +41,8 @@ struct MtoGArgs {
   // runs as two L-point passes; kmap[kx + L ky] is the caller's momentum index. L = 0: dense DFT.
   int grid_L;
   const int* kmap;
-  const int* kneg = nullptr;  // index(-k), where dft(-k, r) = conj dft(k, r): A(-k, -w) = conj A(k, w)
+  bool real_m = true;         // no slot holds complex M
+  const int* kneg = nullptr;  // real M: index(-k), where dft(-k, r) = conj dft(k, r): A(-k, -w) = conj A(k, w)
   // Smallest w1 + w2 (extended frequencies) the consumer reads: nwE - 1 where G is conjugate
   // symmetric and the tile kernel reads that half only, else 0. Blocks of G wholly below it are
   // neither computed nor written.
