@@ -365,6 +365,115 @@ __global__ void __launch_bounds__(256) dft_right_G_kernel(Geo g, int slot0, int 
     }
 }
 
+// S4 with the rows of E that a workgroup's Nc momenta k2 share held in LDS: it owns 64 pairs (k1, w1)
+// (one per lane) and one frequency w2, reads their n_orb columns of E once, and its waves take the
+// momenta k2 in turn (each of the kernel above reads them again: 733 us per batch of 3 bands, 8 sites, 32
+// frequencies, 32 walkers). mirror: M is real, E holds the pairs w1 + w2 >= nwE - 1 only, and
+// M~(-p1, -p2) = conj M~(p1, p2) gives each other entry of G, with its own G0 and band phases.
+template <typename Real, int NB>
+__global__ void __launch_bounds__(256) dft_right_G_shared(Geo g, int slot0, int w_sum_min, bool mirror,
+                                                          const Cplx<Real>* __restrict__ dft,
+                                                          const double2* __restrict__ bphase,
+                                                          const double2* __restrict__ G0,
+                                                          const int* __restrict__ kneg,
+                                                          const Cplx<Real>* __restrict__ E,
+                                                          Cplx<Real>* __restrict__ G) {
+  using C = Cplx<Real>;
+  constexpr int R = 64 * NB, LD = R + 1;  // rows of the block, column stride
+  extern __shared__ unsigned char smem_raw[];
+  C* El = reinterpret_cast<C*>(smem_raw);  // [column][row]
+  const int slot = slot0 + blockIdx.z;
+  const int s = slot & 1;
+  const int nc = g.nc, KW = nc * g.nwE;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int kw1 = blockIdx.x * 64 + lane, w2 = blockIdx.y;
+  if (w2 + (static_cast<int>(blockIdx.x) * 64 + 63) / nc < w_sum_min)
+    return;
+  const C* Es = E + static_cast<size_t>(blockIdx.z) * g.D * g.D + static_cast<size_t>(g.D) * g.n_orb * w2 +
+                static_cast<size_t>(blockIdx.x) * R;
+  const int rows = min(R, g.D - static_cast<int>(blockIdx.x) * R);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < g.n_orb * R; i += 256) {
+    const int row = i % R, col = i / R;
+    El[col * LD + row] = Es[(row < rows ? row : 0) + static_cast<size_t>(g.D) * col];
+  }
+  __syncthreads();
+  if (kw1 >= KW)
+    return;
+  const int k1 = kw1 % nc, w1 = kw1 / nc;
+  if (mirror && w1 + w2 < g.nwE - 1)
+    return;  // with mirror every entry of G has one writer
+  const bool image = mirror && w1 + w2 > g.nwE - 1;
+  const double inv_nc = 1.0 / nc;
+  C* Gs = G + static_cast<size_t>(slot) * g.D * g.D;
+  auto g0 = [&](int b1, int b2, int k, int w) {  // G0 index (b1, b2, s, k, w)
+    return G0[b1 + NB * (b2 + NB * (s + 2 * (k + static_cast<size_t>(nc) * w)))];
+  };
+  auto emit = [&](const double2 (&raw)[NB][NB], bool conj, int ka, int wa, int kb, int wb) {
+    double2 tmp[NB][NB];
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+      double2 mt[NB];
+#pragma unroll
+      for (int f = 0; f < NB; ++f) {
+        mt[f] = double2{raw[e][f].x, conj ? -raw[e][f].y : raw[e][f].y};
+        if (bphase)
+          mt[f] = cmulc(cmul(mt[f], bphase[e + NB * ka]), bphase[f + NB * kb]);
+      }
+#pragma unroll
+      for (int dd = 0; dd < NB; ++dd) {
+        double2 t{0, 0};
+#pragma unroll
+        for (int f = 0; f < NB; ++f)
+          cfma(t, mt[f], g0(f, dd, kb, wb));
+        tmp[e][dd] = t;
+      }
+    }
+    const bool diag = ka == kb && wa == wb;
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      double2 gl[NB];
+#pragma unroll
+      for (int e = 0; e < NB; ++e)
+        gl[e] = g0(c, e, ka, wa);
+#pragma unroll
+      for (int dd = 0; dd < NB; ++dd) {
+        double2 acc{0, 0};
+#pragma unroll
+        for (int e = 0; e < NB; ++e)
+          cfma(acc, gl[e], tmp[e][dd]);
+        acc.x = -acc.x;
+        acc.y = -acc.y;
+        if (diag) {
+          acc.x = fma(gl[dd].x, g.beta, acc.x);
+          acc.y = fma(gl[dd].y, g.beta, acc.y);
+        }
+        // value G_(c, dd, s, ka, kb, wa, wb) is stored at row (dd, ka, wa), column (c, kb, wb)
+        Gs[dd + NB * (ka + static_cast<size_t>(nc) * wa) +
+           static_cast<size_t>(g.D) * (c + NB * (kb + static_cast<size_t>(nc) * wb))] = from_d<C>(acc);
+      }
+    }
+  };
+  for (int k2 = wave; k2 < nc; k2 += 4) {
+    double2 raw[NB][NB];
+#pragma unroll
+    for (int e = 0; e < NB; ++e)
+#pragma unroll
+      for (int f = 0; f < NB; ++f) {
+        C acc{0, 0};
+#pragma unroll 8
+        for (int r2 = 0; r2 < nc; ++r2)
+          cfmac(acc, El[(f + NB * r2) * LD + e + NB * lane], dft[k2 + nc * r2]);
+        raw[e][f] = to_d(acc);
+        raw[e][f].x *= inv_nc;
+        raw[e][f].y *= inv_nc;
+      }
+    emit(raw, false, k1, w1, k2, w2);
+    if (image)
+      emit(raw, true, kneg[k1], g.nwE - 1 - w1, kneg[k2], g.nwE - 1 - w2);
+  }
+}
+
 // M = diag(exp(V) - 1) N: the M matrix a CT-AUX walker hands to the accumulator
 // (CtauxWalker::computeM, ctaux_walker.hpp:1889-1916, which forms exp(V_i) - 1 per vertex and
 // scales the rows of N, src/linalg/lapack/multiply_diagonal_gpu.cu). One thread per entry, rows
@@ -427,8 +536,28 @@ void launch_mtog(const MtoGArgs<Real>& a, hipStream_t st) {
       hipLaunchKernelGGL(dft_left_kernel<Real>, dim3((g.D + 255) / 256, a.n_max, ns), dim3(256), 0, st,
                          a.desc, g, a.n_max, s0, a.dft, a.B, a.A);
     }
+    // S4 from LDS where a block's rows of E fit half of a CU's; with real M and the momenta's inverses S3
+    // then forms half of the frequency pairs.
+    const size_t el = sizeof(Cplx<Real>) * g.n_orb * (64 * static_cast<size_t>(g.nb) + 1);
+    const bool shared = el <= 81920;
+    const bool mirror = shared && a.real_m && a.kneg && a.w_sum_min == 0;
+    const int sum_min = mirror ? g.nwE - 1 : a.w_sum_min;
     hipLaunchKernelGGL(ndft_right_kernel<Real>, dim3((g.D + 255) / 256, g.D, ns), dim3(256), 0, st,
-                       a.desc, g, a.n_max, s0, a.w_sum_min, a.off2, a.T2, a.A, a.E);
+                       a.desc, g, a.n_max, s0, sum_min, a.off2, a.T2, a.A, a.E);
+    if (shared) {
+      const dim3 gs((g.nc * g.nwE + 63) / 64, g.nwE, ns);
+      auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, gs, dim3(256), el, st, g, s0, sum_min, mirror, a.dft, a.bphase, a.G0, a.kneg, a.E,
+                           a.G);
+      };
+      switch (g.nb) {
+        case 1: run(dft_right_G_shared<Real, 1>); break;
+        case 2: run(dft_right_G_shared<Real, 2>); break;
+        case 3: run(dft_right_G_shared<Real, 3>); break;
+        default: run(dft_right_G_shared<Real, 4>); break;
+      }
+      continue;
+    }
     const int KW = g.nc * g.nwE;
     const dim3 grid((KW + 255) / 256, KW, ns);
     switch (g.nb) {
