@@ -85,10 +85,8 @@ struct PairShape {
 // G4[i] += v in two steps, so that a thread's loads are all issued before its stores.
 __device__ __forceinline__ void g4_put(void* g4, size_t i, float4 old, double2 acc, int sum_mode) {
   if (sum_mode == SUM_FP64) {
-    double2 v = *reinterpret_cast<double2*>(&old);
-    v.x += acc.x;
-    v.y += acc.y;
-    static_cast<double2*>(g4)[i] = v;
+    static_cast<double2*>(g4)[i] = double2{__hiloint2double(__float_as_int(old.y), __float_as_int(old.x)) + acc.x,
+                                           __hiloint2double(__float_as_int(old.w), __float_as_int(old.z)) + acc.y};
   }
   else {
     float4 v = old;
@@ -149,6 +147,10 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
   int w1, w2, z;
   if (!tile_coords(a, w1, w2, z))
     return;
+  // Channel tables by select: a run-time index would put the arguments in scratch memory, whose loads
+  // wait behind the G4 loads and stores in flight.
+  auto ch_of = [&](int c) { return c == 0 ? a.ch[0] : c == 1 ? a.ch[1] : c == 2 ? a.ch[2] : a.ch[3]; };
+  auto g4_of = [&](int c) { return c == 0 ? a.g4[0] : c == 1 ? a.g4[1] : c == 2 ? a.g4[2] : a.g4[3]; };
   const int iv = z / a.nqg, q0 = (z % a.nqg) * QG;
   const int nu = a.w_ex[iv];
   const int ld = nc + 1, bs = nc * ld, ncc = nc * nc;
@@ -177,7 +179,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
   // (pair 0 for idle ones). It loads X, Y and Z at the same idx.
   bool ok[PPT];
   unsigned xo[PPT], yo[PPT], zo[PPT];
-  int li[PPT];
+  int li[PPT], kk[PPT];  // LDS place; k1 | k2 << 16
   int yz[PPT][QG];  // LDS places of Y^q and Z^q, 16 bits each (bs <= 64 * 65)
 #pragma unroll
   for (int j = 0; j < PPT; ++j) {
@@ -188,6 +190,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
     yo[j] = element(k1, k2, ym);
     zo[j] = element(k1, k2, zm);
     li[j] = k2 * ld + k1;
+    kk[j] = k1 | (k2 << 16);
 #pragma unroll
     for (int qi = 0; qi < QG; ++qi) {
       const int q = a.k_ex[q0 + qi < g.nq ? q0 + qi : 0];
@@ -329,15 +332,15 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
     return ka + static_cast<size_t>(nc) *
                     (wa + static_cast<size_t>(nw) * (kb + static_cast<size_t>(nc) * (wb + static_cast<size_t>(nw) * qv)));
   };
-  // Index arithmetic below starts from an opaque copy of the thread id per group of entries: held
-  // for all pairs at once it would not fit beside the totals.
-  auto own_index = [&](int tid, int j, int qv) {
-    const int idx = tid + TT * j;
-    return g4_index(idx % nc, w1, idx / nc, w2, qv);
+  // Index arithmetic below starts from an opaque copy of k1 and k2 per group of entries: held for all
+  // entries at once it would not fit beside the totals.
+  auto own_index = [&](int kp, int qv) { return g4_index(kp & 0xffff, w1, kp >> 16, w2, qv); };
+  auto swap_index = [&](int kp, int qv, int q) {
+    return g4_index(a.k_sub[(kp & 0xffff) + nc * q], p1, a.k_sub[(kp >> 16) + nc * q], p2, qv);
   };
-  auto swap_index = [&](int tid, int j, int qv, int q) {
-    const int idx = tid + TT * j;
-    return g4_index(a.k_sub[idx % nc + nc * q], p1, a.k_sub[idx / nc + nc * q], p2, qv);
+  auto opaque = [](int v) {
+    asm volatile("" : "+v"(v));
+    return v;
   };
   // Below four walkers a matrix-core step would be mostly padding, and the launch is the G4
   // read-modify-write: each thread forms its entries' rank-one terms itself (to its own LDS places,
@@ -345,9 +348,8 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
   const bool direct = n_walk < 4;
   const size_t uv_row = static_cast<size_t>(g.nq) * g.nv * P;  // between the planes of one walker
   auto rank_one = [&](int j, int qv, int pl) {
-    const int idx = threadIdx.x + TT * j;
-    const C* U = a.UV + pl * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w1) + idx % nc;
-    const C* V = a.UV + (pl + 2) * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w2) + idx / nc;
+    const C* U = a.UV + pl * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w1) + (kk[j] & 0xffff);
+    const C* V = a.UV + (pl + 2) * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w2) + (kk[j] >> 16);
     double2 r{0, 0};
     for (int m = 0; m < n_walk; ++m)
       cfma(r, to_d(V[4 * uv_row * m]), to_d(U[4 * uv_row * m]));
@@ -367,21 +369,21 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
     const int c_hi = kOneCh ? c_lo + 1 : a.n_ch;
     int n_ph = 0, n_r = 0;  // particle-hole channels, and those of them with a rank-one term
     for (int c = c_lo; c < c_hi; ++c) {
-      n_ph += a.ch[c] != PP_UP_DOWN;
-      n_r += a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE;
+      n_ph += ch_of(c) != PP_UP_DOWN;
+      n_r += ch_of(c) == PH_MAGNETIC || ch_of(c) == PH_CHARGE;
     }
     __syncthreads();
     if (HX && n_r > 0 && direct) {
       int ph = 0;
-      for (int c = c_lo; c < c_hi; ph += a.ch[c] != PP_UP_DOWN, ++c)
-        if (a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE)
+      for (int c = c_lo; c < c_hi; ph += ch_of(c) != PP_UP_DOWN, ++c)
+        if (ch_of(c) == PH_MAGNETIC || ch_of(c) == PH_CHARGE)
 #pragma unroll
           for (int r = 0; r < RB; ++r)
 #pragma unroll
             for (int j = 0; j < PPT; ++j)
               if (r < nr && ok[j])
                 Rl[(r * n_ph + ph) * bs + li[j]] =
-                    rank_one(j, q0 + r0 + r + g.nq * iv, a.ch[c] == PH_MAGNETIC ? 0 : 1);
+                    rank_one(j, q0 + r0 + r + g.nq * iv, ch_of(c) == PH_MAGNETIC ? 0 : 1);
     }
     else if (HX && n_r > 0) {
       // R(k2, k1) blocks of 16 x 16: lane l supplies V[m0 + l/16][k2] and U[m0 + l/16][k1] and holds
@@ -397,13 +399,13 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
         const int ta = it % nt, tb = (it / nt) % nt, cr = (it / (nt * nt)) % n_r, rq = it / (nt * nt * n_r);
         int c = c_lo, ph = 0;  // the cr-th channel with a rank-one term
         for (int left = cr;; ++c) {
-          const bool has = a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE;
+          const bool has = ch_of(c) == PH_MAGNETIC || ch_of(c) == PH_CHARGE;
           if (has && left-- == 0)
             break;
-          ph += a.ch[c] != PP_UP_DOWN;
+          ph += ch_of(c) != PP_UP_DOWN;
         }
         const int k1 = ta * 16 + (lane & 15), k2 = tb * 16 + (lane & 15), kl = lane >> 4;
-        const int pl = a.ch[c] == PH_MAGNETIC ? 0 : 1;
+        const int pl = ch_of(c) == PH_MAGNETIC ? 0 : 1;
         const C* U = a.UV + pl * row + static_cast<size_t>(q0 + r0 + rq + g.nq * iv) * P +
                      nc * static_cast<size_t>(w1) + (k1 < nc ? k1 : 0);
         const C* V = a.UV + (pl + 2) * row + static_cast<size_t>(q0 + r0 + rq + g.nq * iv) * P +
@@ -458,8 +460,10 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
     for (int c0 = c_lo; c0 < c_hi; c0 += CG) {
 #pragma unroll
       for (int i0 = 0; i0 < RB * PPT; i0 += GS) {
-        int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
+        int kp[GS];
+#pragma unroll
+        for (int i = 0; i < GS; ++i)
+          kp[i] = opaque(kk[(i0 + i) % PPT]);
         float4 old[CG][GS], oldp[HZ ? GS : 1];  // at most one pp channel
 #pragma unroll
         for (int k = 0; k < CG; ++k)
@@ -470,18 +474,18 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
               if (r >= nr || !ok[j])
                 continue;
               const int qv = q0 + r0 + r + g.nq * iv;
-              old[k][i] = static_cast<const float4*>(a.g4[c0 + k])[own_index(tid, j, qv)];
-              if (img_p && a.ch[c0 + k] == PP_UP_DOWN)
+              old[k][i] = static_cast<const float4*>(g4_of(c0 + k))[own_index(kp[i], qv)];
+              if (img_p && ch_of(c0 + k) == PP_UP_DOWN)
                 oldp[HZ ? i : 0] =
-                    static_cast<const float4*>(a.g4[c0 + k])[swap_index(tid, j, qv, a.k_ex[q0 + r0 + r])];
+                    static_cast<const float4*>(g4_of(c0 + k))[swap_index(kp[i], qv, a.k_ex[q0 + r0 + r])];
             }
         int ph = ph0;
 #pragma unroll
         for (int k = 0; k < CG; ++k)
           if (c0 + k < c_hi) {
-            const int type = a.ch[c0 + k];
+            const int type = ch_of(c0 + k);
             const bool is_pp = HZ && type == PP_UP_DOWN;
-            void* g4 = a.g4[c0 + k];
+            void* g4 = g4_of(c0 + k);
 #pragma unroll
             for (int i = 0; i < GS; ++i) {
               const int r = (i0 + i) / PPT, j = (i0 + i) % PPT;
@@ -498,17 +502,17 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
               }
               else
                 v = double2{-tt[j][r0 + r].x, -tt[j][r0 + r].y};
-              g4_put(g4, own_index(tid, j, qv), old[k][i], v, a.sum_mode);
+              g4_put(g4, own_index(kp[i], qv), old[k][i], v, a.sum_mode);
               if (!is_pp && (img_t || img_c))
                 Rl[(r * n_ph + ph) * bs + li[j]] = v;
               if (is_pp && img_p)
-                g4_put(g4, swap_index(tid, j, qv, a.k_ex[q0 + r0 + r]), oldp[HZ ? i : 0], v, a.sum_mode);
+                g4_put(g4, swap_index(kp[i], qv, a.k_ex[q0 + r0 + r]), oldp[HZ ? i : 0], v, a.sum_mode);
             }
             ph += !is_pp;
           }
       }
       for (int k = 0; k < CG && c0 + k < c_hi; ++k)
-        ph0 += a.ch[c0 + k] != PP_UP_DOWN;
+        ph0 += ch_of(c0 + k) != PP_UP_DOWN;
     }
     if (n_ph == 0 || (!img_t && !img_c))
       continue;
@@ -522,29 +526,30 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
       for (int c0 = c_lo; c0 < c_hi; c0 += CG) {
 #pragma unroll
         for (int i0 = 0; i0 < RB * PPT; i0 += GS) {
-          int tid = threadIdx.x;
-          asm volatile("" : "+v"(tid));
+          int kp[GS];
+#pragma unroll
+          for (int i = 0; i < GS; ++i)
+            kp[i] = opaque(kk[(i0 + i) % PPT]);
           float4 old[CG][GS];
 #pragma unroll
           for (int k = 0; k < CG; ++k)
-            if (c0 + k < c_hi && a.ch[c0 + k] != PP_UP_DOWN)
+            if (c0 + k < c_hi && ch_of(c0 + k) != PP_UP_DOWN)
 #pragma unroll
               for (int i = 0; i < GS; ++i) {
-                const int r = (i0 + i) / PPT, j = (i0 + i) % PPT, idx = tid + TT * j;
+                const int r = (i0 + i) / PPT, j = (i0 + i) % PPT;
                 if (r < nr && ok[j])
-                  old[k][i] = static_cast<const float4*>(
-                      a.g4[c0 + k])[g4_index(idx % nc, wa, idx / nc, wb, q0 + r0 + r + g.nq * iv)];
+                  old[k][i] = static_cast<const float4*>(g4_of(c0 + k))[g4_index(kp[i] & 0xffff, wa, kp[i] >> 16, wb, q0 + r0 + r + g.nq * iv)];
               }
           int ph = ph0;
 #pragma unroll
           for (int k = 0; k < CG; ++k)
-            if (c0 + k < c_hi && a.ch[c0 + k] != PP_UP_DOWN) {
+            if (c0 + k < c_hi && ch_of(c0 + k) != PP_UP_DOWN) {
 #pragma unroll
               for (int i = 0; i < GS; ++i) {
                 const int r = (i0 + i) / PPT, j = (i0 + i) % PPT;
                 if (r >= nr || !ok[j])
                   continue;
-                const int idx = tid + TT * j, k1 = idx % nc, k2 = idx / nc;
+                const int k1 = kp[i] & 0xffff, k2 = kp[i] >> 16;
                 const int q = a.k_ex[q0 + r0 + r];
                 int s1, s2;
                 if (kind == 0) {
@@ -562,13 +567,13 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
                 double2 v = Rl[(r * n_ph + ph) * bs + s2 * ld + s1];
                 if (kind != 0)
                   v.y = -v.y;
-                g4_put(a.g4[c0 + k], g4_index(k1, wa, k2, wb, q0 + r0 + r + g.nq * iv), old[k][i], v, a.sum_mode);
+                g4_put(g4_of(c0 + k), g4_index(k1, wa, k2, wb, q0 + r0 + r + g.nq * iv), old[k][i], v, a.sum_mode);
               }
               ++ph;
             }
         }
         for (int k = 0; k < CG && c0 + k < c_hi; ++k)
-          ph0 += a.ch[c0 + k] != PP_UP_DOWN;
+          ph0 += ch_of(c0 + k) != PP_UP_DOWN;
       }
     }
     }

@@ -648,7 +648,9 @@ void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
     // for 64 measurements); from two walkers on the tiles' reads and products count.
     a.half_g = own_g && h->half_g();
     a.sym_few = h->g4_sym && h->sym_ok ? SYM_TRANSPOSE : SYM_NONE;
-    a.sym = a.half_g && n_walkers > 1 ? h->conj_sym : a.sym_few;
+    // Where the transpose images are written anyway, the conjugate ones cost nothing more and half of G
+    // less is read.
+    a.sym = a.half_g && (n_walkers > 1 || a.sym_few == SYM_TRANSPOSE) ? h->conj_sym : a.sym_few;
     a.k_neg = h->d_kneg;
     a.sym_tiles = h->d_stab[a.tile_order == 0 ? 0 : 1];
     a.n_sym_tiles = h->n_stab;

@@ -252,11 +252,14 @@ __global__ void __launch_bounds__(256) ndft_right_kernel(const SlotDesc* __restr
   using C = Cplx<Real>;
   const int slot = slot0 + blockIdx.z;
   const int q2 = blockIdx.y;
-  const int p1 = blockIdx.x * blockDim.x + threadIdx.x;
+  // Rows rotate with the column: those with few needed pairs would otherwise all run on the same XCDs
+  // (workgroups are dealt to them round-robin).
+  const int bx = (blockIdx.x + blockIdx.y) % gridDim.x;
+  const int p1 = bx * blockDim.x + threadIdx.x;
   if (p1 >= g.D)
     return;
   const int o2 = q2 % g.n_orb, w2 = q2 / g.n_orb;
-  if (w2 + (static_cast<int>(blockIdx.x) * 256 + 255) / g.n_orb < w_sum_min)
+  if (w2 + (bx * 256 + 255) / g.n_orb < w_sum_min)
     return;
   const int* O = off + static_cast<size_t>(slot) * (g.n_orb + 1);
   const C* Ts = T + static_cast<size_t>(slot) * g.nwE * n_max;
