@@ -18,12 +18,12 @@
 // instructions per walker and no buffer of G4's size.
 //
 // What bounds it: the blocks read from L2 and beyond (4x4, three channels, 256 walkers, 64
-// frequencies, 4 q, 3 v: 20 GB in 2.9 ms; the same block pattern alone reads 7.4 TB/s), with the
+// frequencies, 4 q, 3 v: 20 GB in 2.8 ms; the same block pattern alone reads 7.4 TB/s), with the
 // vector ALUs 60 % busy beside it. So each block is read once per walker for all the momenta whose
 // totals fit the registers. The next walkers' loads are in flight during a walker's products; every
 // load is issued (idle slots and walkers past the batch re-read valid elements).
 // Per batch (256 walkers) the stage went from 3.64 ms, with the rank-one terms in a buffer of G4's
-// size, to 3.0 ms; 6x6 (64 walkers, 64 frequencies, 4 q, 2 v) from 10.6 to 4.8 ms.
+// size, to 2.9 ms; 6x6 (64 walkers, 64 frequencies, 4 q, 2 v) from 10.6 to 4.6 ms.
 // Products are formed in the G precision; with complex64 G, 256-thread tiles sum eight walkers in
 // FP32 before the FP64 totals, larger tiles (whose registers hold the totals) add every walker.
 // G4 is read and written once per launch (FP64, or FP32 value + Kahan compensation).
@@ -69,7 +69,7 @@ constexpr int HAS_X = 1, HAS_Z = 2, HAS_T = 4;
 
 // Registers of a workgroup's threads. 704 threads hold 33..37-site clusters with two pairs each:
 // eleven waves leave 168 registers, enough for the totals of four momenta (6x6, magnetic and pp, 64
-// walkers, 64 frequencies: 4.8 ms per batch; two momenta 6.2, two in 1024 threads 7.6, since each
+// walkers, 64 frequencies: 4.6 ms per batch; two momenta 6.2, two in 1024 threads 7.6, since each
 // group of momenta reads the blocks again).
 template <typename Real, int TT, int PPT, int QG>
 struct PairShape {
@@ -82,7 +82,7 @@ struct PairShape {
   static constexpr bool HOLD = fp32 || TT == 256;
 };
 
-// G4[i] += v in two steps, so that a thread's loads are all issued before its stores.
+// G4[i] += v in two steps, so that a thread's loads are issued ahead of its stores.
 __device__ __forceinline__ void g4_put(void* g4, size_t i, float4 old, double2 acc, int sum_mode) {
   if (sum_mode == SUM_FP64) {
     static_cast<double2*>(g4)[i] = double2{__hiloint2double(__float_as_int(old.y), __float_as_int(old.x)) + acc.x,
