@@ -102,21 +102,44 @@ struct g4acc_handle {
   bool use_band = false;           // LDS-tiled multiband G4 kernel (G4ACC_GENERIC_G4=1 disables)
   int tile_order = -1;             // G4 tile schedule (G4ACC_TILE_ORDER); -1 = by batch size
   SlotDesc* d_desc = nullptr;
-  // Staging of a batch: the slot descriptors, then the walkers' host arrays one after the other, in one
-  // block, so that a batch is one copy. The device has one such block (d_desc is its start), the host
-  // two page-locked ones: the queue fills one while the other's copy may still be in flight (the second
-  // is allocated when the queue first takes host arrays).
-  struct StageBlock {
-    unsigned char* h = nullptr;
+  // Staging of a batch: slot descriptors (d_desc) and the walkers' host arrays, one after the other,
+  // packed into two small page-locked pieces. A batch that fits one piece is one copy on the handle's stream,
+  // descriptors and arrays together. A larger one goes to a device block of its own on a copy stream, piece by
+  // piece: one piece is filled while the other's copy runs, beside the kernels of the batch before.
+  // Page-locked memory costs its first touch as well as its allocation. 4x4, four batches of 32 queued
+  // measurements (14 MB each), first and later phases: 9.5 and 7.6 ms through pageable copies and a block of
+  // a whole batch, 10 - 12 and 4.3 through two such blocks, 5.9 and 3.6 through these pieces.
+  struct StagePiece {
+    unsigned char* h = nullptr;    // descriptors (desc_bytes), then arrays (piece_bytes)
     hipEvent_t done = nullptr;     // its last copy
     bool pending = false;
     SlotDesc* desc() const { return reinterpret_cast<SlotDesc*>(h); }
   };
-  StageBlock stage[2];
-  unsigned char* d_stage = nullptr;
-  size_t stage_cap = 0, desc_bytes = 0;
-  // Queue of g4acc_accumulate_queued: host inputs are packed into a staging block, device inputs copied
-  // into d_qm (M), d_qtau, d_qsb (site, band) slot by slot.
+  StagePiece piece[2];
+  unsigned char* h_stage = nullptr;  // both pieces
+  size_t host_bytes = 0;
+  unsigned char* d_stage = nullptr;  // descriptors, then the arrays of a batch of one piece
+  size_t arrays_cap = 0, desc_bytes = 0, piece_bytes = 0;
+  // Blocks of arrays_cap bytes for larger batches; free once the kernels that read them are through.
+  struct StageBlock {
+    unsigned char* d = nullptr;
+    hipEvent_t read = nullptr;     // after the kernels that read it last (pending: recorded)
+    bool pending = false;
+  };
+  StageBlock block[2];
+  hipStream_t copy_stream = nullptr;
+  hipEvent_t copied = nullptr;
+  int next_block = 0, run_block = -1;  // run_block: read by the batch staged last
+  // A batch being staged: its descriptors (host arrays as byte offsets), the piece that is being filled
+  // (-1: none), the bytes in it, those sent before it and the block they went to (-1: none sent).
+  struct Fill {
+    std::vector<SlotDesc> desc;
+    int piece = -1, block = -1, n = 0, memory = 0;
+    size_t used = 0, sent = 0;
+  };
+  Fill direct;                     // calls other than the queue's, staged whole before they return
+  // Queue of g4acc_accumulate_queued: host inputs are packed into the staging pieces when they are handed
+  // over, device inputs copied into d_qm (M), d_qtau, d_qsb (site, band) slot by slot.
   struct Queued {
     int n[2] = {0, 0};
     double sign = 1;
@@ -125,10 +148,10 @@ struct g4acc_handle {
   };
   std::vector<Queued> queue;       // device arrays (G4ACC_DEVICE_M keeps its host configuration here)
   int queue_kind = G4ACC_HOST;
-  // Host measurements are packed where the batch's copy reads them: block q_block, q_bytes used by
-  // q_n walkers; q_error holds the first packing error, reported when the queue runs.
-  int q_block = -1, q_n = 0, q_error = G4ACC_OK, q_next = 0;
-  size_t q_bytes = 0;
+  // Host measurements handed over (q_walkers of them), the piece that the next batch starts with, and
+  // the first packing error, reported when the queue runs.
+  Fill q;
+  int q_walkers = 0, q_next = 0, q_error = G4ACC_OK;
   std::string q_err_text;
   double* d_qm = nullptr;
   double* d_qtau = nullptr;
@@ -431,14 +454,9 @@ WalkerIn walker_in(const g4acc_handle* h, const g4acc_walker_general& w) {
   return x;
 }
 
-// A staging block that no copy reads any more and the queue does not hold; block 1 is allocated when
-// first asked for.
-int claim_block(g4acc_handle* h, int b) {
-  g4acc_handle::StageBlock& k = h->stage[b];
-  if (!k.h) {
-    G4_TRY(h->check(hipHostMalloc(reinterpret_cast<void**>(&k.h), h->stage_cap), "hipHostMalloc"));
-    G4_TRY(h->check(hipEventCreateWithFlags(&k.done, hipEventDisableTiming), "hipEventCreate"));
-  }
+// Waits until no copy reads piece b any more.
+int claim_piece(g4acc_handle* h, int b) {
+  g4acc_handle::StagePiece& k = h->piece[b];
   if (k.pending) {
     G4_TRY(h->check(hipEventSynchronize(k.done), "hipEventSynchronize"));
     k.pending = false;
@@ -446,26 +464,88 @@ int claim_block(g4acc_handle* h, int b) {
   return G4ACC_OK;
 }
 
-// Copies the first `bytes` of block b to `dst` and marks it in flight.
-int send_block(g4acc_handle* h, int b, void* dst, size_t bytes, hipStream_t st) {
-  G4_TRY(h->check(hipMemcpyAsync(dst, h->stage[b].h, bytes, hipMemcpyHostToDevice, st), "hipMemcpyAsync(stage)"));
-  G4_TRY(h->check(hipEventRecord(h->stage[b].done, st), "hipEventRecord"));
-  h->stage[b].pending = true;
+// Marks piece b in flight, after its copies.
+int piece_sent(g4acc_handle* h, int b, hipStream_t st) {
+  G4_TRY(h->check(hipEventRecord(h->piece[b].done, st), "hipEventRecord"));
+  h->piece[b].pending = true;
   return G4ACC_OK;
 }
 
-// Resolves walker w of a batch into the slot descriptors of block b, appending host arrays at byte
-// `used`. exp(V) values live where M does; left labels where the configuration does.
-int pack_walker(g4acc_handle* h, int b, int w, const WalkerIn& wk, int memory, size_t& used) {
+// Copies `bytes` of piece b, from its start, to `dst`.
+int send_piece(g4acc_handle* h, int b, void* dst, size_t bytes, hipStream_t st) {
+  G4_TRY(h->check(hipMemcpyAsync(dst, h->piece[b].h, bytes, hipMemcpyHostToDevice, st), "hipMemcpyAsync(stage)"));
+  return piece_sent(h, b, st);
+}
+
+// The piece that a call other than the queue's starts with: one that the queue does not hold.
+int free_piece(const g4acc_handle* h) { return h->q.piece == 0 ? 1 : 0; }
+
+// The kernels launched so far have read the block of the batch staged last.
+int release_block(g4acc_handle* h) {
+  if (h->run_block < 0)
+    return G4ACC_OK;
+  const int b = h->run_block;
+  h->run_block = -1;
+  h->block[b].pending = true;
+  return h->check(hipEventRecord(h->block[b].read, h->stream), "hipEventRecord");
+}
+
+// Chooses a device block for batch f, whose copies wait for the kernels that read it last.
+int open_block(g4acc_handle* h, g4acc_handle::Fill& f) {
+  const bool beside = &f != &h->q && h->q.block >= 0;  // the queue holds the other one
+  int b = beside ? 1 - h->q.block : h->next_block;
+  if (!h->copy_stream) {
+    G4_TRY(h->check(hipEventCreateWithFlags(&h->copied, hipEventDisableTiming), "hipEventCreate"));
+    for (auto& k : h->block)
+      G4_TRY(h->check(hipEventCreateWithFlags(&k.read, hipEventDisableTiming), "hipEventCreate"));
+    G4_TRY(h->check(hipStreamCreate(&h->copy_stream), "hipStreamCreate"));
+  }
+  if (!h->block[b].d) {
+    const int rc = h->alloc(&h->block[b].d, h->arrays_cap, "stage block");
+    if (rc != G4ACC_OK && (beside || !h->block[1 - b].d))
+      return rc;
+    if (rc != G4ACC_OK)
+      b = 1 - b;  // no room for a second one: copies wait for the batch before
+  }
+  if (h->run_block == b)
+    G4_TRY(release_block(h));
+  if (h->block[b].pending)
+    G4_TRY(h->check(hipStreamWaitEvent(h->copy_stream, h->block[b].read, 0), "hipStreamWaitEvent"));
+  h->next_block = 1 - b;
+  f.block = b;
+  return G4ACC_OK;
+}
+
+// Sends the arrays of the piece being filled to the batch's block.
+int send_arrays(g4acc_handle* h, g4acc_handle::Fill& f) {
+  const int b = f.piece;
+  G4_TRY(h->check(hipMemcpyAsync(h->block[f.block].d + f.sent, h->piece[b].h + h->desc_bytes, f.used,
+                                 hipMemcpyHostToDevice, h->copy_stream), "hipMemcpyAsync(arrays)"));
+  G4_TRY(piece_sent(h, b, h->copy_stream));
+  f.sent += f.used;
+  f.used = 0;
+  return G4ACC_OK;
+}
+
+// Sends the piece being filled and moves on to the other one, or to the same one again where the queue
+// holds the other.
+int next_piece(g4acc_handle* h, g4acc_handle::Fill& f) {
+  const int next = &f != &h->q && h->q.piece >= 0 ? f.piece : 1 - f.piece;
+  if (f.block < 0)
+    G4_TRY(open_block(h, f));
+  G4_TRY(send_arrays(h, f));
+  G4_TRY(claim_piece(h, next));
+  f.piece = next;
+  return G4ACC_OK;
+}
+
+// Appends walker wk to the batch f: its slot descriptors, and its host arrays in the pieces. exp(V)
+// values live where M does; left labels where the configuration does.
+int pack_walker(g4acc_handle* h, g4acc_handle::Fill& f, const WalkerIn& wk) {
+  const int memory = f.memory;
   const int nb = h->g.nb, nc = h->g.nc;
-  unsigned char* const hb = h->stage[b].h;
-  auto take = [&](size_t bytes, size_t& at) {
-    at = used;
-    used += bytes;
-    return hb + at;
-  };
   for (int s = 0; s < 2; ++s) {
-    SlotDesc& d = h->stage[b].desc()[2 * w + s];
+    SlotDesc& d = f.desc[2 * f.n + s];
     const int n = wk.n[s];
     d.n = n;
     d.sign = wk.sign;
@@ -481,41 +561,54 @@ int pack_walker(g4acc_handle* h, int b, int w, const WalkerIn& wk, int memory, s
       d.ld = 1;
       continue;
     }
-    size_t at;
-    used = (used + 15) / 16 * 16;
-    const size_t col = sizeof(double) * n * (wk.m_cplx ? 2 : 1);  // bytes of a column of M
+    const double* xv = wk.n_form ? wk.expv[s] : nullptr;
+    if (wk.n_form && !xv)
+      return h->fail(G4ACC_INVALID_ARG, "exp_v missing for a non-empty spin sector");
+    const bool left = wk.site_l[s] != nullptr;
+    // The slot's bytes, at most slot_bytes() and so within a piece.
+    const size_t col = sizeof(double) * n * (wk.m_cplx ? 2 : 1);  // of a column of M
+    size_t need = 0;
+    if (!(memory & 1))
+      need += col * n + (xv ? sizeof(double) * n : 0);
+    if (!(memory & 2))
+      need += (sizeof(double) + sizeof(int) * (left ? 4 : 2)) * n;
+    need = (need + 15) / 16 * 16;
+    if (f.used + need > h->piece_bytes)
+      G4_TRY(next_piece(h, f));
+    unsigned char* at = h->piece[f.piece].h + h->desc_bytes + f.used;
+    size_t off = f.sent + f.used;
+    f.used += need;
+    auto take = [&](size_t bytes) {  // the next `bytes`
+      unsigned char* p = at;
+      at += bytes;
+      off += bytes;
+      return p;
+    };
     if (!(memory & 1)) {  // M in host memory: packed column by column
-      unsigned char* fm = take(col * n, at);
+      d.m = reinterpret_cast<double*>(off);
+      d.ld = n;
+      unsigned char* fm = take(col * n);
       const unsigned char* src = reinterpret_cast<const unsigned char*>(wk.m[s]);
       if (wk.ld[s] == n)
         std::memcpy(fm, src, col * n);
       else
         for (int j = 0; j < n; ++j)
           std::memcpy(fm + col * j, src + col / n * wk.ld[s] * j, col);
-      d.m = reinterpret_cast<double*>(h->d_stage + at);
-      d.ld = n;
+      if (xv) {
+        d.expv = reinterpret_cast<double*>(off);
+        std::memcpy(take(sizeof(double) * n), xv, sizeof(double) * n);
+      }
     }
     else {
       d.m = wk.m[s];
       d.ld = wk.ld[s];
+      d.expv = xv;
     }
-    if (wk.n_form) {
-      const double* xv = wk.expv[s];
-      if (!xv)
-        return h->fail(G4ACC_INVALID_ARG, "exp_v missing for a non-empty spin sector");
-      if (!(memory & 1)) {
-        std::memcpy(take(sizeof(double) * n, at), xv, sizeof(double) * n);
-        d.expv = reinterpret_cast<double*>(h->d_stage + at);
-      }
-      else
-        d.expv = xv;
-    }
-    const bool left = wk.site_l[s] != nullptr;
     if (!(memory & 2)) {  // configuration in host memory: validated and packed
-      std::memcpy(take(sizeof(double) * n, at), wk.tau[s], sizeof(double) * n);
-      d.tau = reinterpret_cast<double*>(h->d_stage + at);
-      int* im = reinterpret_cast<int*>(take(sizeof(int) * (left ? 4 : 2) * n, at));
-      const int* di = reinterpret_cast<int*>(h->d_stage + at);
+      d.tau = reinterpret_cast<double*>(off);
+      std::memcpy(take(sizeof(double) * n), wk.tau[s], sizeof(double) * n);
+      const int* di = reinterpret_cast<int*>(off);
+      int* im = reinterpret_cast<int*>(take(sizeof(int) * (left ? 4 : 2) * n));
       for (int i = 0; i < n; ++i) {
         const int r = wk.site[s][i], bd = wk.band[s][i];
         if (r < 0 || r >= nc || bd < 0 || bd >= nb)
@@ -545,26 +638,70 @@ int pack_walker(g4acc_handle* h, int b, int w, const WalkerIn& wk, int memory, s
       d.band_l = wk.band_l[s];
     }
   }
+  ++f.n;
   return G4ACC_OK;
 }
 
-// Copies block b's descriptors of nw_ walkers, and the host arrays behind them, to the device.
-int send_walkers(g4acc_handle* h, int b, int nw_, size_t used, hipStream_t st) {
-  return send_block(h, b, h->d_stage, used > h->desc_bytes ? used : 2 * sizeof(SlotDesc) * nw_, st);
+// Begins a batch in piece b.
+int begin_fill(g4acc_handle* h, g4acc_handle::Fill& f, int b, int memory) {
+  f.n = 0;
+  f.used = f.sent = 0;
+  f.memory = memory;
+  f.piece = f.block = -1;
+  G4_TRY(claim_piece(h, b));
+  f.piece = b;
+  return G4ACC_OK;
 }
 
-// The block that calls other than the queue stage in.
-int free_block(const g4acc_handle* h) { return h->q_block == 0 ? 1 : 0; }
+// Sends what is left of the batch: its arrays and descriptors in one copy, or the last piece to the
+// batch's block and the descriptors by themselves.
+int send_fill(g4acc_handle* h, g4acc_handle::Fill& f) {
+  const int b = f.piece;
+  unsigned char* dev = h->d_stage + h->desc_bytes;
+  const size_t db = 2 * sizeof(SlotDesc) * f.n;
+  size_t bytes = f.used > 0 ? h->desc_bytes + f.used : db;
+  int rc = release_block(h);
+  if (f.block >= 0) {
+    dev = h->block[f.block].d;
+    bytes = db;
+    if (rc == G4ACC_OK)
+      rc = send_arrays(h, f);
+    if (rc == G4ACC_OK)
+      rc = h->check(hipEventRecord(h->copied, h->copy_stream), "hipEventRecord");
+    if (rc == G4ACC_OK)
+      rc = h->check(hipStreamWaitEvent(h->stream, h->copied, 0), "hipStreamWaitEvent");
+    h->run_block = f.block;
+  }
+  f.piece = f.block = -1;
+  G4_TRY(rc);
+  // Host arrays' offsets to device addresses (an array that is not there is null in both).
+  auto place = [&](auto*& p, bool there) {
+    using T = std::remove_reference_t<decltype(p)>;
+    if (there)
+      p = reinterpret_cast<T>(dev + reinterpret_cast<size_t>(p));
+  };
+  for (int i = 0; i < 2 * f.n; ++i) {
+    SlotDesc& d = f.desc[i];
+    const bool m = !(f.memory & 1) && d.n > 0, c = !(f.memory & 2) && d.n > 0;
+    place(d.m, m);
+    place(d.expv, m && d.expv);
+    place(d.tau, c);
+    place(d.site, c);
+    place(d.band, c);
+    place(d.site_l, c && d.site_l);
+    place(d.band_l, c && d.band_l);
+  }
+  std::memcpy(h->piece[b].h, f.desc.data(), db);
+  return send_piece(h, b, h->d_stage, bytes, h->stream);
+}
 
-// Resolves the walkers of one chunk into slot descriptors on the device; host inputs travel with them
-// in one copy.
-int stage_walkers(g4acc_handle* h, const WalkerIn* ws, int nw_, int memory, hipStream_t st) {
-  const int b = free_block(h);
-  G4_TRY(claim_block(h, b));
-  size_t used = h->desc_bytes;
+// Resolves the walkers of one chunk into slot descriptors on the device, with their host arrays.
+int stage_walkers(g4acc_handle* h, const WalkerIn* ws, int nw_, int memory) {
+  g4acc_handle::Fill& f = h->direct;
+  G4_TRY(begin_fill(h, f, free_piece(h), memory));
   for (int w = 0; w < nw_; ++w)
-    G4_TRY(pack_walker(h, b, w, ws[w], memory, used));
-  return send_walkers(h, b, nw_, used, st);
+    G4_TRY(pack_walker(h, f, ws[w]));
+  return send_fill(h, f);
 }
 
 template <typename Real>
@@ -798,8 +935,10 @@ int run_batch(g4acc_handle* h, int n_walkers) {
 
 // Waits for all work of the handle.
 int quiesce(g4acc_handle* h) {
+  if (h->copy_stream)
+    G4_TRY(h->check(hipStreamSynchronize(h->copy_stream), "hipStreamSynchronize"));
   G4_TRY(h->check(hipStreamSynchronize(h->stream), "hipStreamSynchronize"));
-  h->stage[0].pending = h->stage[1].pending = false;
+  h->piece[0].pending = h->piece[1].pending = false;
   return G4ACC_OK;
 }
 
@@ -1058,13 +1197,25 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
   for (auto& p : h->d_g4)
     if ((rc = h->alloc(reinterpret_cast<double2**>(&p), h->g4_entries, "G4")))
       return bail(rc);
-  // Per slot: M (or N; complex M takes two doubles per entry), tau and exp(V); right and left labels;
-  // 16-byte alignment.
+  // Per slot: M (or N; complex M takes two doubles per entry), tau and exp(V); right and left labels. A
+  // piece holds a slot at least; two MiB copy in 40 us, well above a copy's own cost.
   h->desc_bytes = (sizeof(SlotDesc) * W2 + 15) / 16 * 16;
-  h->stage_cap = h->desc_bytes + W2 * (sizeof(double) * ((h->complex_m ? 2 : 1) * NM * NM + 2 * NM) +
-                                       sizeof(int) * (h->non_dd ? 4 : 2) * NM + 16);
-  if ((rc = h->alloc(&h->d_stage, h->stage_cap, "stage")) || (rc = claim_block(h, 0)))
+  const size_t slot_bytes = (sizeof(double) * ((h->complex_m ? 2 : 1) * NM * NM + 2 * NM) +
+                             sizeof(int) * (h->non_dd ? 4 : 2) * NM + 15) / 16 * 16;
+  h->arrays_cap = W2 * slot_bytes;
+  h->piece_bytes = std::min(h->arrays_cap, std::max(slot_bytes, size_t(2) << 20));
+  h->host_bytes = 2 * (h->desc_bytes + h->piece_bytes);
+  if ((rc = h->alloc(&h->d_stage, h->desc_bytes + h->piece_bytes, "stage")) ||
+      (h->piece_bytes < h->arrays_cap && (rc = h->alloc(&h->block[0].d, h->arrays_cap, "stage block"))) ||
+      (rc = h->check(hipHostMalloc(reinterpret_cast<void**>(&h->h_stage), h->host_bytes), "hipHostMalloc")))
     return bail(rc);
+  for (int b = 0; b < 2; ++b) {
+    h->piece[b].h = h->h_stage + b * (h->desc_bytes + h->piece_bytes);
+    if ((rc = h->check(hipEventCreateWithFlags(&h->piece[b].done, hipEventDisableTiming), "hipEventCreate")))
+      return bail(rc);
+  }
+  h->direct.desc.resize(W2);
+  h->q.desc.resize(W2);
   h->d_desc = reinterpret_cast<SlotDesc*>(h->d_stage);
 
   // Constant tables. On a square cluster the sites are relabelled x + L y (the sort orders the
@@ -1121,18 +1272,26 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
 int g4acc_destroy(g4acc_handle* h) {
   if (!h)
     return G4ACC_OK;
+  if (h->copy_stream)
+    (void)hipStreamSynchronize(h->copy_stream);
   if (h->stream)
     (void)hipStreamSynchronize(h->stream);
   for (auto& e : h->graphs)
     (void)hipGraphExecDestroy(e.second);
   for (void* p : h->allocations)
     (void)hipFree(p);
-  for (auto& k : h->stage) {
-    if (k.h)
-      (void)hipHostFree(k.h);
+  if (h->h_stage)
+    (void)hipHostFree(h->h_stage);
+  for (auto& k : h->piece)
     if (k.done)
       (void)hipEventDestroy(k.done);
-  }
+  for (auto& k : h->block)
+    if (k.read)
+      (void)hipEventDestroy(k.read);
+  if (h->copied)
+    (void)hipEventDestroy(h->copied);
+  if (h->copy_stream)
+    (void)hipStreamDestroy(h->copy_stream);
   for (auto e : h->ev)
     if (e)
       (void)hipEventDestroy(e);
@@ -1147,7 +1306,7 @@ int g4acc_reset(g4acc_handle* h) {
     return G4ACC_INVALID_ARG;
   G4_TRY(h->check(hipSetDevice(h->device), "hipSetDevice"));
   h->queue.clear();
-  h->q_block = -1;
+  h->q.piece = h->q.block = -1;
   for (auto* p : h->d_g4)
     launch_zero16(p, h->g4_entries, h->stream);
   if (h->sp) {
@@ -1190,7 +1349,7 @@ int accumulate_walkers(g4acc_handle* h, const std::vector<WalkerIn>& all, int me
       todo.push_back(w);
   for (size_t i0 = 0; i0 < todo.size(); i0 += h->max_walkers) {
     const int nw_ = static_cast<int>(std::min<size_t>(h->max_walkers, todo.size() - i0));
-    G4_TRY(stage_walkers(h, todo.data() + i0, nw_, memory, h->stream));
+    G4_TRY(stage_walkers(h, todo.data() + i0, nw_, memory));
     G4_TRY(run_batch(h, nw_));
   }
   return G4ACC_OK;
@@ -1255,16 +1414,15 @@ int g4acc_accumulate(g4acc_handle* h, const g4acc_walker* walker, int memory) {
 int g4acc_flush(g4acc_handle* h) {
   if (!h)
     return G4ACC_INVALID_ARG;
-  if (h->q_block >= 0) {  // host measurements, packed as they came
-    const int b = h->q_block, n = h->q_n;
-    h->q_block = -1;
-    if (h->q_error != G4ACC_OK)
-      return h->fail(h->q_error, h->q_err_text);
-    if (!h->g4_present)
-      return G4ACC_OK;
+  if (h->q.piece >= 0) {  // host measurements, packed as they came
+    if (h->q_error != G4ACC_OK || !h->g4_present) {
+      h->q.piece = h->q.block = -1;
+      return h->q_error != G4ACC_OK ? h->fail(h->q_error, h->q_err_text) : G4ACC_OK;
+    }
     G4_TRY(h->check(hipSetDevice(h->device), "hipSetDevice"));
-    G4_TRY(send_walkers(h, b, n, h->q_bytes, h->stream));
-    return run_batch(h, n);
+    h->q_next = 1 - h->q.piece;
+    G4_TRY(send_fill(h, h->q));
+    return run_batch(h, h->q.n);
   }
   if (h->queue.empty())
     return G4ACC_OK;
@@ -1319,24 +1477,24 @@ int g4acc_accumulate_queued(g4acc_handle* h, const g4acc_walker* walker, int mem
   G4_TRY(check_walker(h, w));
   if (w.n[0] + w.n[1] == 0)
     return G4ACC_OK;  // empty configuration: no-op (tp_accumulator_cpu.hpp:238-239)
-  if ((h->q_block >= 0 && memory != G4ACC_HOST) || (!h->queue.empty() && h->queue_kind != memory))
+  if ((h->q.piece >= 0 && memory != G4ACC_HOST) || (!h->queue.empty() && h->queue_kind != memory))
     G4_TRY(g4acc_flush(h));
   if (memory == G4ACC_HOST) {
-    if (h->q_block < 0) {
-      const int b = h->q_next;
-      G4_TRY(claim_block(h, b));
-      h->q_next = 1 - b;
-      h->q_block = b;
-      h->q_n = 0;
-      h->q_bytes = h->desc_bytes;
+    if (h->q.piece < 0) {
+      G4_TRY(begin_fill(h, h->q, h->q_next, memory));
       h->q_error = G4ACC_OK;
+      h->q_walkers = 0;
     }
     if (h->q_error == G4ACC_OK) {
-      h->q_error = pack_walker(h, h->q_block, h->q_n, walker_in(w), memory, h->q_bytes);
+      h->q_error = pack_walker(h, h->q, walker_in(w));
+      if (h->q_error != G4ACC_OK && h->q_error != G4ACC_INVALID_ARG) {
+        h->q.piece = h->q.block = -1;  // a copy failed: the queue is lost
+        return h->q_error;
+      }
       if (h->q_error != G4ACC_OK)
         h->q_err_text = h->err;
     }
-    return ++h->q_n == h->max_walkers ? g4acc_flush(h) : G4ACC_OK;
+    return ++h->q_walkers == h->max_walkers ? g4acc_flush(h) : G4ACC_OK;
   }
   const size_t NM = h->max_vertices, NM2 = NM * NM, W2 = 2 * static_cast<size_t>(h->max_walkers);
   if (!h->d_qm)
@@ -1470,6 +1628,7 @@ int g4acc_sum_to(g4acc_handle* src, g4acc_handle* dst) {
 
 size_t g4acc_g4_size(const g4acc_handle* h) { return h ? h->g4_entries : 0; }
 size_t g4acc_bytes(const g4acc_handle* h) { return h ? h->bytes : 0; }
+size_t g4acc_host_bytes(const g4acc_handle* h) { return h ? h->host_bytes : 0; }
 void* g4acc_stream(g4acc_handle* h) { return h ? static_cast<void*>(h->stream) : nullptr; }
 
 const char* g4acc_last_error(const g4acc_handle* h) {
@@ -1495,7 +1654,7 @@ int compute_G_impl(g4acc_handle* h, const WalkerIn& w, bool general, int memory,
   G4_TRY(check_walker(h, w, general));
   G4_TRY(quiesce(h));
   h->dirty = true;
-  G4_TRY(stage_walkers(h, &w, 1, memory, h->stream));
+  G4_TRY(stage_walkers(h, &w, 1, memory));
   if (h->precision == G4ACC_FP64)
     run_mtog<double>(h, 2, h->stream, false);  // the caller gets all of G
   else
@@ -1613,12 +1772,12 @@ int g4acc_compute_G_noalloc(g4acc_handle* h, const g4acc_walker* walker, double*
     return h->fail(G4ACC_INVALID_ARG, "compute_G_noalloc: this measurement needs " + std::to_string(l.total) +
                                           " B of workspace, more than the static " +
                                           std::to_string(G4ACC_NOALLOC_SCRATCH_BYTES) + " B");
-  // Measurements queued by g4acc_accumulate_queued stay queued (their block is not touched here).
-  const int blk = free_block(h);
-  G4_TRY(claim_block(h, blk));
+  // Measurements queued by g4acc_accumulate_queued stay queued (their piece is not touched here).
+  const int blk = free_piece(h);
+  G4_TRY(claim_piece(h, blk));
   h->dirty = true;
   for (int s = 0; s < 2; ++s) {
-    SlotDesc& d = h->stage[blk].desc()[s];
+    SlotDesc& d = h->piece[blk].desc()[s];
     d.n = walker->n[s];
     d.ld = walker->ld[s];
     d.sign = walker->sign;
@@ -1631,7 +1790,7 @@ int g4acc_compute_G_noalloc(g4acc_handle* h, const g4acc_walker* walker, double*
     d.site = d.n ? walker->site[s] : nullptr;
     d.band = d.n ? walker->band[s] : nullptr;
   }
-  G4_TRY(send_block(h, blk, h->d_scratch + l.desc, 2 * sizeof(SlotDesc), h->stream));
+  G4_TRY(send_piece(h, blk, h->d_scratch + l.desc, 2 * sizeof(SlotDesc), h->stream));
   if (h->precision == G4ACC_FP64)
     launch_mtog_noalloc<double>(h, l, n_max, G_dev);
   else
@@ -1655,14 +1814,14 @@ int g4acc_accumulate_G(g4acc_handle* h, const double* G_ref, double sign) {
   G4_TRY(h->check(hipMalloc(&tmp, sizeof(double2) * n), "hipMalloc(import)"));
   int rc = h->check(hipMemcpyAsync(tmp, G_ref, sizeof(double2) * n, hipMemcpyHostToDevice, h->stream),
                     "copy G");
-  const int blk = free_block(h);
+  const int blk = free_piece(h);
   if (rc == G4ACC_OK)
-    rc = claim_block(h, blk);
+    rc = claim_piece(h, blk);
   if (rc == G4ACC_OK) {
-    SlotDesc* d = h->stage[blk].desc();
+    SlotDesc* d = h->piece[blk].desc();
     d[0] = SlotDesc{nullptr, nullptr, nullptr, nullptr, 1, 1, sign, nullptr, nullptr, nullptr, 0.0, 0};
     d[1] = d[0];
-    rc = send_block(h, blk, h->d_desc, 2 * sizeof(SlotDesc), h->stream);
+    rc = send_piece(h, blk, h->d_desc, 2 * sizeof(SlotDesc), h->stream);
   }
   if (rc == G4ACC_OK) {
     if (h->precision == G4ACC_FP64) {

@@ -30,7 +30,7 @@ HOST, DEVICE_M, DEVICE = 0, 1, 3
 
 EXPORTED = [
     "g4acc_create", "g4acc_destroy", "g4acc_reset", "g4acc_accumulate", "g4acc_accumulate_batch",
-    "g4acc_finalize", "g4acc_sync", "g4acc_get_g4", "g4acc_get_g4_normalized", "g4acc_sum_to", "g4acc_g4_size", "g4acc_bytes",
+    "g4acc_finalize", "g4acc_sync", "g4acc_get_g4", "g4acc_get_g4_normalized", "g4acc_sum_to", "g4acc_g4_size", "g4acc_bytes", "g4acc_host_bytes",
     "g4acc_stream", "g4acc_last_error", "g4acc_compute_G", "g4acc_g_size", "g4acc_accumulate_G",
     "g4acc_set_timing", "g4acc_get_timing", "g4acc_set_tuning", "g4acc_accumulate_queued",
     "g4acc_accumulate_single",
@@ -133,6 +133,7 @@ def load_library(path: str = LIB_PATH):
         "g4acc_sum_to": (i32, [vp, vp]),
         "g4acc_g4_size": (sz, [vp]),
         "g4acc_bytes": (sz, [vp]),
+        "g4acc_host_bytes": (sz, [vp]),
         "g4acc_stream": (vp, [vp]),
         "g4acc_last_error": (ctypes.c_char_p, [vp]),
         "g4acc_compute_G": (i32, [vp, ctypes.POINTER(Walker_c), i32, vp, sz]),

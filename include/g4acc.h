@@ -207,6 +207,8 @@ int g4acc_sum_to(g4acc_handle* src, g4acc_handle* dst);
 size_t g4acc_g4_size(const g4acc_handle* h);
 /* Device bytes held by the handle. */
 size_t g4acc_bytes(const g4acc_handle* h);
+/* Page-locked host bytes held by the handle: the staging of host inputs, all allocated by g4acc_create. */
+size_t g4acc_host_bytes(const g4acc_handle* h);
 /* get_stream() (tp_accumulator_gpu.hpp): the hipStream_t the handle launches on. */
 void* g4acc_stream(g4acc_handle* h);
 /* Message of the last failed call on h (or of the last failed g4acc_create when h is NULL). */
