@@ -67,19 +67,28 @@ __device__ __forceinline__ pair_f64x4 mma4(double a, double b, pair_f64x4 c) {
 // Terms formed by the walker loop.
 constexpr int HAS_X = 1, HAS_Z = 2, HAS_T = 4;
 
-// Registers of a workgroup's threads. 704 threads hold 33..37-site clusters with two pairs each:
-// eleven waves leave 168 registers, enough for the totals of four momenta (6x6, magnetic and pp, 64
-// walkers, 64 frequencies: 4.6 ms per batch; two momenta 6.2, two in 1024 threads 7.6, since each
-// group of momenta reads the blocks again).
-template <typename Real, int TT, int PPT, int QG>
+// Registers of a workgroup's threads (waves per SIMD that must fit: 64 registers for eight, 128 for four,
+// 168 for three, 256 for two). 704 threads hold 33..37-site clusters with two pairs each: eleven waves
+// leave 168 registers, enough for the totals of four momenta (6x6, magnetic and pp, 64 walkers, 64
+// frequencies: 2.4 ms per batch; two momenta 3.0, one 4.9, since each group of momenta reads the blocks
+// again). 256 threads take what their totals need: held to 128, two pairs of complex128 G spilled 147
+// registers (20 sites, magnetic and pp, 16 walkers, 48 frequencies: 1.41 ms against 0.31).
+// 1024 threads with few totals fit 64 registers or nearly so: two workgroups per CU instead of one (25
+// sites, magnetic, complex64, 8 walkers: 58 -> 36 us).
+template <typename Real, int TT, int PPT, int QG, int SET>
 struct PairShape {
   static constexpr bool fp32 = sizeof(Real) == 4;
-  static constexpr int DEPTH = fp32 && TT == 1024 && PPT * QG <= 2 ? 2 : 1;  // walkers in flight
+  static constexpr int TOTALS = PPT * QG * ((SET & 1) + (SET >> 1 & 1) + (SET >> 2 & 1));  // complex FP64, per thread
   static constexpr int FLUSH = fp32 && TT == 256 ? 8 : 1;
-  static constexpr int WAVES = TT == 704 ? 3 : 4;  // per SIMD: 168 or 128 registers
-  // The compiler sinks the loads to their use, behind the products they are to overlap; kept in
-  // place they must fit beside everything else, which complex128 G in large tiles does not.
-  static constexpr bool HOLD = fp32 || TT == 256;
+  static constexpr int WAVES =
+      TT == 704    ? 3
+      : TT == 1024 ? (fp32 && PPT == 1 && TOTALS <= 2 ? 8 : 4)
+      : PPT == 1   ? (TOTALS >= (fp32 ? 12 : 8) ? 3 : 4)
+      : fp32       ? (TOTALS >= 8 ? 3 : 4)
+                   : (TOTALS <= 2 ? 4 : TOTALS <= 4 ? 3 : 2);
+  // The compiler sinks the loads to their use, behind the products they are to overlap; kept in place
+  // they must fit beside everything else, which complex128 G in large tiles does not.
+  static constexpr bool HOLD = fp32 || TT == 256 || (PPT == 1 && TOTALS <= 4);
 };
 
 // G4[i] += v in two steps, so that a thread's loads are issued ahead of its stores.
@@ -134,12 +143,12 @@ __global__ void __launch_bounds__(256) uv_kernel(TiledArgs<Real> a) {
 }
 
 template <typename Real, int TT, int PPT, int QG, int SET>
-__global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_pair_kernel(TiledArgs<Real> a) {
+__global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)) g4_pair_kernel(TiledArgs<Real> a) {
   using C = Cplx<Real>;
   using P2 = CPair<C>;
-  using Shape = PairShape<Real, TT, PPT, QG>;
+  using Shape = PairShape<Real, TT, PPT, QG, SET>;
   constexpr bool HX = (SET & HAS_X) != 0, HZ = (SET & HAS_Z) != 0, HT = (SET & HAS_T) != 0, HY = HX || HT;
-  constexpr int DEPTH = Shape::DEPTH, FLUSH = Shape::FLUSH;
+  constexpr int FLUSH = Shape::FLUSH;
   extern __shared__ unsigned char smem_raw[];
   const Geo& g = a.g;
   const int nc = g.nc, nw = g.nw, e = g.ext, P = nc * nw;
@@ -209,12 +218,12 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
       fx[j][qi] = fz[j][qi] = ft[j][qi] = C{0, 0};
     }
   const int n_walk = a.n_walkers;
-  C px[DEPTH][PPT][2], py[DEPTH][PPT][2], pz[DEPTH][PPT][2];
-  double sign[DEPTH];
-  auto fetch = [&](int m, int d) {
+  C px[PPT][2], py[PPT][2], pz[PPT][2];  // the next walker's
+  double sign = 0;
+  auto fetch = [&](int m) {
     const int mc = m < n_walk ? m : n_walk - 1;
     const size_t mo = 2 * static_cast<size_t>(mc) * DD;
-    sign[d] = a.desc[2 * mc].sign;
+    sign = a.desc[2 * mc].sign;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const C* X = Xg + mo + s * DD;
@@ -223,13 +232,13 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
 #pragma unroll
       for (int j = 0; j < PPT; ++j) {
         if (HY)
-          py[d][j][s] = Y[yo[j]];
+          py[j][s] = Y[yo[j]];
         if (HZ)
-          pz[d][j][s] = Z[zo[j]];
+          pz[j][s] = Z[zo[j]];
       }
 #pragma unroll
       for (int j = 0; j < PPT; ++j)
-        px[d][j][s] = X[xo[j]];
+        px[j][s] = X[xo[j]];
     }
   };
   auto flush = [&]() {
@@ -246,25 +255,25 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
         fx[j][qi] = fz[j][qi] = ft[j][qi] = C{0, 0};
       }
   };
-  auto walker = [&](int m, int d) {
+  auto walker = [&](int m) {
     __syncthreads();  // the previous walker's blocks have been read
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
       if (ok[j]) {
         if (HY)
-          store_pair(Yl[li[j]], C{py[d][j][0].x, py[d][j][0].y * ys_im}, C{py[d][j][1].x, py[d][j][1].y * ys_im});
+          store_pair(Yl[li[j]], C{py[j][0].x, py[j][0].y * ys_im}, C{py[j][1].x, py[j][1].y * ys_im});
         if (HZ)
-          store_pair(Zl[li[j]], C{pz[d][j][0].x, pz[d][j][0].y * zs_im}, C{pz[d][j][1].x, pz[d][j][1].y * zs_im});
+          store_pair(Zl[li[j]], C{pz[j][0].x, pz[j][0].y * zs_im}, C{pz[j][1].x, pz[j][1].y * zs_im});
       }
-    const Real al = static_cast<Real>(0.5 * sign[d]), ali = al * xs_im;
+    const Real al = static_cast<Real>(0.5 * sign), ali = al * xs_im;
     C x0[PPT], x1[PPT];
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
-      x0[j] = C{al * px[d][j][0].x, ali * px[d][j][0].y};
-      x1[j] = C{al * px[d][j][1].x, ali * px[d][j][1].y};
+      x0[j] = C{al * px[j][0].x, ali * px[j][0].y};
+      x1[j] = C{al * px[j][1].x, ali * px[j][1].y};
     }
     __syncthreads();
-    fetch(m + DEPTH, d);
+    fetch(m + 1);
     if constexpr (Shape::HOLD)
       asm volatile("" ::: "memory");
 #pragma unroll
@@ -295,17 +304,9 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
       flush();
   };
   if (n_walk > 0) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d)
-      fetch(d, d);
-    int m = 0;
-    for (; m + DEPTH <= n_walk; m += DEPTH)
-#pragma unroll
-      for (int d = 0; d < DEPTH; ++d)
-        walker(m + d, d);
-    if constexpr (DEPTH > 1)
-      if (m < n_walk)
-        walker(m, 0);
+    fetch(0);
+    for (int m = 0; m < n_walk; ++m)
+      walker(m);
     if (FLUSH > 1)
       flush();
   }
@@ -582,10 +583,19 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG>::WAVES)) g4_
 
 namespace {
 
+// Complex totals (pairs x momenta x terms, four registers each) that a thread may hold: 16; 8 where the loads
+// in flight need the others (complex128 G, or several pairs per thread, in a 1024-thread workgroup's 128
+// registers: 40 sites, magnetic and pp, complex64, 32 walkers, 32 frequencies, four momenta with 16
+// totals 1.13 ms, two with 8 0.58).
+constexpr int totals_limit(bool fp32, int threads, int ppt) { return threads == 1024 && (!fp32 || ppt > 1) ? 8 : 16; }
+
 template <typename Real, int TT, int PPT, int QG, int SET>
 void launch_pair_set(TiledArgs<Real> a, size_t lds, hipStream_t st) {
-  const unsigned tiles = tile_schedule(a);
-  hipLaunchKernelGGL((g4_pair_kernel<Real, TT, PPT, QG, SET>), dim3(tiles), dim3(TT), lds, st, a);
+  using Shape = PairShape<Real, TT, PPT, QG, SET>;
+  if constexpr (QG == 1 || Shape::TOTALS <= totals_limit(Shape::fp32, TT, PPT)) {  // others are never chosen
+    const unsigned tiles = tile_schedule(a);
+    hipLaunchKernelGGL((g4_pair_kernel<Real, TT, PPT, QG, SET>), dim3(tiles), dim3(TT), lds, st, a);
+  }
 }
 
 template <typename Real, int TT, int PPT, int QG>
@@ -710,15 +720,10 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
     set |= a.ch[c] == PP_UP_DOWN ? HAS_Z : a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE ? HAS_X : HAS_T;
     n_ph += a.ch[c] != PP_UP_DOWN;
   }
-  // Momenta per workgroup: as many as keep the FP64 totals (pairs x momenta x terms, four registers
-  // each) at 64 registers; at 32 where the loads in flight need the others (complex128 G or four
-  // pairs per thread in a 1024-thread workgroup, 128 registers).
+  // Momenta per workgroup: as many as the totals allow.
   const int terms = set == (HAS_X | HAS_Z) ? 2 : set == HAS_X || set == HAS_Z ? 1 : set & HAS_Z ? 3 : 2;
-  const int budget = ts.threads == 1024 && (sizeof(Real) == 8 || ppt == 4) ? 8 : 16;
   int qg = g.nq >= 3 ? 4 : g.nq;
-  if (ppt == 4 && qg > 2)
-    qg = 2;
-  while (qg > 1 && ppt * qg * terms > budget)
+  while (qg > 1 && ppt * qg * terms > totals_limit(sizeof(Real) == 4, ts.threads, ppt))
     qg /= 2;
   while (a.qg_cap > 0 && qg > a.qg_cap)
     qg /= 2;
