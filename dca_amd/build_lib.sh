@@ -6,13 +6,13 @@ HERE="$(cd "$(dirname "${BASH_SOURCE[0]}")" && pwd)"
 OUT="$HERE/libg4acc.so"
 OBJ="$HERE/_build"
 mkdir -p "$OBJ"
-SRC=(g4acc_api mtog_kernels mtog_fused mtog_small mtog_large g4_kernels g4_tiled g4_band sp_acc)
+SRC=(g4acc_api mtog_kernels mtog_fused mtog_small mtog_large g4_kernels g4_tiled g4_tiled32 g4_band sp_acc)
 FLAGS=(--offload-arch=gfx950 -O3 -std=c++17 -fPIC -Wall
        -Xclang -target-feature -Xclang -packed-fp32-ops)
 filter() { grep -v "packed-fp32-ops' is not a recognized feature" >&2 || true; }
 pids=()
 # The matrix-core M -> G and G4 tile kernels keep their accumulators in VGPRs (no AGPR copies).
-extra() { case "$1" in mtog_small|g4_tiled) echo "-mllvm -amdgpu-mfma-vgpr-form=1" ;; esac; }
+extra() { case "$1" in mtog_small|g4_tiled|g4_tiled32) echo "-mllvm -amdgpu-mfma-vgpr-form=1" ;; esac; }
 for s in "${SRC[@]}"; do
   /opt/rocm/bin/hipcc "${FLAGS[@]}" $(extra "$s") -c "$HERE/csrc/$s.hip" -o "$OBJ/$s.o" 2> >(filter) &
   pids+=($!)

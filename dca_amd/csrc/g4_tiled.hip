@@ -24,13 +24,21 @@
 // load is issued (idle slots and walkers past the batch re-read valid elements).
 // Per batch (256 walkers) the stage went from 3.64 ms, with the rank-one terms in a buffer of G4's
 // size, to 2.9 ms; 6x6 (64 walkers, 64 frequencies, 4 q, 2 v) from 10.6 to 4.6 ms.
-// Products are formed in the G precision; with complex64 G, 256-thread tiles sum eight walkers in
+// Launches of few walkers (up to five, on 17..32 sites up to eight) are the G4 read-modify-write with little
+// before it (FEW): all tiles, without images, the rank-one factors staged in LDS beside the blocks, and one
+// entry (complex128 G in small tiles: four) loaded before it is stored. With the code for many walkers
+// (images, factors read from memory in the tail, twelve entries in flight) a launch took, 4x4, three channels, 64
+// frequencies, 4 q, 3 v: one walker FP64 340 against 279 us, FP32 336 against 257; three 452 against 342 and
+// 445 against 303.
+// Products are formed in the G precision; with complex64 G, tiles of up to 256 threads sum eight walkers in
 // FP32 before the FP64 totals, larger tiles (whose registers hold the totals) add every walker.
 // G4 is read and written once per launch (FP64, or FP32 value + Kahan compensation).
+// Compiled once per precision: complex64 through g4_tiled32.hip.
 #include <algorithm>
 #include <type_traits>
 
 #include "g4_tile_common.hpp"
+#include "mfma16.hpp"
 
 namespace g4acc {
 
@@ -55,15 +63,6 @@ __device__ __forceinline__ void store_pair(CPair<C>& dst, C a, C b) {
   }
 }
 
-typedef float pair_f32x4 __attribute__((ext_vector_type(4)));
-typedef double pair_f64x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ pair_f32x4 mma4(float a, float b, pair_f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ pair_f64x4 mma4(double a, double b, pair_f64x4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 // Terms formed by the walker loop.
 constexpr int HAS_X = 1, HAS_Z = 2, HAS_T = 4;
 
@@ -72,23 +71,33 @@ constexpr int HAS_X = 1, HAS_Z = 2, HAS_T = 4;
 // leave 168 registers, enough for the totals of four momenta (6x6, magnetic and pp, 64 walkers, 64
 // frequencies: 2.4 ms per batch; two momenta 3.0, one 4.9, since each group of momenta reads the blocks
 // again). 256 threads take what their totals need: held to 128, two pairs of complex128 G spilled 147
-// registers (20 sites, magnetic and pp, 16 walkers, 48 frequencies: 1.41 ms against 0.31).
+// registers (20 sites, magnetic and pp, 16 walkers, 48 frequencies: 1.41 ms against 0.32).
 // 1024 threads with few totals fit 64 registers or nearly so: two workgroups per CU instead of one (25
-// sites, magnetic, complex64, 8 walkers: 58 -> 36 us).
-template <typename Real, int TT, int PPT, int QG, int SET>
+// sites, magnetic, complex64, 8 walkers: 60 -> 51 us). Without images and matrix-core tail (FEW) small shapes
+// take less.
+template <typename Real, int TT, int PPT, int QG, int SET, bool FEW>
 struct PairShape {
   static constexpr bool fp32 = sizeof(Real) == 4;
-  static constexpr int TOTALS = PPT * QG * ((SET & 1) + (SET >> 1 & 1) + (SET >> 2 & 1));  // complex FP64, per thread
-  static constexpr int FLUSH = fp32 && TT == 256 ? 8 : 1;
+  static constexpr int TERMS = (SET & 1) + (SET >> 1 & 1) + (SET >> 2 & 1);
+  static constexpr int TOTALS = PPT * QG * TERMS;  // complex FP64, per thread
+  // Fits 64 registers.
+  static constexpr bool SMALL = PPT == 1 && TOTALS <= 2 && (fp32 || (FEW && TERMS == 1));
+  static constexpr int FLUSH = fp32 && TT <= 256 ? 8 : 1;
+  // Walkers in flight: two where one workgroup fills a CU and its registers allow it (complex128, magnetic, 32
+  // sites, 32 walkers, 48 frequencies: 881 -> 809 us).
+  static constexpr int DEPTH = !fp32 && !FEW && TT == 1024 && PPT == 1 && TERMS == 1 ? 2 : 1;
   static constexpr int WAVES =
       TT == 704    ? 3
-      : TT == 1024 ? (fp32 && PPT == 1 && TOTALS <= 2 ? 8 : 4)
+      : TT == 1024 ? (SMALL ? 8 : 4)
+      : FEW        ? (SMALL ? 8 : PPT == 1 && TOTALS <= 8 ? 4 : 2)
       : PPT == 1   ? (TOTALS >= (fp32 ? 12 : 8) ? 3 : 4)
       : fp32       ? (TOTALS >= 8 ? 3 : 4)
                    : (TOTALS <= 2 ? 4 : TOTALS <= 4 ? 3 : 2);
   // The compiler sinks the loads to their use, behind the products they are to overlap; kept in place
   // they must fit beside everything else, which complex128 G in large tiles does not.
-  static constexpr bool HOLD = fp32 || TT == 256 || (PPT == 1 && TOTALS <= 4);
+  static constexpr bool HOLD = fp32 || TT <= 256 || (PPT == 1 && TOTALS <= 4);
+  // FEW: no loads past the last walker, where a branch around them costs no registers.
+  static constexpr bool EXACT = FEW && (fp32 || TT <= 256 || PPT == 1);
 };
 
 // G4[i] += v in two steps, so that a thread's loads are issued ahead of its stores.
@@ -142,13 +151,13 @@ __global__ void __launch_bounds__(256) uv_kernel(TiledArgs<Real> a) {
   out[3 * plane] = C{v0.x + v1.x, v0.y + v1.y};
 }
 
-template <typename Real, int TT, int PPT, int QG, int SET>
-__global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)) g4_pair_kernel(TiledArgs<Real> a) {
+template <typename Real, int TT, int PPT, int QG, int SET, bool FEW>
+__global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET, FEW>::WAVES)) g4_pair_kernel(TiledArgs<Real> a) {
   using C = Cplx<Real>;
   using P2 = CPair<C>;
-  using Shape = PairShape<Real, TT, PPT, QG, SET>;
+  using Shape = PairShape<Real, TT, PPT, QG, SET, FEW>;
   constexpr bool HX = (SET & HAS_X) != 0, HZ = (SET & HAS_Z) != 0, HT = (SET & HAS_T) != 0, HY = HX || HT;
-  constexpr int FLUSH = Shape::FLUSH;
+  constexpr int DEPTH = Shape::DEPTH, FLUSH = Shape::FLUSH;
   extern __shared__ unsigned char smem_raw[];
   const Geo& g = a.g;
   const int nc = g.nc, nw = g.nw, e = g.ext, P = nc * nw;
@@ -165,6 +174,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
   const int ld = nc + 1, bs = nc * ld, ncc = nc * nc;
   P2* Yl = reinterpret_cast<P2*>(smem_raw);  // [b][a] (a fastest): {spin 0, spin 1}
   P2* Zl = Yl + (HY ? bs : 0);
+  C* const Fl = reinterpret_cast<C*>(smem_raw + a.uv_lds);  // FEW: rank-one factors [walker][plane][momentum][k]
   // Blocks (wa, wb) of G (extended frequencies). Of a conjugate symmetric G only the half
   // wa + wb >= nwE - 1 is read: another block is the conjugate of (-wa, -wb) at (-ka, -kb); its sign
   // is applied where the block is staged (Y, Z) or scaled by alpha (X).
@@ -218,12 +228,14 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
       fx[j][qi] = fz[j][qi] = ft[j][qi] = C{0, 0};
     }
   const int n_walk = a.n_walkers;
-  C px[PPT][2], py[PPT][2], pz[PPT][2];  // the next walker's
-  double sign = 0;
-  auto fetch = [&](int m) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t uv_row = static_cast<size_t>(g.nq) * g.nv * P;  // between the planes of one walker
+  C px[DEPTH][PPT][2], py[DEPTH][PPT][2], pz[DEPTH][PPT][2];  // the next walkers'
+  double sign[DEPTH];
+  auto fetch = [&](int m, int d) {
     const int mc = m < n_walk ? m : n_walk - 1;
     const size_t mo = 2 * static_cast<size_t>(mc) * DD;
-    sign = a.desc[2 * mc].sign;
+    sign[d] = a.desc[2 * mc].sign;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const C* X = Xg + mo + s * DD;
@@ -232,50 +244,62 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
 #pragma unroll
       for (int j = 0; j < PPT; ++j) {
         if (HY)
-          py[j][s] = Y[yo[j]];
+          py[d][j][s] = Y[yo[j]];
         if (HZ)
-          pz[j][s] = Z[zo[j]];
+          pz[d][j][s] = Z[zo[j]];
       }
 #pragma unroll
       for (int j = 0; j < PPT; ++j)
-        px[j][s] = X[xo[j]];
+        px[d][j][s] = X[xo[j]];
     }
   };
   auto flush = [&]() {
+    auto add = [](double2& t, C f) {
+      if constexpr (FEW && FLUSH > 1)
+        t = to_d(f);  // the one sum of the launch
+      else
+        t = double2{t.x + static_cast<double>(f.x), t.y + static_cast<double>(f.y)};
+    };
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
 #pragma unroll
       for (int qi = 0; qi < QG; ++qi) {
         if (HX)
-          tx[j][qi] = double2{tx[j][qi].x + static_cast<double>(fx[j][qi].x), tx[j][qi].y + static_cast<double>(fx[j][qi].y)};
+          add(tx[j][qi], fx[j][qi]);
         if (HZ)
-          tz[j][qi] = double2{tz[j][qi].x + static_cast<double>(fz[j][qi].x), tz[j][qi].y + static_cast<double>(fz[j][qi].y)};
+          add(tz[j][qi], fz[j][qi]);
         if (HT)
-          tt[j][qi] = double2{tt[j][qi].x + static_cast<double>(ft[j][qi].x), tt[j][qi].y + static_cast<double>(ft[j][qi].y)};
+          add(tt[j][qi], ft[j][qi]);
         fx[j][qi] = fz[j][qi] = ft[j][qi] = C{0, 0};
       }
   };
-  auto walker = [&](int m) {
+  auto walker = [&](int m, int d) {
     __syncthreads();  // the previous walker's blocks have been read
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
       if (ok[j]) {
         if (HY)
-          store_pair(Yl[li[j]], C{py[j][0].x, py[j][0].y * ys_im}, C{py[j][1].x, py[j][1].y * ys_im});
+          store_pair(Yl[li[j]], C{py[d][j][0].x, py[d][j][0].y * ys_im}, C{py[d][j][1].x, py[d][j][1].y * ys_im});
         if (HZ)
-          store_pair(Zl[li[j]], C{pz[j][0].x, pz[j][0].y * zs_im}, C{pz[j][1].x, pz[j][1].y * zs_im});
+          store_pair(Zl[li[j]], C{pz[d][j][0].x, pz[d][j][0].y * zs_im}, C{pz[d][j][1].x, pz[d][j][1].y * zs_im});
       }
-    const Real al = static_cast<Real>(0.5 * sign), ali = al * xs_im;
+    const Real al = static_cast<Real>(0.5 * sign[d]), ali = al * xs_im;
     C x0[PPT], x1[PPT];
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
-      x0[j] = C{al * px[j][0].x, ali * px[j][0].y};
-      x1[j] = C{al * px[j][1].x, ali * px[j][1].y};
+      x0[j] = C{al * px[d][j][0].x, ali * px[d][j][0].y};
+      x1[j] = C{al * px[d][j][1].x, ali * px[d][j][1].y};
     }
     __syncthreads();
-    fetch(m + 1);
-    if constexpr (Shape::HOLD)
-      asm volatile("" ::: "memory");
+    if constexpr (Shape::EXACT) {
+      if (m + 1 < n_walk)
+        fetch(m + 1, d);
+    }
+    else {
+      fetch(m + DEPTH, d);
+      if constexpr (Shape::HOLD)
+        asm volatile("" ::: "memory");
+    }
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
 #pragma unroll
@@ -300,13 +324,35 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
         }
       }
     }
-    if (FLUSH == 1 || (m + 1) % FLUSH == 0)
+    if (FLUSH == 1 || (!FEW && (m + 1) % FLUSH == 0))
       flush();
   };
   if (n_walk > 0) {
-    fetch(0);
-    for (int m = 0; m < n_walk; ++m)
-      walker(m);
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      fetch(d, d);
+    if constexpr (FEW && HX)
+      for (int i = threadIdx.x; i < (a.rank_one ? n_walk * 4 * QG * nc : 0); i += TT) {
+        const int k = i % nc, r = i / nc, qi = r % QG, row = r / QG;  // row: plane + 4 walker
+        const int qc = q0 + qi < g.nq ? q0 + qi : q0;
+        Fl[i] = a.UV[uv_row * row + static_cast<size_t>(qc + g.nq * iv) * P + nc * static_cast<size_t>((row & 2) ? w2 : w1) + k];
+      }
+    if (wave * 64 >= ncc) {  // a wave without pairs
+      for (int m = 0; m < n_walk; ++m) {
+        __syncthreads();
+        __syncthreads();
+      }
+    }
+    else {
+      int m = 0;
+      for (; m + DEPTH <= n_walk; m += DEPTH)
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+          walker(m + d, d);
+      if constexpr (DEPTH > 1)
+        if (m < n_walk)
+          walker(m, 0);
+    }
     if (FLUSH > 1)
       flush();
   }
@@ -318,7 +364,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
   // thread (k1, k2) of an image takes the tile's pair below.
   // LDS holds the particle-hole channels of those momenta together, or one channel at a time where a
   // plane is large (PPT = 4: up to 66.5 KB).
-  constexpr int RB = TT == 256 && PPT == 1 ? QG : 1;
+  constexpr int RB = TT <= 256 && PPT == 1 ? QG : 1;
   constexpr bool kOneCh = PPT == 4;
   auto left_out = [&](int wa, int wb) {
     return wa >= 0 && wa < nw && wb >= 0 && wb < nw && !sym_tile_computed(nw, nu, wa, wb, HY, HZ, a.sym);
@@ -343,24 +389,18 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
     asm volatile("" : "+v"(v));
     return v;
   };
-  // Below four walkers a matrix-core step would be mostly padding, and the launch is the G4
-  // read-modify-write: each thread forms its entries' rank-one terms itself (to its own LDS places,
-  // ahead of the G4 loads and stores).
-  const bool direct = n_walk < 4;
-  const size_t uv_row = static_cast<size_t>(g.nq) * g.nv * P;  // between the planes of one walker
-  auto rank_one = [&](int j, int qv, int pl) {
-    const C* U = a.UV + pl * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w1) + (kk[j] & 0xffff);
-    const C* V = a.UV + (pl + 2) * uv_row + static_cast<size_t>(qv) * P + nc * static_cast<size_t>(w2) + (kk[j] >> 16);
+  // FEW: a matrix-core step would be mostly padding; each thread forms its entries' rank-one terms.
+  auto rank_one = [&](int j, int qi, int pl) {
     double2 r{0, 0};
     for (int m = 0; m < n_walk; ++m)
-      cfma(r, to_d(V[4 * uv_row * m]), to_d(U[4 * uv_row * m]));
+      cfma(r, to_d(Fl[((4 * m + pl + 2) * QG + qi) * nc + (kk[j] >> 16)]),
+           to_d(Fl[((4 * m + pl) * QG + qi) * nc + (kk[j] & 0xffff)]));
     return r;
   };
-  constexpr int GS = RB * PPT >= 4 ? 4 : RB * PPT >= 2 ? 2 : 1;  // G4 entries per channel in flight
-  // Channels whose entries are in flight together (one where four groups of momenta are unrolled: the
-  // loop over them must unroll for the totals to stay in registers).
-  constexpr int CG = kOneCh || QG / RB > 2 ? 1 : 3;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // G4 entries per channel in flight, and channels whose entries are in flight together (one where four
+  // groups of momenta are unrolled: the loop over them must unroll for the totals to stay in registers).
+  constexpr int GS = RB * PPT >= 4 && !(FEW && Shape::fp32) ? 4 : RB * PPT >= 2 && !FEW ? 2 : 1;
+  constexpr int CG = FEW || kOneCh || QG / RB > 2 ? 1 : 3;
 #pragma unroll
   for (int r0 = 0; r0 < QG; r0 += RB) {
     if (q0 + r0 >= g.nq)
@@ -373,27 +413,16 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
       n_ph += ch_of(c) != PP_UP_DOWN;
       n_r += ch_of(c) == PH_MAGNETIC || ch_of(c) == PH_CHARGE;
     }
-    __syncthreads();
-    if (HX && n_r > 0 && direct) {
-      int ph = 0;
-      for (int c = c_lo; c < c_hi; ph += ch_of(c) != PP_UP_DOWN, ++c)
-        if (ch_of(c) == PH_MAGNETIC || ch_of(c) == PH_CHARGE)
-#pragma unroll
-          for (int r = 0; r < RB; ++r)
-#pragma unroll
-            for (int j = 0; j < PPT; ++j)
-              if (r < nr && ok[j])
-                Rl[(r * n_ph + ph) * bs + li[j]] =
-                    rank_one(j, q0 + r0 + r + g.nq * iv, ch_of(c) == PH_MAGNETIC ? 0 : 1);
-    }
-    else if (HX && n_r > 0) {
+    if constexpr (!FEW)
+      __syncthreads();
+    if (!FEW && HX && n_r > 0) {
       // R(k2, k1) blocks of 16 x 16: lane l supplies V[m0 + l/16][k2] and U[m0 + l/16][k1] and holds
       // rows k2 = 4 (l/16) + i (FP32) or l/16 + 4 i (FP64) of column k1 = l % 16.
-      // complex64 G: 256-thread tiles add eight walkers' FP32 products to FP64 sums, as their walker
+      // complex64 G: tiles of up to 256 threads add eight walkers' FP32 products to FP64 sums, as their walker
       // loop does; larger tiles, whose walker loop adds every walker, multiply in FP64.
-      constexpr bool kR32 = Shape::fp32 && TT == 256;
+      constexpr bool kR32 = Shape::fp32 && TT <= 256;
       using RT = std::conditional_t<kR32, float, double>;
-      using V4 = std::conditional_t<kR32, pair_f32x4, pair_f64x4>;
+      using V4 = typename Mfma16<RT>::acc_t;
       const int nt = (nc + 15) / 16, n_items = nr * n_r * nt * nt;
       const size_t row = uv_row;
       for (int it = wave; it < n_items; it += TT / 64) {
@@ -432,10 +461,10 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
             // R += V U = (Vx Ux - Vy Uy) + i (Vy Ux + Vx Uy)
             const C vv = live[i] ? v[i] : C{0, 0}, uu = live[i] ? u[i] : C{0, 0};
             const RT vr = vv.x, vi = vv.y, ur = uu.x, ui = uu.y;
-            fr = mma4(vr, ur, fr);
-            fi = mma4(vi, ur, fi);
-            fr = mma4(-vi, ui, fr);
-            fi = mma4(vr, ui, fi);
+            fr = Mfma16<RT>::mma(vr, ur, fr);
+            fi = Mfma16<RT>::mma(vi, ur, fi);
+            fr = Mfma16<RT>::mma(-vi, ui, fr);
+            fi = Mfma16<RT>::mma(vr, ui, fi);
             if (kR32 && (i % 2 == 1 || m0 + 4 * i + 4 >= n_walk)) {  // eight walkers per FP32 sum
 #pragma unroll
               for (int h = 0; h < 4; ++h) {
@@ -476,7 +505,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
                 continue;
               const int qv = q0 + r0 + r + g.nq * iv;
               old[k][i] = static_cast<const float4*>(g4_of(c0 + k))[own_index(kp[i], qv)];
-              if (img_p && ch_of(c0 + k) == PP_UP_DOWN)
+              if (!FEW && img_p && ch_of(c0 + k) == PP_UP_DOWN)
                 oldp[HZ ? i : 0] =
                     static_cast<const float4*>(g4_of(c0 + k))[swap_index(kp[i], qv, a.k_ex[q0 + r0 + r])];
             }
@@ -497,16 +526,19 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
               if (is_pp)
                 v = tz[j][r0 + r];
               else if (HX && (type == PH_MAGNETIC || type == PH_CHARGE)) {
-                v = Rl[(r * n_ph + ph) * bs + li[j]];
+                if constexpr (FEW)
+                  v = rank_one(j, r0 + r, type == PH_MAGNETIC ? 0 : 1);
+                else
+                  v = Rl[(r * n_ph + ph) * bs + li[j]];
                 v.x -= tx[j][r0 + r].x;
                 v.y -= tx[j][r0 + r].y;
               }
               else
                 v = double2{-tt[j][r0 + r].x, -tt[j][r0 + r].y};
               g4_put(g4, own_index(kp[i], qv), old[k][i], v, a.sum_mode);
-              if (!is_pp && (img_t || img_c))
+              if (!FEW && !is_pp && (img_t || img_c))
                 Rl[(r * n_ph + ph) * bs + li[j]] = v;
-              if (is_pp && img_p)
+              if (!FEW && is_pp && img_p)
                 g4_put(g4, swap_index(kp[i], qv, a.k_ex[q0 + r0 + r]), oldp[HZ ? i : 0], v, a.sum_mode);
             }
             ph += !is_pp;
@@ -515,7 +547,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET>::WAVES)
       for (int k = 0; k < CG && c0 + k < c_hi; ++k)
         ph0 += ch_of(c0 + k) != PP_UP_DOWN;
     }
-    if (n_ph == 0 || (!img_t && !img_c))
+    if (FEW || n_ph == 0 || (!img_t && !img_c))
       continue;
     __syncthreads();
     // Images of the particle-hole channels.
@@ -586,16 +618,38 @@ namespace {
 // Complex totals (pairs x momenta x terms, four registers each) that a thread may hold: 16; 8 where the loads
 // in flight need the others (complex128 G, or several pairs per thread, in a 1024-thread workgroup's 128
 // registers: 40 sites, magnetic and pp, complex64, 32 walkers, 32 frequencies, four momenta with 16
-// totals 1.13 ms, two with 8 0.58).
-constexpr int totals_limit(bool fp32, int threads, int ppt) { return threads == 1024 && (!fp32 || ppt > 1) ? 8 : 16; }
+// totals 1.13 ms, two with 8 0.58). With few walkers fewer groups save less reading: 12 or 8, and 2 where two
+// workgroups then share a CU (complex128, magnetic, 32 sites, four momenta: 1.16 of the time of two).
+constexpr int totals_limit(bool fp32, int threads, int ppt, int terms, bool few) {
+  if (few)
+    return threads == 1024 && ppt == 1 && terms == 1 ? 2 : threads == 704 || (ppt == 1 && (fp32 || threads < 1024)) ? 12 : 8;
+  return threads == 1024 && (!fp32 || ppt > 1) ? 8 : 16;
+}
+
+// Launches of fewer walkers than this take the FEW kernel, up to two pairs per thread (its registers hold
+// no more). Geometric means over the channel sets, against the other kernel: five walkers 4x4 0.92, 18 and 20
+// sites 0.85, 25 sites 0.80; eight walkers 4x4 1.1, 18 to 32 sites 0.9 - 1.0 (one channel, 25 sites,
+// complex64: 0.85), 36 sites and more 1.2.
+constexpr int few_walkers(int threads, int ppt) {
+  return ppt == 4 ? 0 : threads == 1024 && ppt == 1 ? 9 : threads == 256 && ppt == 2 ? 8 : 6;
+}
+constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
+
+template <typename Real, int TT, int PPT, int QG, int SET, bool FEW>
+void launch_pair_kernel(TiledArgs<Real> a, size_t lds, hipStream_t st) {
+  constexpr int terms = (SET & 1) + (SET >> 1 & 1) + (SET >> 2 & 1);
+  if constexpr (QG == 1 || PPT * QG * terms <= totals_limit(sizeof(Real) == 4, TT, PPT, terms, FEW)) {  // others are never chosen
+    const unsigned tiles = tile_schedule(a);
+    hipLaunchKernelGGL((g4_pair_kernel<Real, TT, PPT, QG, SET, FEW>), dim3(tiles), dim3(TT), lds, st, a);
+  }
+}
 
 template <typename Real, int TT, int PPT, int QG, int SET>
-void launch_pair_set(TiledArgs<Real> a, size_t lds, hipStream_t st) {
-  using Shape = PairShape<Real, TT, PPT, QG, SET>;
-  if constexpr (QG == 1 || Shape::TOTALS <= totals_limit(Shape::fp32, TT, PPT)) {  // others are never chosen
-    const unsigned tiles = tile_schedule(a);
-    hipLaunchKernelGGL((g4_pair_kernel<Real, TT, PPT, QG, SET>), dim3(tiles), dim3(TT), lds, st, a);
-  }
+void launch_pair_set(const TiledArgs<Real>& a, size_t lds, hipStream_t st) {
+  if constexpr (few_walkers(TT, PPT) > 0)
+    if (a.uv_lds >= 0)
+      return launch_pair_kernel<Real, TT, PPT, QG, SET, true>(a, lds, st);
+  launch_pair_kernel<Real, TT, PPT, QG, SET, false>(a, lds, st);
 }
 
 template <typename Real, int TT, int PPT, int QG>
@@ -610,13 +664,18 @@ void launch_pair_shape(const TiledArgs<Real>& a, int set, size_t lds, hipStream_
   }
 }
 
-// Workgroup shape: 256 threads while a thread owns at most 2 of the nc^2 (k1, k2) pairs,
-// 1024 threads (at most 4 pairs each) for larger clusters.
+// Workgroup shape: up to 256 threads while a thread owns at most 2 of the nc^2 (k1, k2) pairs, as few as
+// hold the pairs (8 sites in 256 threads, three waves of four idle: 1.6 times the time of 64), 1024 threads
+// (at most 4 pairs each) for larger clusters.
 struct TileShape {
   int threads, ppt;
 };
 TileShape tile_shape(int nc) {
   const int pairs = nc * nc;
+  if (pairs <= 64)
+    return {64, 1};
+  if (pairs <= 128)
+    return {128, 1};
   if (pairs <= 256)
     return {256, 1};
   if (pairs <= 512)
@@ -634,6 +693,7 @@ TileShape tile_shape(int nc) {
 
 }  // namespace
 
+#ifndef G4_TILED_FLOAT
 int tiled_pairs_per_thread(int nc) { return tile_shape(nc).ppt; }
 
 // Tile (w1, w2) of G4 reads the G blocks X = (w1, w2), Y = (w2 + v, w1 + v) and
@@ -704,9 +764,10 @@ std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>&
 size_t tiled_lds_bytes(const Geo& g, int n_ph, bool need_z, size_t cplx_bytes, int qg) {
   const size_t bs = static_cast<size_t>(g.nc) * (g.nc + 1);
   const TileShape ts = tile_shape(g.nc);
-  const int planes = (ts.threads == 256 && ts.ppt == 1 ? qg : 1) * (ts.ppt == 4 ? std::min(n_ph, 1) : n_ph);
+  const int planes = (ts.threads <= 256 && ts.ppt == 1 ? qg : 1) * (ts.ppt == 4 ? std::min(n_ph, 1) : n_ph);
   return bs * std::max(cplx_bytes * 2 * ((n_ph > 0 ? 1 : 0) + (need_z ? 1 : 0)), sizeof(double2) * planes);
 }
+#endif
 
 template <typename Real>
 bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
@@ -720,30 +781,48 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
     set |= a.ch[c] == PP_UP_DOWN ? HAS_Z : a.ch[c] == PH_MAGNETIC || a.ch[c] == PH_CHARGE ? HAS_X : HAS_T;
     n_ph += a.ch[c] != PP_UP_DOWN;
   }
-  // Momenta per workgroup: as many as the totals allow.
+  a.rank_one = (set & HAS_X) != 0;
   const int terms = set == (HAS_X | HAS_Z) ? 2 : set == HAS_X || set == HAS_Z ? 1 : set & HAS_Z ? 3 : 2;
-  int qg = g.nq >= 3 ? 4 : g.nq;
-  while (qg > 1 && ppt * qg * terms > totals_limit(sizeof(Real) == 4, ts.threads, ppt))
-    qg /= 2;
-  while (a.qg_cap > 0 && qg > a.qg_cap)
-    qg /= 2;
-  a.nqg = (g.nq + qg - 1) / qg;
-  // Where every tile is resident at once (four 256-thread workgroups per CU, one of 1024), half of
+  auto plan = [&](bool few) {  // LDS of the launch
+    // Momenta per workgroup: as many as the totals allow.
+    int qg = g.nq >= 3 ? 4 : g.nq;
+    while (qg > 1 && ppt * qg * terms > totals_limit(sizeof(Real) == 4, ts.threads, ppt, terms, few))
+      qg /= 2;
+    while (a.qg_cap > 0 && qg > a.qg_cap)
+      qg /= 2;
+    a.nqg = (g.nq + qg - 1) / qg;
+    a.qg = qg;
+    if (!few) {
+      a.uv_lds = -1;
+      return tiled_lds_bytes(g, n_ph, a.need_z, sizeof(Cplx<Real>), qg);
+    }
+    const size_t block = static_cast<size_t>(g.nc) * (g.nc + 1) * 2 * sizeof(Cplx<Real>);  // Y or Z, both spins
+    a.uv_lds = static_cast<int>(block * ((n_ph > 0 ? 1 : 0) + (a.need_z ? 1 : 0)));
+    return a.uv_lds + (a.rank_one ? sizeof(Cplx<Real>) * a.n_walkers * 4 * qg * g.nc : 0);
+  };
+  bool few = a.n_walkers < few_walkers(ts.threads, ppt);
+  size_t lds = plan(few);
+  if (few && lds > kLdsBytes) {
+    few = false;
+    lds = plan(few);
+  }
+  // Where every tile is resident at once (four workgroups of up to 256 threads per CU, one of 1024), half of
   // them take as long as all, and writing the images comes on top: 6x6, 16 walkers, 16 frequencies
   // (256 tiles) 183 us against 179; 24 frequencies 305 against 329.
-  if (a.sym >= SYM_CONJ &&
-      static_cast<size_t>(g.nw) * g.nw * g.nv * a.nqg <= (ts.threads == 256 ? size_t(1024) : size_t(256)))
+  if (few)
+    a.sym = SYM_NONE;
+  else if (a.sym >= SYM_CONJ &&
+           static_cast<size_t>(g.nw) * g.nw * g.nv * a.nqg <= (ts.threads <= 256 ? size_t(1024) : size_t(256)))
     a.sym = a.sym_few;
-  const size_t lds = tiled_lds_bytes(g, n_ph, a.need_z, sizeof(Cplx<Real>), qg);
-  if (set & HAS_X) {
+  if (a.rank_one) {
     const dim3 ug((g.nc * g.nw + 255) / 256, g.nq * g.nv, a.n_walkers);
     hipLaunchKernelGGL(uv_kernel<Real>, ug, dim3(256), 0, st, a);
   }
   auto by_qg = [&](auto tt, auto pp) {
     constexpr int TT = decltype(tt)::value, PP = decltype(pp)::value;
-    if (qg == 4)
+    if (a.qg == 4)
       launch_pair_shape<Real, TT, PP, (PP <= 2 ? 4 : 2)>(a, set, lds, st);
-    else if (qg == 2)
+    else if (a.qg == 2)
       launch_pair_shape<Real, TT, PP, 2>(a, set, lds, st);
     else
       launch_pair_shape<Real, TT, PP, 1>(a, set, lds, st);
@@ -751,7 +830,11 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
   using I256 = std::integral_constant<int, 256>;
   using I704 = std::integral_constant<int, 704>;
   using I1024 = std::integral_constant<int, 1024>;
-  if (ts.threads == 256 && ppt == 1)
+  if (ts.threads == 64)
+    by_qg(std::integral_constant<int, 64>{}, std::integral_constant<int, 1>{});
+  else if (ts.threads == 128)
+    by_qg(std::integral_constant<int, 128>{}, std::integral_constant<int, 1>{});
+  else if (ts.threads == 256 && ppt == 1)
     by_qg(I256{}, std::integral_constant<int, 1>{});
   else if (ts.threads == 256)
     by_qg(I256{}, std::integral_constant<int, 2>{});
@@ -766,7 +849,10 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
   return true;
 }
 
-template bool launch_g4_tiled<double>(TiledArgs<double>, hipStream_t);
+#ifdef G4_TILED_FLOAT
 template bool launch_g4_tiled<float>(TiledArgs<float>, hipStream_t);
+#else
+template bool launch_g4_tiled<double>(TiledArgs<double>, hipStream_t);
+#endif
 
 }  // namespace g4acc

@@ -780,14 +780,9 @@ void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
     a.tile_order = h->tile_order >= 0 ? h->tile_order : (n_walkers > 1 ? 2 : 0);
     a.tile_perm = h->d_tperm;
     a.sum_mode = h->sum_mode;
-    // One walker's launch is the G4 read-modify-write, which half of the tiles with scattered
-    // images does no faster (4x4, 8 transfers, three channels, 32 frequencies: 13.6 against 13.1 ms
-    // for 64 measurements); from two walkers on the tiles' reads and products count.
     a.half_g = own_g && h->half_g();
     a.sym_few = h->g4_sym && h->sym_ok ? SYM_TRANSPOSE : SYM_NONE;
-    // Where the transpose images are written anyway, the conjugate ones cost nothing more and half of G
-    // less is read.
-    a.sym = a.half_g && (n_walkers > 1 || a.sym_few == SYM_TRANSPOSE) ? h->conj_sym : a.sym_few;
+    a.sym = a.half_g ? h->conj_sym : a.sym_few;
     a.k_neg = h->d_kneg;
     a.sym_tiles = h->d_stab[a.tile_order == 0 ? 0 : 1];
     a.n_sym_tiles = h->n_stab;

@@ -153,6 +153,9 @@ struct TiledArgs {
   const int* k_neg = nullptr;       // device [Nc], index(-k); half_g only
   const int* sym_tiles = nullptr;   // computed tiles (w1 | w2 << 16) for sym >= SYM_CONJ, in dispatch order
   int n_sym_tiles = 0;
+  int qg = 0;                       // momenta per workgroup (set by the launcher)
+  bool rank_one = false;            // magnetic or charge among the channels (set by the launcher)
+  int uv_lds = -1;                  // few walkers: place of their rank-one factors in LDS (set by the launcher)
 };
 
 template <typename Real>
