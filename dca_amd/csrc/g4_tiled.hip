@@ -366,14 +366,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET, FEW>::W
   // plane is large (PPT = 4: up to 66.5 KB).
   constexpr int RB = TT <= 256 && PPT == 1 ? QG : 1;
   constexpr bool kOneCh = PPT == 4;
-  auto left_out = [&](int wa, int wb) {
-    return wa >= 0 && wa < nw && wb >= 0 && wb < nw && !sym_tile_computed(nw, nu, wa, wb, HY, HZ, a.sym);
-  };
-  const int c1 = nw - 1 - nu - w2, c2 = nw - 1 - nu - w1;  // C
-  const int p1 = nw - 1 + nu - w1, p2 = nw - 1 + nu - w2;  // P
-  const bool img_t = (a.sym & 1) && w1 != w2;
-  const bool img_c = a.sym == SYM_CONJ ? left_out(c1, c2) : a.sym == SYM_CONJ_TRANSPOSE && w1 + w2 != nw - 1;
-  const bool img_p = HZ && a.sym == SYM_CONJ && left_out(p1, p2);
+  const TileImages im = tile_images(nw, nu, w1, w2, HY, HZ, a.sym);
   double2* Rl = reinterpret_cast<double2*>(smem_raw);  // [momentum][particle-hole channel][k2][k1]
   auto g4_index = [&](int ka, int wa, int kb, int wb, int qv) {
     return ka + static_cast<size_t>(nc) *
@@ -383,7 +376,8 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET, FEW>::W
   // entries at once it would not fit beside the totals.
   auto own_index = [&](int kp, int qv) { return g4_index(kp & 0xffff, w1, kp >> 16, w2, qv); };
   auto swap_index = [&](int kp, int qv, int q) {
-    return g4_index(a.k_sub[(kp & 0xffff) + nc * q], p1, a.k_sub[(kp >> 16) + nc * q], p2, qv);
+    return g4_index(swap_momentum(nc, a.k_sub, q, kp & 0xffff), im.p1, swap_momentum(nc, a.k_sub, q, kp >> 16), im.p2,
+                    qv);
   };
   auto opaque = [](int v) {
     asm volatile("" : "+v"(v));
@@ -505,7 +499,7 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET, FEW>::W
                 continue;
               const int qv = q0 + r0 + r + g.nq * iv;
               old[k][i] = static_cast<const float4*>(g4_of(c0 + k))[own_index(kp[i], qv)];
-              if (!FEW && img_p && ch_of(c0 + k) == PP_UP_DOWN)
+              if (!FEW && im.p && ch_of(c0 + k) == PP_UP_DOWN)
                 oldp[HZ ? i : 0] =
                     static_cast<const float4*>(g4_of(c0 + k))[swap_index(kp[i], qv, a.k_ex[q0 + r0 + r])];
             }
@@ -536,9 +530,9 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET, FEW>::W
               else
                 v = double2{-tt[j][r0 + r].x, -tt[j][r0 + r].y};
               g4_put(g4, own_index(kp[i], qv), old[k][i], v, a.sum_mode);
-              if (!FEW && !is_pp && (img_t || img_c))
+              if (!FEW && !is_pp && (im.t || im.c))
                 Rl[(r * n_ph + ph) * bs + li[j]] = v;
-              if (!FEW && is_pp && img_p)
+              if (!FEW && is_pp && im.p)
                 g4_put(g4, swap_index(kp[i], qv, a.k_ex[q0 + r0 + r]), oldp[HZ ? i : 0], v, a.sum_mode);
             }
             ph += !is_pp;
@@ -547,14 +541,14 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET, FEW>::W
       for (int k = 0; k < CG && c0 + k < c_hi; ++k)
         ph0 += ch_of(c0 + k) != PP_UP_DOWN;
     }
-    if (FEW || n_ph == 0 || (!img_t && !img_c))
+    if (FEW || n_ph == 0 || (!im.t && !im.c))
       continue;
     __syncthreads();
     // Images of the particle-hole channels.
     for (int kind = 0; kind < 3; ++kind) {  // T, C, both
-      if (!(kind == 0 ? img_t : kind == 1 ? img_c : img_t && img_c))
+      if (!(kind == 0 ? im.t : kind == 1 ? im.c : im.t && im.c))
         continue;
-      const int wa = kind == 0 ? w2 : kind == 1 ? c1 : c2, wb = kind == 0 ? w1 : kind == 1 ? c2 : c1;
+      const int wa = kind == 0 ? w2 : kind == 1 ? im.c1 : im.c2, wb = kind == 0 ? w1 : kind == 1 ? im.c2 : im.c1;
       int ph0 = 0;
       for (int c0 = c_lo; c0 < c_hi; c0 += CG) {
 #pragma unroll
@@ -583,20 +577,8 @@ __global__ void __launch_bounds__(TT, (PairShape<Real, TT, PPT, QG, SET, FEW>::W
                 if (r >= nr || !ok[j])
                   continue;
                 const int k1 = kp[i] & 0xffff, k2 = kp[i] >> 16;
-                const int q = a.k_ex[q0 + r0 + r];
                 int s1, s2;
-                if (kind == 0) {
-                  s1 = a.k_sub[q + nc * k2];
-                  s2 = a.k_sub[q + nc * k1];
-                }
-                else if (kind == 1) {
-                  s1 = a.k_neg[a.k_add[k2 + nc * q]];
-                  s2 = a.k_neg[a.k_add[k1 + nc * q]];
-                }
-                else {
-                  s1 = a.k_neg[k1];
-                  s2 = a.k_neg[k2];
-                }
+                image_source(kind, nc, a.k_add, a.k_sub, a.k_neg, a.k_ex[q0 + r0 + r], k1, k2, s1, s2);
                 double2 v = Rl[(r * n_ph + ph) * bs + s2 * ld + s1];
                 if (kind != 0)
                   v.y = -v.y;
@@ -695,69 +677,6 @@ TileShape tile_shape(int nc) {
 
 #ifndef G4_TILED_FLOAT
 int tiled_pairs_per_thread(int nc) { return tile_shape(nc).ppt; }
-
-// Tile (w1, w2) of G4 reads the G blocks X = (w1, w2), Y = (w2 + v, w1 + v) and
-// Z = (v + nw - 1 - w1, v + nw - 1 - w2) (extended frequencies). The transpose of a tile holds its
-// Y block as X, its mirror (w -> nw - 1 - w) its Z block, and the neighbour along the diagonal
-// the next v. So a group is `strip` consecutive positions on the diagonals w1 - w2 = +d and -d
-// together with their mirror images; the workgroups resident on one XCD at a time cover a few
-// groups and find most of their blocks in its L2.
-std::vector<int> diagonal_tile_order(int nw, int strip) {
-  std::vector<int> out;
-  out.reserve(static_cast<size_t>(nw) * nw);
-  std::vector<char> seen(static_cast<size_t>(nw) * nw, 0);
-  for (int d = 0; d < nw; ++d)
-    for (int p0 = 0; p0 < nw - d; p0 += strip)
-      for (int sgn = 0; sgn < 2; ++sgn) {
-        if (d == 0 && sgn == 1)
-          continue;
-        for (int p = p0; p < std::min(p0 + strip, nw - d); ++p)
-          for (int mir = 0; mir < 2; ++mir) {
-            int w2 = p, w1 = p + d;
-            if (sgn)
-              std::swap(w1, w2);
-            if (mir) {
-              w1 = nw - 1 - w1;
-              w2 = nw - 1 - w2;
-            }
-            char& s = seen[w1 + static_cast<size_t>(nw) * w2];
-            if (s)
-              continue;
-            s = 1;
-            out.push_back(w1 | (w2 << 16));
-          }
-      }
-  return out;
-}
-
-std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>& w_ex, bool has_ph, bool has_pp,
-                                      int sym) {
-  std::vector<int> out;
-  auto used = [&](int w1, int w2) {
-    for (int nu : w_ex)
-      if (sym_tile_computed(nw, nu, w1, w2, has_ph, has_pp, sym))
-        return true;
-    return false;
-  };
-  // A tile's X block lies on the diagonal w1 - w2 = d, its Y block on -d and the conjugate of its Z
-  // block on d again, each shifted along it by v: strips of both diagonals together.
-  if (strip <= 0) {
-    for (int w2 = 0; w2 < nw; ++w2)
-      for (int w1 = 0; w1 < nw; ++w1)
-        if (used(w1, w2))
-          out.push_back(w1 | (w2 << 16));
-    return out;
-  }
-  for (int d = 0; d < nw; ++d)
-    for (int p0 = 0; p0 < nw - d; p0 += strip)
-      for (int sgn = 0; sgn < (d == 0 ? 1 : 2); ++sgn)
-        for (int p = p0; p < std::min(p0 + strip, nw - d); ++p) {
-          const int w1 = sgn ? p : p + d, w2 = sgn ? p + d : p;
-          if (used(w1, w2))
-            out.push_back(w1 | (w2 << 16));
-        }
-  return out;
-}
 
 // LDS of a workgroup: the staged blocks (both spins), or the rank-one planes of the particle-hole
 // channels that are finished together.

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "g4acc_common.hpp"
+#include "g4_tile_order.hpp"
 #include "g4acc_kernels.hpp"
 
 using namespace g4acc;

@@ -123,6 +123,44 @@ __host__ __device__ inline bool sym_tile_computed(int nw, int nu, int w1, int w2
          (has_pp && (nw - 1 + nu - hi < 0 || nw - 1 + nu - lo >= nw));
 }
 
+// The images that a computed tile (w1, w2) writes, and their tiles: t (w2, w1), c (c1, c2) and both
+// (c2, c1) of the particle-hole channels, p (p1, p2) of the pp channel.
+struct TileImages {
+  int c1, c2, p1, p2;
+  bool t, c, p;
+};
+__host__ __device__ inline TileImages tile_images(int nw, int nu, int w1, int w2, bool has_ph, bool has_pp, int sym) {
+  TileImages m{nw - 1 - nu - w2, nw - 1 - nu - w1, nw - 1 + nu - w1, nw - 1 + nu - w2, false, false, false};
+  auto left_out = [&](int a, int b) {
+    return a >= 0 && a < nw && b >= 0 && b < nw && !sym_tile_computed(nw, nu, a, b, has_ph, has_pp, sym);
+  };
+  m.t = (sym & 1) && w1 != w2;
+  m.c = sym == SYM_CONJ ? left_out(m.c1, m.c2) : sym == SYM_CONJ_TRANSPOSE && w1 + w2 != nw - 1;
+  m.p = has_pp && sym == SYM_CONJ && left_out(m.p1, m.p2);
+  return m;
+}
+
+// The pair (s1, s2) of the tile that entry (k1, k2) of an image holds, kind 0: T, 1: C (conjugated),
+// 2: both (conjugated); q is the exchange momentum.
+__host__ __device__ inline void image_source(int kind, int nc, const int* k_add, const int* k_sub, const int* k_neg,
+                                             int q, int k1, int k2, int& s1, int& s2) {
+  if (kind == 0) {
+    s1 = k_sub[q + nc * k2];
+    s2 = k_sub[q + nc * k1];
+  }
+  else if (kind == 1) {
+    s1 = k_neg[k_add[k2 + nc * q]];
+    s2 = k_neg[k_add[k1 + nc * q]];
+  }
+  else {
+    s1 = k_neg[k1];
+    s2 = k_neg[k2];
+  }
+}
+
+// The momentum of the pair-swap image that momentum k of the tile moves to.
+__host__ __device__ inline int swap_momentum(int nc, const int* k_sub, int q, int k) { return k_sub[k + nc * q]; }
+
 // Single-band, all channels in one launch (g4_tiled.hip). Returns false when the geometry is
 // outside what the tiled kernel handles (the caller then uses launch_g4 per channel).
 template <typename Real>
@@ -165,12 +203,6 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st);
 template <typename Real>
 bool launch_g4_band(TiledArgs<Real> a, hipStream_t st);
 int tiled_pairs_per_thread(int nc);
-// Tile schedule 2: (w1 | w2 << 16) for all nw^2 frequency pairs, in dispatch order.
-std::vector<int> diagonal_tile_order(int nw, int strip);
-// The tiles computed for any of the exchange frequencies under sym >= SYM_CONJ, on diagonal strips
-// (strip > 0) or w1 fastest (strip = 0).
-std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>& w_ex, bool has_ph, bool has_pp,
-                                      int sym);
 // LDS of one tile workgroup with momentum groups of qg and n_ph particle-hole channels.
 size_t tiled_lds_bytes(const Geo& g, int n_ph, bool need_z, size_t cplx_bytes, int qg);
 

@@ -24,3 +24,7 @@ mv "$HERE/_build/site_fft_test.tmp" "$HERE/_build/site_fft_test"
 g++ -std=c++17 -O2 -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__ -I/opt/rocm/include \
     "$HERE/sym_tiles_test.cpp" -o "$HERE/_build/sym_tiles_test.tmp"
 mv "$HERE/_build/sym_tiles_test.tmp" "$HERE/_build/sym_tiles_test"
+# Their images (index maps of the kernel) and dispatch order.
+g++ -std=c++17 -O2 -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__ -I/opt/rocm/include \
+    "$HERE/sym_images_test.cpp" -o "$HERE/_build/sym_images_test.tmp"
+mv "$HERE/_build/sym_images_test.tmp" "$HERE/_build/sym_images_test"
