@@ -1847,7 +1847,7 @@ int g4acc_set_tuning(g4acc_handle* h, const char* key, int value) {
     h->mtog_large = value;
   else if (k == "mtog_chunk" && value >= 0)
     h->mtog_chunk = value;
-  else if (k == "g4_sym" && (value == 0 || (value == 1 && h->sym_ok)))
+  else if (k == "g4_sym" && (value == 0 || (value == 1 && (h->sym_ok || h->conj_sym))))
     h->g4_sym = value;
   else if (k == "g4_qg" && (value == 0 || value == 1 || value == 2 || value == 4))
     h->g4_qg = value;

@@ -284,7 +284,7 @@ int g4acc_set_timing(g4acc_handle* h, int enable);
  * that output kept in LDS, the FP32 default), "mtog_chunk" (slots per M -> G pass, below the
  * number the workspace was sized for; 0: that number, a whole batch where its workspace fits
  * 24 GiB), "g4_sym" (0: all G4 tiles and all of G, instead of the part that the symmetries of the
- * handle's G leave; 1, accepted where the transpose symmetry alone applies: back to the default).
+ * handle's G leave; 1, accepted where it has one: back to the default).
  * Results do not depend on the tuning beyond FP32 summation order. */
 int g4acc_set_tuning(g4acc_handle* h, const char* key, int value);
 int g4acc_get_timing(const g4acc_handle* h, double* mtog_ms, double* g4_ms, long long* batches);
