@@ -44,34 +44,34 @@ inline std::vector<int> diagonal_tile_order(int nw, int strip) {
   return out;
 }
 
-// The tiles computed for any of the exchange frequencies under sym >= SYM_CONJ, on diagonal strips
-// (strip > 0) or w1 fastest (strip = 0).
-inline std::vector<int> symmetric_tile_order(int nw, int strip, const std::vector<int>& w_ex, bool has_ph, bool has_pp,
-                                      int sym) {
+// The tiles computed for any of the exchange frequencies under sym >= SYM_CONJ, by schedule: 0 w1 fastest, 1
+// super-tiles of 8 x 8, 2 diagonal strips.
+inline std::vector<int> symmetric_tile_order(int nw, int schedule, int strip, const std::vector<int>& w_ex, bool has_ph,
+                                             bool has_pp, int sym) {
   std::vector<int> out;
-  auto used = [&](int w1, int w2) {
+  auto add = [&](int w1, int w2) {
     for (int nu : w_ex)
-      if (sym_tile_computed(nw, nu, w1, w2, has_ph, has_pp, sym))
-        return true;
-    return false;
+      if (sym_tile_computed(nw, nu, w1, w2, has_ph, has_pp, sym)) {
+        out.push_back(w1 | (w2 << 16));
+        return;
+      }
   };
-  // A tile's X block lies on the diagonal w1 - w2 = d, its Y block on -d and the conjugate of its Z
-  // block on d again, each shifted along it by v: strips of both diagonals together.
-  if (strip <= 0) {
-    for (int w2 = 0; w2 < nw; ++w2)
-      for (int w1 = 0; w1 < nw; ++w1)
-        if (used(w1, w2))
-          out.push_back(w1 | (w2 << 16));
+  if (schedule < 2) {
+    const int side = schedule == 0 ? nw : 8;
+    for (int b2 = 0; b2 < nw; b2 += side)
+      for (int b1 = 0; b1 < nw; b1 += side)
+        for (int w2 = b2; w2 < std::min(b2 + side, nw); ++w2)
+          for (int w1 = b1; w1 < std::min(b1 + side, nw); ++w1)
+            add(w1, w2);
     return out;
   }
+  // A tile's X block lies on the diagonal w1 - w2 = d, its Y block on -d and the conjugate of its Z
+  // block on d again, each shifted along it by v: strips of both diagonals together.
   for (int d = 0; d < nw; ++d)
     for (int p0 = 0; p0 < nw - d; p0 += strip)
       for (int sgn = 0; sgn < (d == 0 ? 1 : 2); ++sgn)
-        for (int p = p0; p < std::min(p0 + strip, nw - d); ++p) {
-          const int w1 = sgn ? p : p + d, w2 = sgn ? p + d : p;
-          if (used(w1, w2))
-            out.push_back(w1 | (w2 << 16));
-        }
+        for (int p = p0; p < std::min(p0 + strip, nw - d); ++p)
+          add(sgn ? p : p + d, sgn ? p + d : p);
   return out;
 }
 

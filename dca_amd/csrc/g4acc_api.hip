@@ -170,12 +170,12 @@ struct g4acc_handle {
   int g4_qg = 0;                   // tuning: momenta per G4 workgroup (0: register limit)
   // tuning: g4_sym = 0 computes every G4 tile. sym_ok: the transpose symmetry alone applies (one
   // q = 0, one v = 0, channels among magnetic, charge, transverse). conj_sym: G4Sym of handles
-  // whose G is conjugate symmetric (SYM_NONE otherwise), their inversion table and tile tables in
-  // natural and diagonal order.
+  // whose G is conjugate symmetric (SYM_NONE otherwise), their inversion table and tile tables of
+  // the three schedules.
   int g4_sym = 0;
   bool sym_ok = false;
   int conj_sym = SYM_NONE;
-  int *d_kneg = nullptr, *d_stab[2] = {nullptr, nullptr};
+  int *d_kneg = nullptr, *d_stab[3] = {nullptr, nullptr, nullptr};
   int n_stab = 0;
   // This device's address of the static workspace of g4acc_compute_G_noalloc.
   unsigned char* d_scratch = nullptr;
@@ -402,6 +402,14 @@ bool conjugate_symmetric(const Geo& g, const g4acc_geometry* gm, double tol, con
           return false;
       }
   return true;
+}
+
+// Tile table of a conjugate symmetric handle for one schedule.
+std::vector<int> symmetric_tiles(const g4acc_handle* h, int schedule, int strip) {
+  bool has_ph = false, has_pp = false;
+  for (int c : h->channels)
+    (c == G4ACC_PARTICLE_PARTICLE_UP_DOWN ? has_pp : has_ph) = true;
+  return symmetric_tile_order(h->g.nw, schedule, strip, h->w_ex, has_ph, has_pp, h->conj_sym);
 }
 
 // One walker's inputs as the staging reads them. The real walker (g4acc_walker), the CT-AUX
@@ -785,7 +793,7 @@ void run_g4(g4acc_handle* h, int n_walkers, bool own_g = true) {
     a.sym_few = h->g4_sym && h->sym_ok ? SYM_TRANSPOSE : SYM_NONE;
     a.sym = a.half_g ? h->conj_sym : a.sym_few;
     a.k_neg = h->d_kneg;
-    a.sym_tiles = h->d_stab[a.tile_order == 0 ? 0 : 1];
+    a.sym_tiles = h->d_stab[a.tile_order == 0 || a.tile_order == 1 ? a.tile_order : 2];
     a.n_sym_tiles = h->n_stab;
     if (launch_g4_tiled<Real>(a, h->stream))
       return;
@@ -1175,14 +1183,14 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
       table(&h->d_kneg, neg);
     if (inv && h->use_tiled && getenv("G4ACC_NO_SYM") == nullptr &&
         conjugate_symmetric(g, gm, dp ? 16 * eps : 0x1p-30, neg)) {
-      bool has_ph = false, has_pp = false, self = g.nv == 1 && gm->w_ex[0] == 0;
+      bool self = g.nv == 1 && gm->w_ex[0] == 0;
       for (int c : h->channels)
-        (c == G4ACC_PARTICLE_PARTICLE_UP_DOWN ? has_pp : has_ph) = true;
+        self = self && c != G4ACC_PARTICLE_PARTICLE_UP_DOWN;
       for (int q : h->k_ex)
         self = self && neg[q] == q;
-      h->conj_sym = self && !has_pp ? SYM_CONJ_TRANSPOSE : SYM_CONJ;
-      for (int k = 0; k < 2; ++k) {  // w1 fastest, and on diagonal strips of two
-        const std::vector<int> t = symmetric_tile_order(g.nw, 2 * k, h->w_ex, has_ph, has_pp, h->conj_sym);
+      h->conj_sym = self ? SYM_CONJ_TRANSPOSE : SYM_CONJ;
+      for (int k = 0; k < 3; ++k) {
+        const std::vector<int> t = symmetric_tiles(h, k, 2);
         h->n_stab = static_cast<int>(t.size());
         table(&h->d_stab[k], t);
       }
@@ -1860,11 +1868,14 @@ int g4acc_set_tuning(g4acc_handle* h, const char* key, int value) {
   else if (k == "g4_tile_strip" && value >= 1 && value <= 16) {
     // Diagonal positions per group of schedule 2 (table uploaded now, outside any batch).
     const std::vector<int> tperm = diagonal_tile_order(h->g.nw, value);
-    int rs;
-    if ((rs = h->check(hipSetDevice(h->device), "hipSetDevice")) ||
-        (rs = h->check(hipMemcpy(h->d_tperm, tperm.data(), tperm.size() * sizeof(int), hipMemcpyHostToDevice),
-                       "hipMemcpy")))
-      return rs;
+    G4_TRY(h->check(hipSetDevice(h->device), "hipSetDevice"));
+    G4_TRY(quiesce(h));
+    G4_TRY(h->check(hipMemcpy(h->d_tperm, tperm.data(), tperm.size() * sizeof(int), hipMemcpyHostToDevice),
+                    "hipMemcpy"));
+    if (h->conj_sym) {
+      const std::vector<int> t = symmetric_tiles(h, 2, value);
+      G4_TRY(h->check(hipMemcpy(h->d_stab[2], t.data(), t.size() * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy"));
+    }
   }
   else if (k == "graph" && (value == 0 || value == 1))
     h->use_graph = value != 0;

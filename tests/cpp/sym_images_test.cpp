@@ -55,10 +55,10 @@ static int check(const Torus& t, int nw, const std::vector<int>& w_ex, int q, bo
           g[a + static_cast<size_t>(D) * b] = g[a + static_cast<size_t>(D) * b].real();
       }
   }
-  const std::vector<int> order0 = symmetric_tile_order(nw, 0, w_ex, ph, pp, sym);
+  const std::vector<int> order0 = symmetric_tile_order(nw, 0, 2, w_ex, ph, pp, sym);
   int bad = 0;
-  for (int strip : {0, 1, 2, 5}) {
-    std::vector<int> o = symmetric_tile_order(nw, strip, w_ex, ph, pp, sym), r = order0;
+  for (auto [schedule, strip] : {std::pair<int, int>{0, 2}, {1, 2}, {2, 1}, {2, 2}, {2, 5}}) {
+    std::vector<int> o = symmetric_tile_order(nw, schedule, strip, w_ex, ph, pp, sym), r = order0;
     std::sort(o.begin(), o.end());
     std::sort(r.begin(), r.end());
     bad += o != r || std::unique(o.begin(), o.end()) != o.end();
@@ -139,6 +139,13 @@ int main() {
         for (int nw : {2, 6})
           bad += check(t, nw, {0}, q, true, false, SYM_CONJ_TRANSPOSE);
     }
+  // Each schedule and strip is an order of its own, over the same tiles.
+  std::vector<std::vector<int>> orders;
+  for (auto [schedule, strip] : {std::pair<int, int>{0, 2}, {1, 2}, {2, 1}, {2, 2}, {2, 5}}) {
+    orders.push_back(symmetric_tile_order(24, schedule, strip, {0, 1}, true, true, SYM_CONJ));
+    for (size_t i = 0; i + 1 < orders.size(); ++i)
+      bad += orders[i] == orders.back() || orders[i].size() != orders.back().size();
+  }
   if (!bad)
     std::printf("OK\n");
   return bad != 0;

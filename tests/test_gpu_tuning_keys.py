@@ -47,3 +47,18 @@ def test_g4_sym_is_refused_without_a_symmetry():
     with pytest.raises(g4acc.LogicError, match="g4_sym"):
         acc.set_tuning(g4_sym=1)
     acc.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_tile_schedules_and_strips_of_the_symmetric_tiles(precision):
+    """Every schedule and strip, set between batches of one handle: each tile sums the same products in the same
+    order wherever it runs, so the results are equal bit for bit."""
+    wl = _workload()
+    ms = wl.draw(12)
+    acc = g4acc.TpAccumulator(wl.geometry, precision=precision, max_walkers=12, max_vertices=wl.n_max, tuned=False)
+    first = _run(acc, ms)
+    for order, strip in ((0, 2), (1, 2), (2, 1), (2, 5), (2, 16), (-1, 2)):
+        acc.set_tuning(g4_tile_strip=strip, g4_tile_order=order)
+        for a, b in zip(first, _run(acc, ms)):
+            assert np.array_equal(a, b)
+    acc.close()
