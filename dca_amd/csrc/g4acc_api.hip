@@ -385,8 +385,7 @@ bool find_inversion(const Geo& g, const g4acc_geometry* gm, double dft_tol, std:
 }
 
 // Whether G(-p1, -p2) = conj G(p1, p2) for real M: G0(-p) = conj G0(p) and the band phases likewise, to
-// `tol` of |G0|, so that the conjugate stands for an entry that differs from it by less than G's own
-// rounding. A G0 without the symmetry (or holding a NaN) fails the test, and every tile is computed.
+// `tol` of |G0|. A G0 without the symmetry (or holding a NaN) fails the test, and every tile is computed.
 bool conjugate_symmetric(const Geo& g, const g4acc_geometry* gm, double tol, const std::vector<int>& neg) {
   const int nc = g.nc;
   if (gm->band_phase)
@@ -1171,18 +1170,20 @@ int g4acc_create_model(const g4acc_geometry* gm, const g4acc_options* opt, const
                   c == G4ACC_PARTICLE_HOLE_TRANSVERSE);
     h->sym_ok = ok && getenv("G4ACC_NO_SYM") == nullptr;
   }
-  // Inversion of the momenta (real M) and conjugate symmetry of G (single band). Tolerances: complex64
-  // G rounds at 2^-24, so 2^-30 of G0 does not show; complex128 G allows 16 roundings of G0 itself.
-  // The L x L transforms of the fused kernels do not read the DFT table; the others do.
+  // Inversion of the momenta (real M) and conjugate symmetry of G (single band). Tolerances: complex64 G
+  // rounds at 2^-24, so 2^-30 of G0 does not show; complex128 G takes the conjugate of an entry for its
+  // partner only where the partner's own G0 is that conjugate exactly. The L x L transforms of the fused
+  // kernels do not read the DFT table; the others do, and 4 eps is what cos and sin of the same angle differ
+  // by (8 sites 3.3; tables from rounded angles, 3x3 32 eps and more, are used as they are).
   if (!h->complex_m) {
     const bool dp = h->precision == G4ACC_FP64;
     const double eps = 2.220446049250313e-16;
     std::vector<int> neg;
-    const bool inv = find_inversion(g, gm, dp && !(h->fused_mtog && h->grid_L) ? 64 * eps : 1e-9, neg);
+    const bool inv = find_inversion(g, gm, dp && !(h->fused_mtog && h->grid_L) ? 4 * eps : 1e-9, neg);
     if (inv)
       table(&h->d_kneg, neg);
     if (inv && h->use_tiled && getenv("G4ACC_NO_SYM") == nullptr &&
-        conjugate_symmetric(g, gm, dp ? 16 * eps : 0x1p-30, neg)) {
+        conjugate_symmetric(g, gm, dp ? 0 : 0x1p-30, neg)) {
       bool self = g.nv == 1 && gm->w_ex[0] == 0;
       for (int c : h->channels)
         self = self && c != G4ACC_PARTICLE_PARTICLE_UP_DOWN;
