@@ -539,26 +539,29 @@ void launch_mtog(const MtoGArgs<Real>& a, hipStream_t st) {
       hipLaunchKernelGGL(dft_left_kernel<Real>, dim3((g.D + 255) / 256, a.n_max, ns), dim3(256), 0, st,
                          a.desc, g, a.n_max, s0, a.dft, a.B, a.A);
     }
-    // S4 from LDS where a block's rows of E fit half of a CU's; with real M and the momenta's inverses S3
-    // then forms half of the frequency pairs.
+    // S4 from LDS where eight momenta and more share a block's rows and the workgroups fill the card; with
+    // real M and the momenta's inverses S3 then forms half of the frequency pairs. M -> G against S4 without LDS
+    // and all of S3, 32 frequencies, 8 walkers: 3 bands, 8 sites 0.93 (8 frequencies 1.28), 10 sites 0.8 - 0.95;
+    // it loses at 4 sites (2 to 4 bands 1.0 - 1.2), with 4 bands, and with 2 in complex64 (1.08).
     const size_t el = sizeof(Cplx<Real>) * g.n_orb * (64 * static_cast<size_t>(g.nb) + 1);
-    const bool shared = el <= 81920;
+    const dim3 gs((g.nc * g.nwE + 63) / 64, g.nwE, ns);
+    const bool shared = el <= 81920 && g.nc >= 8 && (g.nb == 1 || g.nb == 3 || (g.nb == 2 && sizeof(Real) == 8)) &&
+                        g.nwE >= 16 && static_cast<size_t>(gs.x) * gs.y * gs.z >= 512;
     const bool mirror = shared && a.real_m && a.kneg && a.w_sum_min == 0;
     const int sum_min = mirror ? g.nwE - 1 : a.w_sum_min;
     hipLaunchKernelGGL(ndft_right_kernel<Real>, dim3((g.D + 255) / 256, g.D, ns), dim3(256), 0, st,
                        a.desc, g, a.n_max, s0, sum_min, a.off2, a.T2, a.A, a.E);
     if (shared) {
-      const dim3 gs((g.nc * g.nwE + 63) / 64, g.nwE, ns);
       auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, gs, dim3(256), el, st, g, s0, sum_min, mirror, a.dft, a.bphase, a.G0, a.kneg, a.E,
                            a.G);
       };
-      switch (g.nb) {
-        case 1: run(dft_right_G_shared<Real, 1>); break;
-        case 2: run(dft_right_G_shared<Real, 2>); break;
-        case 3: run(dft_right_G_shared<Real, 3>); break;
-        default: run(dft_right_G_shared<Real, 4>); break;
-      }
+      if (g.nb == 1)
+        run(dft_right_G_shared<Real, 1>);
+      else if (g.nb == 3)
+        run(dft_right_G_shared<Real, 3>);
+      else if constexpr (sizeof(Real) == 8)
+        run(dft_right_G_shared<Real, 2>);
       continue;
     }
     const int KW = g.nc * g.nwE;

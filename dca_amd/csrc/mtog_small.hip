@@ -464,9 +464,28 @@ void launch_small(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st) {
 
 }  // namespace
 
+namespace {
+
+// Vertices up to which the register-fused kernels are the faster ones: there the products are few and the
+// time is the writing of G, which they do with less per tile. Each against the other at that count, M -> G:
+// 8 sites, complex128, 64 frequencies, 8 walkers: 8 vertices 1.5, 48 1.05; 32 frequencies, 48 walkers: 8
+// 1.44, 48 1.06; with little G to write (8 frequencies, 8 walkers) 8 1.05, 16 1.0, 48 0.65.
+template <typename Real>
+int mtog_small_min_vertices(const Geo& g, int ns) {
+  constexpr bool dp = sizeof(Real) == 8;
+  const bool writes = static_cast<size_t>(g.D) * g.D * ns * sizeof(Cplx<Real>) >= size_t(32) << 20;
+  switch (g.nc) {
+    case 4: return writes ? 24 : 8;
+    case 8: return writes ? (dp ? 80 : 40) : (dp ? 12 : 0);
+    default: return writes ? (dp ? 24 : 32) : (dp ? 8 : 0);
+  }
+}
+
+}  // namespace
+
 template <typename Real>
 bool launch_mtog_small(const MtoGArgs<Real>& a, int s0, int ns, hipStream_t st) {
-  if (a.n_max > mtog_small_max_vertices(a.g.nc))
+  if (a.n_max <= mtog_small_min_vertices<Real>(a.g, ns) || a.n_max > mtog_small_max_vertices(a.g.nc))
     return false;
   const bool torus = a.kmap && a.grid_L * a.grid_L == a.g.nc;
   switch (a.g.nc) {
