@@ -389,12 +389,14 @@ __global__ void __launch_bounds__(256) dft_right_G_shared(Geo g, int slot0, int 
   const int s = slot & 1;
   const int nc = g.nc, KW = nc * g.nwE;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int kw1 = blockIdx.x * 64 + lane, w2 = blockIdx.y;
-  if (w2 + (static_cast<int>(blockIdx.x) * 64 + 63) / nc < w_sum_min)
+  // Rows rotate with the column and slot: those with few needed pairs would otherwise share their XCDs.
+  const int bx = static_cast<int>((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
+  const int kw1 = bx * 64 + lane, w2 = blockIdx.y;
+  if (w2 + (bx * 64 + 63) / nc < w_sum_min)
     return;
   const C* Es = E + static_cast<size_t>(blockIdx.z) * g.D * g.D + static_cast<size_t>(g.D) * g.n_orb * w2 +
-                static_cast<size_t>(blockIdx.x) * R;
-  const int rows = min(R, g.D - static_cast<int>(blockIdx.x) * R);
+                static_cast<size_t>(bx) * R;
+  const int rows = min(R, g.D - bx * R);
 #pragma unroll 4
   for (int i = threadIdx.x; i < g.n_orb * R; i += 256) {
     const int row = i % R, col = i / R;

@@ -343,10 +343,12 @@ __global__ void __launch_bounds__(256) mtog_right_small(Geo g, int n_max, int sl
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int part = wave % TL::SPLIT;
-  const int p0 = (blockIdx.x * TL::TPW + wave / TL::SPLIT) * 16;
+  // Rows rotate with the slot, as those with few needed frequencies would otherwise share their XCDs.
+  const int bx = static_cast<int>((blockIdx.x + blockIdx.z) % gridDim.x);
+  const int p0 = (bx * TL::TPW + wave / TL::SPLIT) * 16;
   const int n_wt = (g.nwE + 15) / 16;
   // The first frequency tile that reaches w_sum_min with the workgroup's highest row.
-  const int w_first = w_sum_min - 15 - static_cast<int>((blockIdx.x + 1) * (16 * TL::TPW) - 1) / NC;
+  const int w_first = w_sum_min - 15 - ((bx + 1) * (16 * TL::TPW) - 1) / NC;
   const int wt_first = w_first > 0 ? (w_first + 15) / 16 : 0;
   if (wt_first + static_cast<int>(blockIdx.y) >= n_wt)
     return;
