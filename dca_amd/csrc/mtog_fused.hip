@@ -114,17 +114,19 @@ __global__ void __launch_bounds__(256) mtog_right_fused(const SlotDesc* __restri
   const int s = slot & 1;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int p1 = blockIdx.x * 64 + lane;
+  // Rows rotate with the slot, as those with few needed pairs would otherwise share their XCDs.
+  const int bx = static_cast<int>((blockIdx.x + blockIdx.z) % gridDim.x);
+  const int p1 = bx * 64 + lane;
   const int w2wg = blockIdx.y * WT;           // first frequency of the workgroup
   const int w2b = w2wg + wave * TW;           // first frequency of this wave
-  if (w2wg + WT - 1 + (static_cast<int>(blockIdx.x) * 64 + 63) / NC < w_sum_min)
+  if (w2wg + WT - 1 + (bx * 64 + 63) / NC < w_sum_min)
     return;
   const int n = desc[slot].n;
   const bool active = p1 < g.D && w2b < g.nwE;
   const int* O = off + static_cast<size_t>(slot) * (NC + 1);
   const C* Ts = T + static_cast<size_t>(slot) * g.nwE * n_max;
-  const C* Ab = A + static_cast<size_t>(blockIdx.z) * g.D * n_max + static_cast<size_t>(blockIdx.x) * 64;
-  const int rows = g.D - blockIdx.x * 64;     // valid p1 rows of the workgroup
+  const C* Ab = A + static_cast<size_t>(blockIdx.z) * g.D * n_max + static_cast<size_t>(bx) * 64;
+  const int rows = g.D - bx * 64;     // valid p1 rows of the workgroup
 
   for (int i = threadIdx.x; i < NC * NC; i += 256)
     Dl[i] = dft[i];
