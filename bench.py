@@ -123,20 +123,35 @@ def run_batches(acc, batches, steps):
             acc._check(rc)
 
 
+def half_of_g(g):
+    """Whether the mixed form computes and reads only the blocks of G with w1 + w2 >= nwE - 1: the
+    single-band tiled handles (every workload's G0 is conjugate symmetric at complex64)."""
+    return g.nb == 1 and g.nc >= 8
+
+
+def g_entries(g):
+    """Entries of G per slot that the mixed form forms and reads."""
+    nwE = g.n_ext
+    return g.D * g.D * (nwE + 1) // (2 * nwE) if half_of_g(g) else g.D * g.D
+
+
 def mtog_flops(g, n):
     """FP operations of the M -> G algorithm this library runs, per slot of n vertices (complex
     multiply-add = 8, real x complex = 4; a site transform of Nc points as an L x L FFT,
-    5 Nc log2 Nc, or as a dense Nc x Nc product, 8 Nc^2)."""
+    5 Nc log2 Nc, or as a dense Nc x Nc product, 8 Nc^2). M is real: the left half is formed at the
+    positive frequencies, the right one for the pairs with w1 + w2 >= nwE - 1; their conjugates are
+    the other halves."""
     import math
     nwE, nc, D = g.n_ext, g.nc, g.D
     L = int(round(math.sqrt(nc)))
     fft = L * L == nc and L in (2, 4, 8) and g.nb == 1
     site = 5 * nc * math.log2(nc) if fft else 8 * nc * nc
-    return (4 * nwE * n * n            # S1: left NDFT (real M)
-            + nwE * n * g.nb * site    # S2: left site transform
-            + 8 * D * n * nwE          # S3: right NDFT
-            + D * nwE * g.nb * site    # S4: right site transform
-            + 12 * D * D)              # G = -G0 M~ G0 + beta G0 delta
+    right = (nwE + 1) / (2 * nwE)
+    return (4 * nwE * n * n / 2        # S1: left NDFT (real M)
+            + nwE * n * g.nb * site / 2  # S2: left site transform
+            + 8 * D * n * nwE * right  # S3: right NDFT
+            + D * nwE * g.nb * site * right  # S4: right site transform
+            + 12 * g_entries(g))       # G = -G0 M~ G0 + beta G0 delta
 
 
 def time_config(cfg, steps, warmup, walkers, pool_n, plain_steps, torch, keep_sample=0, fixed_n=0,
@@ -249,14 +264,13 @@ def roofline(cfg, ctx):
     from dca_amd import geometry as geo
     g, W = ctx["g"], ctx["W"]
     mtog_ms, g4_ms = ctx["mtog_ms"], ctx["g4_ms"]
-    D = g.D
-    # G4 stage: one FP64 complex read + write of every G4 entry plus one read of every walker's
-    # G (complex64, both spins).
-    g4_bytes = len(g.channels) * 32 * g.g4_size() + W * 2 * D * D * 8
+    # G4 stage: one FP64 complex read + write of every G4 entry plus one read of the part of every
+    # walker's G that is formed (complex64, both spins).
+    g4_bytes = len(g.channels) * 32 * g.g4_size() + W * 2 * g_entries(g) * 8
     g4_gbs = g4_bytes / (g4_ms * 1e-3) / 1e9
-    # M -> G stage: compulsory bytes (M in, G out as complex64) and this library's flops.
+    # M -> G stage: compulsory bytes (M in, that part of G out as complex64) and this library's flops.
     pool = ctx["pool"][:W]
-    mtog_bytes = sum(8 * n * n + 8 * n for m in pool for n in m.n) + W * 2 * D * D * 8
+    mtog_bytes = sum(8 * n * n + 8 * n for m in pool for n in m.n) + W * 2 * g_entries(g) * 8
     mtog_gbs = mtog_bytes / (mtog_ms * 1e-3) / 1e9
     flops = sum(mtog_flops(g, n) for m in pool for n in m.n)
     mtog_tf = flops / (mtog_ms * 1e-3) / 1e12
@@ -266,7 +280,8 @@ def roofline(cfg, ctx):
     if g4_ms >= mtog_ms:
         return {"bound": "hbm", "achieved": round(g4_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(g4_gbs / HBM_PEAK_GBS, 4), "traffic": g4_traffic,
-                "kernel": "G4 update stage (uv_kernel + g4_tiled_kernel per batch)",
+                "kernel": "G4 update stage (" + ("uv_kernel + g4_pair_kernel" if g.nb == 1 else
+                                                 "g4_band_kernel") + " per batch)",
                 "dominant_stage": "g4", "algorithmic_bytes_per_launch": g4_bytes,
                 "traffic_source": g4_src,
                 "other_stage": {"stage": "mtog", "ms": round(mtog_ms, 4), "achieved_tflops": round(mtog_tf, 2),

@@ -2,8 +2,8 @@
 
 For a workload and a batch size it measures, with the library's own HIP-event stage timing on
 its stream, every candidate of each tunable of include/g4acc.h (g4acc_set_tuning):
-  mtog_tw        frequencies per thread of the fused single-band M -> G kernel (M -> G stage)
-  mtog_mfma      right half of that kernel on the matrix cores (complex64, Nc <= 16)
+  mtog_tw        frequencies per thread of the register-fused single-band M -> G kernel (M -> G stage)
+  mtog_mfma      M -> G of 4 and 8 sites and the 4x4 torus on the matrix cores, in either precision
   g4_qg          momenta per G4 workgroup                                        (G4 stage)
   g4_tile_order  natural, XCD-aware super-tile or diagonal-strip tile schedule   (G4 stage)
 The stages are independent, so each is tuned on its own (the G4 knobs jointly). Results go to a
@@ -77,8 +77,8 @@ def tune(cfg: int, walkers: int, precision: str, reps: int = 4, log=print) -> di
     _stage_times(acc, batches, 1)  # warm up
     measured = {"mtog": {}, "g4": {}}
     best_tw, best_mm, best_t = 0, 0, float("inf")
-    # The matrix-core kernel has one shape (mtog_tw does not apply to it); where it does not
-    # apply (complex128, Nc > 16) the setting falls back to the vector kernel and measures alike.
+    # The matrix-core kernels have one shape (mtog_tw does not apply to them). Where they do not apply
+    # (other clusters, vertex counts outside their range) both settings run the same kernels.
     for mm, tw in [(0, tw) for tw in CANDIDATES["mtog_tw"]] + [(1, 0)]:
         acc.set_tuning(mtog_tw=tw, mtog_mfma=mm)
         t, _ = _stage_times(acc, batches, reps)

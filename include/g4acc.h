@@ -269,14 +269,14 @@ int g4acc_set_timing(g4acc_handle* h, int enable);
 /* Launch-shape tuning (no counterpart in the reference, whose launch shapes are fixed; set by
  * the autotuner's table, dca_amd/autotune.py). Keys: "mtog_tw" (frequencies per thread of the
  * fused single-band M -> G kernel: 0 default, 1, 2, 4, 8), "mtog_mfma" (1: M -> G on the matrix
- * cores for 4 and 8 sites and the 4x4 torus, max_vertices <= 4 (128 - Nc), the default there;
- * 0: the fused kernel), "g4_qg" (momenta per G4 workgroup:
- * 0 = as many as registers allow, 1, 2, 4), "g4_tile_order" (-1 by batch size: 2 for batches, 0 for
- * one walker; 0 natural,
- * 1 XCD-aware super-tiles, 2 XCD-aware diagonal strips with their mirror images),
- * "g4_tile_strip" (diagonal positions per group of schedule 2: 1..16, default 2), "g4_mfma" and
- * "g4_rank1" (accepted and without effect: the single-band tile kernel always forms the rank-one
- * MAGNETIC / CHARGE terms on the matrix cores),
+ * cores for 4 and 8 sites and the 4x4 torus, where max_vertices <= 4 (128 - Nc) and above the counts,
+ * 8 to 80, up to which the fused kernel is faster; the default there. 0: the fused kernel), "g4_qg"
+ * (momenta per G4 workgroup: 0 = as many as registers allow, 1, 2, 4), "g4_tile_order" (-1 by batch
+ * size: 2 for batches, 0 for one walker; 0 natural, 1 XCD-aware super-tiles, 2 XCD-aware
+ * diagonal strips with their mirror images), "g4_tile_strip" (diagonal positions per group of
+ * schedule 2: 1..16, default 2), "g4_mfma" and "g4_rank1" (accepted and without effect: the
+ * single-band tile kernel forms the rank-one MAGNETIC / CHARGE terms on the matrix cores for
+ * batches and on the vector units for few walkers),
  * "graph" (1: replay captured batch sequences, 0: launch eagerly), "mtog_large" (6x6 and 8x8 tori:
  * 0 register-fused M -> G kernels; 1 matrix-core S1/S3 with a D x D workspace per slot of a chunk
  * for S3's output, the FP64 default, in FP32 only when the environment variable G4ACC_MTOG_E was
