@@ -17,19 +17,18 @@
 // 16 x 16 blocks of it on the matrix cores after the walker loop, so they cost no vector
 // instructions per walker and no buffer of G4's size.
 //
-// What bounds it: the blocks read from L2 and beyond (4x4, three channels, 256 walkers, 64
-// frequencies, 4 q, 3 v: 20 GB in 2.8 ms; the same block pattern alone reads 7.4 TB/s), with the
-// vector ALUs 60 % busy beside it. So each block is read once per walker for all the momenta whose
+// What bounds it: the blocks read from L2 and beyond, with the vector ALUs half busy beside it (4x4, three
+// channels, 256 walkers, 64 frequencies, 4 q, 3 v: 2.88 ms, 24.6 GB asked of L2, 13.3 GB of that from
+// beyond it, vector ALUs 52 %). So each block is read once per walker for all the momenta whose
 // totals fit the registers. The next walkers' loads are in flight during a walker's products; every
 // load is issued (idle slots and walkers past the batch re-read valid elements).
 // Per batch (256 walkers) the stage went from 3.64 ms, with the rank-one terms in a buffer of G4's
 // size, to 2.9 ms; 6x6 (64 walkers, 64 frequencies, 4 q, 2 v) from 10.6 to 4.6 ms.
-// Launches of few walkers (up to five, on 17..32 sites up to eight) are the G4 read-modify-write with little
-// before it (FEW): all tiles, without images, the rank-one factors staged in LDS beside the blocks, and one
-// entry (complex128 G in small tiles: four) loaded before it is stored. With the code for many walkers
-// (images, factors read from memory in the tail, twelve entries in flight) a launch took, 4x4, three channels, 64
-// frequencies, 4 q, 3 v: one walker FP64 340 against 279 us, FP32 336 against 257; three 452 against 342 and
-// 445 against 303.
+// Launches of few walkers (few_walkers) are the G4 read-modify-write with little before it (FEW): all tiles,
+// without images, the rank-one factors staged in LDS beside the blocks, and one entry (complex128 G in small
+// tiles: four) loaded before it is stored. With the code for many walkers (images, factors read from memory in
+// the tail, twelve entries in flight) a launch of one walker took, 4x4, three channels, 64 frequencies, 4 q,
+// 3 v: FP64 340 against 279 us, FP32 336 against 257; of three, FP32 445 against 303.
 // Products are formed in the G precision; with complex64 G, tiles of up to 256 threads sum eight walkers in
 // FP32 before the FP64 totals, larger tiles (whose registers hold the totals) add every walker.
 // G4 is read and written once per launch (FP64, or FP32 value + Kahan compensation).
@@ -608,12 +607,30 @@ constexpr int totals_limit(bool fp32, int threads, int ppt, int terms, bool few)
   return threads == 1024 && (!fp32 || ppt > 1) ? 8 : 16;
 }
 
-// Launches of fewer walkers than this take the FEW kernel, up to two pairs per thread (its registers hold
-// no more). Geometric means over the channel sets, against the other kernel: five walkers 4x4 0.92, 18 and 20
-// sites 0.85, 25 sites 0.80; eight walkers 4x4 1.1, 18 to 32 sites 0.9 - 1.0 (one channel, 25 sites,
-// complex64: 0.85), 36 sites and more 1.2.
-constexpr int few_walkers(int threads, int ppt) {
-  return ppt == 4 ? 0 : threads == 1024 && ppt == 1 ? 9 : threads == 256 && ppt == 2 ? 8 : 6;
+// Launches of fewer walkers than this take the FEW kernel, up to two pairs per thread (its registers hold no
+// more). It computes every tile. Where all of them are resident at once, or nearly so, the other kernel gains
+// little from computing half; with many it does (`many`, 2048 frequency tiles, for tiles of more than 256
+// threads), and the more walkers the sooner. Each against the other, G4 stage with four momenta, over the channel
+// sets (one term; two):
+//   8 to 16 sites  complex64 three walkers 0.9 - 1.05; 0.6 - 0.97, five 1.0 - 1.1; 0.7 - 1.04. complex128 two
+//                  0.9 - 1.0, three 0.9 - 1.1; 0.7 - 1.0, five 0.9 - 1.4; 0.9 - 1.3
+//   18, 20 sites   four walkers 0.9 - 1.1; 0.75 - 1.05
+//   25, 32 sites   few tiles: five 0.8 - 1.0; 0.8 - 1.1. Many: three 0.8 - 0.9; 0.95 - 1.06, five 0.8 - 1.04; 0.93 - 1.1
+//   36 sites       few tiles: five 0.9; 0.8 - 0.97. Many: complex64 one 0.9 - 1.03; 0.9 - 1.06, two 1.03;
+//                  1.01 - 1.05; complex128 five 0.95; one 1.02 - 1.1
+//   40, 45 sites   complex64 few tiles: three 0.9 - 1.0; two 0.92 - 1.0, three 0.98 - 1.1. Many: one 0.91 - 0.98, two
+//                  1.0; one 0.97 - 1.09. complex128 five 0.93 - 0.97; one 1.05 - 1.33
+constexpr int few_walkers(bool fp32, int threads, int ppt, int terms, bool many) {
+  const bool one = terms == 1;
+  if (ppt == 4)
+    return 0;
+  if (threads <= 256)
+    return ppt == 2 ? 8 : fp32 ? (one ? 4 : 6) : (one ? 3 : 4);
+  if (ppt == 1)
+    return !many ? 9 : !one ? 3 : fp32 ? 6 : 4;
+  if (threads == 704)
+    return !many ? 6 : fp32 ? 2 : one ? 6 : 0;
+  return !fp32 ? (one ? 6 : 0) : !many ? (one ? 4 : 3) : one ? 2 : 0;
 }
 constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
 
@@ -628,7 +645,8 @@ void launch_pair_kernel(TiledArgs<Real> a, size_t lds, hipStream_t st) {
 
 template <typename Real, int TT, int PPT, int QG, int SET>
 void launch_pair_set(const TiledArgs<Real>& a, size_t lds, hipStream_t st) {
-  if constexpr (few_walkers(TT, PPT) > 0)
+  constexpr int terms = (SET & 1) + (SET >> 1 & 1) + (SET >> 2 & 1);
+  if constexpr (few_walkers(sizeof(Real) == 4, TT, PPT, terms, false) > 0)
     if (a.uv_lds >= 0)
       return launch_pair_kernel<Real, TT, PPT, QG, SET, true>(a, lds, st);
   launch_pair_kernel<Real, TT, PPT, QG, SET, false>(a, lds, st);
@@ -719,7 +737,8 @@ bool launch_g4_tiled(TiledArgs<Real> a, hipStream_t st) {
     a.uv_lds = static_cast<int>(block * ((n_ph > 0 ? 1 : 0) + (a.need_z ? 1 : 0)));
     return a.uv_lds + (a.rank_one ? sizeof(Cplx<Real>) * a.n_walkers * 4 * qg * g.nc : 0);
   };
-  bool few = a.n_walkers < few_walkers(ts.threads, ppt);
+  const bool many = static_cast<size_t>(g.nw) * g.nw * g.nv > 2048;
+  bool few = a.n_walkers < few_walkers(sizeof(Real) == 4, ts.threads, ppt, terms, many);
   size_t lds = plan(few);
   if (few && lds > kLdsBytes) {
     few = false;

@@ -69,3 +69,39 @@ def test_few_walkers_over_launches_equal_one_batch(nc, precision):
             # 17 sums of FP64 products; complex64: products of eight walkers in FP32 before FP64
             assert bf.difference(a, b)["l_inf"] < (1e-14 if precision == "fp64" else 1e-6)
     acc.close()
+
+
+@pytest.mark.parametrize("nc", [25, 36, 40])
+@pytest.mark.parametrize("n_freq", [44, 46])
+def test_few_walkers_around_the_tile_count(monkeypatch, nc, n_freq):
+    """Tiles of more than 256 threads: the count of walkers below which the form for few is taken falls at 2048
+    frequency tiles (46 squared is more, 44 squared less). Both sides against the per-entry kernel."""
+    channels = [MAG, PP] if nc > 25 else [MAG]
+    wl = synth.tiny_workload(cluster=geo.cluster_2d(*CLUSTERS[nc]), n_freq=n_freq, w_ex=(1,), channels=channels,
+                             n_range=(3, 20), seed_cfg=960 + nc)
+    g = wl.geometry
+    g.k_ex = [0, nc // 2]
+    ms = wl.draw(6)
+    make = lambda p: g4acc.TpAccumulator(g, precision=p, max_walkers=6, max_vertices=wl.n_max, tuned=False)
+    monkeypatch.setenv("G4ACC_GENERIC_G4", "1")
+    ref = make("fp64")
+    monkeypatch.delenv("G4ACC_GENERIC_G4")
+    accs = {p: make(p) for p in ("fp64", "fp32")}
+    ref.resetAccumulation()
+    total, size, done = [0.0] * len(channels), [0.0] * len(channels), 0
+    for m in ms:
+        ref.resetAccumulation()
+        ref.accumulate_batch([m])
+        for c, x in enumerate(ref.get_G4()):
+            total[c] = total[c] + x
+            size[c] = size[c] + np.abs(x)
+        done += 1
+        for p, tol in (("fp64", 1e-12), ("fp32", 1e-6)):
+            accs[p].resetAccumulation()
+            accs[p].accumulate_batch(ms[:done])
+            for c, x in enumerate(accs[p].get_G4()):
+                err = np.abs(x - total[c]).max() / size[c].max()
+                print(f"nc={nc} freq={n_freq} {p} W={done} channel {channels[c]}: {err:.3e}", flush=True)
+                assert err < tol
+    for a in (ref, *accs.values()):
+        a.close()
