@@ -100,6 +100,16 @@ struct G4Args {
 template <typename Real>
 void launch_g4(const G4Args<Real>& a, hipStream_t st);
 
+// Row block of the M -> G workgroup at place x of its plane (a column or slot) of n row blocks; planes start
+// `stride` workgroups apart. Over half of the pairs higher rows have more to do, and workgroups go to the eight
+// XCDs round-robin: with an even stride a row keeps to half of them or fewer (with a multiple of eight to one: 6x6,
+// complex128, 56 frequencies, 14 slots of 7..42 vertices: the last had 1.22 of the mean, 588 us before the halves,
+// 672 with them, 530 with the rows turned by one per plane). An odd stride spreads the rows by itself; turned as
+// well, they stayed (3 bands, 8 sites, 64 frequencies, 2 slots, complex128: S4 52.6 us, turned 69.9).
+__host__ __device__ inline int turned_row(unsigned x, unsigned plane, unsigned stride, unsigned n) {
+  return static_cast<int>((x + (stride % 2 ? 0 : plane)) % n);
+}
+
 // Symmetries of the single-band G4 over the pairs p = (k, w), with Q = (q, v) the transfer:
 //   transpose    T: (p1, p2) -> (p2 + Q, p1 + Q): for particle-hole channels X and Y, and the two
 //                   rank-one factors, swap. Needs 2 Q = 0 (v = 0, q its own inverse).

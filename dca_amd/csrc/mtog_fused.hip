@@ -114,8 +114,7 @@ __global__ void __launch_bounds__(256) mtog_right_fused(const SlotDesc* __restri
   const int s = slot & 1;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Rows rotate with the slot, as those with few needed pairs would otherwise share their XCDs.
-  const int bx = static_cast<int>((blockIdx.x + blockIdx.z) % gridDim.x);
+  const int bx = turned_row(blockIdx.x, blockIdx.z, gridDim.x * gridDim.y, gridDim.x);
   const int p1 = bx * 64 + lane;
   const int w2wg = blockIdx.y * WT;           // first frequency of the workgroup
   const int w2b = w2wg + wave * TW;           // first frequency of this wave

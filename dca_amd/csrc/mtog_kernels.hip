@@ -389,8 +389,7 @@ __global__ void __launch_bounds__(256) dft_right_G_shared(Geo g, int slot0, int 
   const int s = slot & 1;
   const int nc = g.nc, KW = nc * g.nwE;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // Rows rotate with the column and slot: those with few needed pairs would otherwise share their XCDs.
-  const int bx = static_cast<int>((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);
+  const int bx = turned_row(blockIdx.x, blockIdx.y, gridDim.x, gridDim.x);
   const int kw1 = bx * 64 + lane, w2 = blockIdx.y;
   if (w2 + (bx * 64 + 63) / nc < w_sum_min)
     return;

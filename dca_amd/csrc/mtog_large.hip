@@ -50,10 +50,8 @@ __global__ void __launch_bounds__(256) mtog_s3_mfma(Geo g, int n_max, int slot0,
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int D = g.D, nwE = g.nwE;
   const int w0 = blockIdx.y * 64;
-  // Rows rotate with the slot: higher ones have more of the needed half, and with a multiple of eight row
-  // blocks the same rows of every slot would run on the same XCD (6x6, 56 frequencies, 14 slots of 7..42
-  // vertices: the last of eight XCDs had 1.22 of the mean, 588 us before the halves, 672 with them).
-  const int bx = static_cast<int>((blockIdx.x + blockIdx.z) % gridDim.x);
+  // By slot: the columns of a row share its A.
+  const int bx = turned_row(blockIdx.x, blockIdx.z, gridDim.x * gridDim.y, gridDim.x);
   // Frequency tiles t_lo <= t < t_hi: mtog_site_G reads blocks of 64 rows and one w2.
   const int w1_hi = (bx * 64 + 63) / NC;
   const int below = w_sum_min - 15 - w1_hi - w0;
@@ -175,7 +173,7 @@ __global__ void __launch_bounds__(256) mtog_site_G(Geo g, int slot0, int w_sum_m
   const int s = slot & 1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int D = g.D;
-  const int bx = static_cast<int>((blockIdx.x + blockIdx.y + blockIdx.z) % gridDim.x);  // rotated, as in mtog_s3_mfma
+  const int bx = turned_row(blockIdx.x, blockIdx.y, gridDim.x, gridDim.x);
   const int p1 = bx * 64 + lane;
   const bool p_ok = p1 < D;
   const int pc = p_ok ? p1 : D - 1;

@@ -343,8 +343,7 @@ __global__ void __launch_bounds__(256) mtog_right_small(Geo g, int n_max, int sl
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int part = wave % TL::SPLIT;
-  // Rows rotate with the slot, as those with few needed frequencies would otherwise share their XCDs.
-  const int bx = static_cast<int>((blockIdx.x + blockIdx.z) % gridDim.x);
+  const int bx = turned_row(blockIdx.x, blockIdx.z, gridDim.x * gridDim.y, gridDim.x);
   const int p0 = (bx * TL::TPW + wave / TL::SPLIT) * 16;
   const int n_wt = (g.nwE + 15) / 16;
   // The first frequency tile that reaches w_sum_min with the workgroup's highest row.

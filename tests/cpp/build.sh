@@ -28,3 +28,7 @@ mv "$HERE/_build/sym_tiles_test.tmp" "$HERE/_build/sym_tiles_test"
 g++ -std=c++17 -O2 -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__ -I/opt/rocm/include \
     "$HERE/sym_images_test.cpp" -o "$HERE/_build/sym_images_test.tmp"
 mv "$HERE/_build/sym_images_test.tmp" "$HERE/_build/sym_images_test"
+# The row blocks of the M -> G workgroups.
+g++ -std=c++17 -O2 -Wall -Wno-unknown-pragmas -D__HIP_PLATFORM_AMD__ -I/opt/rocm/include \
+    "$HERE/turned_rows_test.cpp" -o "$HERE/_build/turned_rows_test.tmp"
+mv "$HERE/_build/turned_rows_test.tmp" "$HERE/_build/turned_rows_test"

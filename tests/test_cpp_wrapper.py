@@ -122,6 +122,18 @@ def test_symmetric_tiles_cover_g4_once():
     assert out.returncode == 0 and out.stdout.strip() == "OK", out.stdout
 
 
+def test_row_blocks_spread_over_the_xcds():
+    """The row blocks of the M -> G workgroups (tests/cpp/turned_rows_test.cpp)."""
+    exe = os.path.join(HERE, "cpp", "_build", "turned_rows_test")
+    if not os.path.exists(exe):
+        os.makedirs(os.path.dirname(exe), exist_ok=True)
+        subprocess.run(["g++", "-std=c++17", "-O2", "-Wno-unknown-pragmas", "-D__HIP_PLATFORM_AMD__",
+                        "-I/opt/rocm/include", os.path.join(HERE, "cpp", "turned_rows_test.cpp"), "-o", exe],
+                       check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.strip() == "OK", out.stdout
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("nb,L,precision,tol", [(1, 4, 0, 1e-12), (1, 4, 1, 1e-6), (3, 2, 0, 1e-12)])
 def test_cpp_mirror_matches_oracle(oracle_lib, tmp_path, nb, L, precision, tol):
