@@ -543,11 +543,18 @@ void launch_mtog(const MtoGArgs<Real>& a, hipStream_t st) {
     // S4 from LDS where eight momenta and more share a block's rows and the workgroups fill the card; with
     // real M and the momenta's inverses S3 then forms half of the frequency pairs. M -> G against S4 without LDS
     // and all of S3, 32 frequencies, 8 walkers: 3 bands, 8 sites 0.93 (8 frequencies 1.28), 10 sites 0.8 - 0.95;
-    // it loses at 4 sites (2 to 4 bands 1.0 - 1.2), with 4 bands, and with 2 in complex64 (1.08).
+    // it loses at 4 sites (2 to 4 bands 1.0 - 1.2), with 4 bands, and with 2 in complex64 (1.08). With 3 bands in
+    // complex128 it gains more, so earlier: 8 sites, 32 frequencies, one walker (256 workgroups) 0.9, 8 frequencies,
+    // 48 walkers 0.85, 4 sites, 32 frequencies, 48 walkers 0.87 - 0.91.
     const size_t el = sizeof(Cplx<Real>) * g.n_orb * (64 * static_cast<size_t>(g.nb) + 1);
     const dim3 gs((g.nc * g.nwE + 63) / 64, g.nwE, ns);
-    const bool shared = el <= 81920 && g.nc >= 8 && (g.nb == 1 || g.nb == 3 || (g.nb == 2 && sizeof(Real) == 8)) &&
-                        g.nwE >= 16 && static_cast<size_t>(gs.x) * gs.y * gs.z >= 512;
+    const size_t blocks = static_cast<size_t>(gs.x) * gs.y * gs.z;
+    const int KW = g.nc * g.nwE;
+    const bool shared = el <= 81920 &&
+                        (g.nb == 3 && sizeof(Real) == 8
+                             ? KW >= 64 && blocks >= (KW >= 256 ? 256 : 512)
+                             : g.nc >= 8 && (g.nb == 1 || g.nb == 3 || (g.nb == 2 && sizeof(Real) == 8)) && g.nwE >= 16 &&
+                                   blocks >= 512);
     const bool mirror = shared && a.real_m && a.kneg && a.w_sum_min == 0;
     const int sum_min = mirror ? g.nwE - 1 : a.w_sum_min;
     hipLaunchKernelGGL(ndft_right_kernel<Real>, dim3((g.D + 255) / 256, g.D, ns), dim3(256), 0, st,
@@ -565,7 +572,6 @@ void launch_mtog(const MtoGArgs<Real>& a, hipStream_t st) {
         run(dft_right_G_shared<Real, 2>);
       continue;
     }
-    const int KW = g.nc * g.nwE;
     const dim3 grid((KW + 255) / 256, KW, ns);
     switch (g.nb) {
       case 1: hipLaunchKernelGGL((dft_right_G_kernel<Real, 1>), grid, dim3(256), 0, st, g, s0, a.w_sum_min, a.dft, a.bphase, a.G0, a.E, a.G); break;

@@ -41,3 +41,12 @@ def test_batches_match_oracle(oracle_lib, nb, nc, nf, walkers):
             print(f"nb={nb} nc={nc} nf={nf} W={walkers} {precision} channel {ch}: {err:.3e}", flush=True)
             assert err < tol
         acc.close()
+
+
+CLUSTERS[4] = ((2, 0), (0, 2))
+
+
+# 3 bands, complex128: from 512 blocks on with 64 pairs (k, w), 256 with 256 pairs, and below
+@pytest.mark.parametrize("nc,nf,walkers", [(8, 32, 1), (8, 30, 1), (8, 8, 32), (8, 8, 31), (4, 32, 4), (4, 14, 20)])
+def test_three_bands_match_oracle(oracle_lib, nc, nf, walkers):
+    test_batches_match_oracle(oracle_lib, 3, nc, nf, walkers)
